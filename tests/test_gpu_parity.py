@@ -188,6 +188,45 @@ def test_sorted_mover_bit_exact_against_oracle(periodic):
         assert np.array_equal(got[k].view(np.uint8), sp.a[k].view(np.uint8)), k
 
 
+@pytest.mark.parametrize("per_cell", [1, 6, 19, 20, 31, 47, 48, 150])
+def test_sorted_mover_at_every_block_span(per_cell):
+    """64-particle blocks that span one to many bins, rows and empty cells
+    (staged bins and lanes past them), at both sides of the lines between the
+    staged bin counts; bit for bit against the oracle."""
+    cells, lengths = (5, 3, 4), (1.25, 0.75, 1.0)
+    rng = np.random.default_rng(100 + per_cell)
+    g, a = random_state(cells, lengths, per_cell, rng, vscale=1.5)
+    # A third of the cells hand their particles to the cell above them.
+    ncell = cells[0] * cells[1] * cells[2]
+    home = np.arange(ncell)
+    emptied = rng.permutation(ncell - 1)[:ncell // 3]
+    home[emptied] += 1
+    c = np.repeat(home, per_cell)
+    a["cell"] = O.encode(g, c % cells[0], (c // cells[0]) % cells[1], c // (cells[0] * cells[1])).astype(np.int32)
+    # Flights of many boxes, onto whole boxes and a rejected record.
+    a["u"][0], a["v"][1], a["w"][2 % len(c)] = 4e6, -4e6, 250.0
+    a["rx"][len(c) // 2] = 1.5
+    order = rng.permutation(len(c))
+    a = {k: v[order] for k, v in a.items()}
+    e = periodic_nodes(cells, rng, 0.2)
+    b = periodic_nodes(cells, rng, 0.6)
+    qom, dt = 2.5, 0.11
+    with gpu(cells, lengths, [(qom, len(c))], dt=dt, particle_periodic=(1, 0, 1)) as sim:
+        sim.set_particles(0, a)
+        sim.sort(0)
+        sim.set_field(R.FIELD_ETHETA, e)
+        sim.set_field(R.FIELD_BNODE, b)
+        sim.move(0)
+        got = sim.get_particles(0)
+        flags = sim.validation()
+    g.particle_periodic[0], g.particle_periodic[1], g.particle_periodic[2] = 1, 0, 1
+    sp, _, _, _ = O.sort(g, to_oracle(a))
+    oflags = O.move(g, O.mover_params(qom, dt, 1.0, g.spacing), sp, e, b)
+    assert flags == oflags == R.INVALID_FRACTION
+    for k in got:
+        assert np.array_equal(got[k].view(np.uint8), sp.a[k].view(np.uint8)), k
+
+
 def test_sorted_mover_skips_halo_bins_and_a_failed_sort():
     """The sorted mover pushes the records of interior bins only: records
     sorted into halo bins stay as they are and raise no flag (the sort has

@@ -33,11 +33,31 @@ constexpr unsigned kWaves = kThreads / 64;
 
 struct MoverParams {
   double beta, beta_over_c, dt, inverse_spacing[3];
+  double extent[3];  // cells per axis
 };
 
-__device__ __forceinline__ int64_t positive_modulo(int64_t cell, int64_t extent) {
-  const int64_t r = cell % extent;
-  return r < 0 ? r + extent : r;
+// cell modulo extent in [0, extent) for whole numbers below 2^34: they and
+// the products are exact, and a quotient rounds across a whole number only
+// from nearer than its own last place, where cell / extent never lies (it is a
+// multiple of 1 / extent). A 64-bit integer remainder here held 30 registers.
+__device__ __forceinline__ double modulo(double cell, double extent) {
+  return cell - extent * floor(cell / extent);
+}
+
+// The mirror fold of a cell index in [extent, 2 extent): the reflected box,
+// fraction and velocity reversed, an exact 1.0 carried back into the box.
+__device__ __forceinline__ void mirror(double extent, double& whole, double& frac, double& vel) {
+  whole = 2.0 * extent - whole - 1.0;
+  frac = 1.0 - frac;
+  vel = -vel;
+  if (frac == 1.0) {
+    if (whole + 1.0 < extent) {
+      whole += 1.0;
+      frac = 0.0;
+    } else {
+      frac = 1.0 - 1.1102230246251565e-16;  // 1 - epsilon/2
+    }
+  }
 }
 
 // The record of one particle as the mover reads it (60 B).
@@ -57,6 +77,14 @@ __device__ __forceinline__ void load_raw(const ParticleView& s, uint32_t index, 
   r.key = s.cell[index];
 }
 
+// The same of particle `lane` of an aligned 64-particle block: the block's
+// base is wave-uniform, so every address is a scalar base plus the lane's
+// 32-bit offset.
+__device__ __forceinline__ ParticleView block_view(const ParticleView& s, uint32_t block) {
+  const size_t at = size_t(block) * 64u;
+  return ParticleView{s.rx + at, s.ry + at, s.rz + at, s.u + at, s.v + at, s.w + at, s.q + at, s.cell + at, s.id};
+}
+
 // The pushed state of one particle: new key, fractions and velocity.
 struct Pushed {
   int32_t key;
@@ -66,9 +94,9 @@ struct Pushed {
 // Record checks and the 8 CIC weights of the stored fractions (corners
 // x-fastest). Returns the validation flags of a rejection, or 0.
 __device__ __forceinline__ unsigned particle_weights(const Raw& r, double (&w)[8]) {
-  if (!finite_value(r.q)) return kInvalidNonfinite;
   const double fx = r.rx, fy = r.ry, fz = r.rz;
-  if (!(fx >= 0.0 && fx < 1.0 && fy >= 0.0 && fy < 1.0 && fz >= 0.0 && fz < 1.0)) return kInvalidFraction;
+  const bool inside = fx >= 0.0 && fx < 1.0 && fy >= 0.0 && fy < 1.0 && fz >= 0.0 && fz < 1.0;
+  const unsigned bad = !finite_value(r.q) ? kInvalidNonfinite : (!inside ? kInvalidFraction : 0u);
   const double cx = 1.0 - fx, cy = 1.0 - fy, cz = 1.0 - fz;
   w[0] = cx * cy * cz;
   w[1] = fx * cy * cz;
@@ -78,7 +106,7 @@ __device__ __forceinline__ unsigned particle_weights(const Raw& r, double (&w)[8
   w[5] = fx * cy * fz;
   w[6] = cx * fy * fz;
   w[7] = fx * fy * fz;
-  return 0u;
+  return bad;
 }
 
 // B and E_theta at the particle: component c (Bx, By, Bz, Ex, Ey, Ez) is the
@@ -91,6 +119,8 @@ __device__ __forceinline__ void interpolate(const double (&w)[8], const Corner& 
 #pragma unroll
     for (int a = 0; a < 8; ++a) value += w[a] * corner(c, a);
     f[c] = value;
+    // Two components' corner values in flight (all 48 would hold 96 registers).
+    if (c & 1) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -123,10 +153,10 @@ __device__ __forceinline__ unsigned push_particle(const Grid& g, const MoverPara
                                                   int ck, const Corner& corner, Pushed& out) {
   double w[8];
   const unsigned bad = particle_weights(r, w);
-  if (bad) return bad;
   double f[6];
   interpolate(w, corner, f);
-  return push_fields(g, p, r, ci, cj, ck, f, out);
+  const unsigned flags = push_fields(g, p, r, ci, cj, ck, f, out);
+  return bad ? bad : flags;
 }
 
 // The push from the interpolated fields: response, velocity update,
@@ -151,57 +181,45 @@ __device__ __forceinline__ unsigned push_fields(const Grid& g, const MoverParams
   const double aey = a3 * ex + a4 * ey + a5 * ez;
   const double aez = a6 * ex + a7 * ey + a8 * ez;
   const double px = hx + p.beta * aex, py = hy + p.beta * aey, pz = hz + p.beta * aez;
-  int64_t pc[3] = {ci, cj, ck};
+  const int cell[3] = {ci, cj, ck};
+  int pc[3];
   double frac[3] = {fx, fy, fz};
   double vel[3] = {2.0 * px - u, 2.0 * py - v, 2.0 * pz - ww};
+  // Straight-line, with the first failing axis's flag kept: early returns
+  // held the new state across their joins, in scratch memory.
+  unsigned flags = 0;
 #pragma unroll
   for (int axis = 0; axis < 3; ++axis) {
-    if (!finite_value(vel[axis])) return kInvalidNonfinite;
     const double displacement = p.dt * vel[axis] * p.inverse_spacing[axis];
     const double moved = frac[axis] + displacement;
     const double shift = floor(moved);
-    if (!(shift >= -2147483648.0 && shift <= 2147483647.0)) return kInvalidFlight;
-    pc[axis] += int64_t(shift);
+    const bool flight = shift >= -2147483648.0 && shift <= 2147483647.0;
+    if (flags == 0u) flags = !finite_value(vel[axis]) ? kInvalidNonfinite : (!flight ? kInvalidFlight : 0u);
     frac[axis] = moved - shift;
+    double whole = double(cell[axis]) + (flight ? shift : 0.0);
     if (frac[axis] == 1.0) {
-      ++pc[axis];
+      whole += 1.0;
       frac[axis] = 0.0;
     }
-  }
-  const int extents[3] = {g.nx, g.ny, g.nz};
-#pragma unroll
-  for (int axis = 0; axis < 3; ++axis) {
-    const int64_t extent = extents[axis];
-    int64_t global = pc[axis];
-    if (global >= 0 && global < extent) continue;
-    if (g.particle_periodic[axis]) {
-      pc[axis] = positive_modulo(global, extent);
-    } else {
-      global = positive_modulo(global, 2 * extent);
-      if (global >= extent) {
-        global = 2 * extent - global - 1;
-        frac[axis] = 1.0 - frac[axis];
-        vel[axis] = -vel[axis];
-        if (frac[axis] == 1.0) {
-          if (global + 1 < extent) {
-            ++global;
-            frac[axis] = 0.0;
-          } else {
-            frac[axis] = 1.0 - 1.1102230246251565e-16;  // 1 - epsilon/2
-          }
-        }
+    const double extent = p.extent[axis];
+    if (!(whole >= 0.0 && whole < extent)) {
+      if (g.particle_periodic[axis]) {
+        whole = modulo(whole, extent);
+      } else {
+        whole = modulo(whole, 2.0 * extent);
+        if (whole >= extent) mirror(extent, whole, frac[axis], vel[axis]);
       }
-      pc[axis] = global;
     }
+    pc[axis] = int(whole);
   }
-  out.key = g.encode(int(pc[0]), int(pc[1]), int(pc[2]));
+  out.key = g.encode(pc[0], pc[1], pc[2]);
   out.r[0] = frac[0];
   out.r[1] = frac[1];
   out.r[2] = frac[2];
   out.v[0] = vel[0];
   out.v[1] = vel[1];
   out.v[2] = vel[2];
-  return 0u;
+  return flags;
 }
 
 // The accepted state overwrites the record in place (a rejected record keeps
@@ -229,16 +247,39 @@ __device__ __forceinline__ void corner_nodes(const Grid& g, int ci, int cj, int 
   at[7] = n0 + sz + sy + 1;
 }
 
+// The interpolation of the rare lanes past the staged bins, one component at
+// a time (48 node values in flight would take the registers of a whole block).
+__device__ __forceinline__ void interpolate_nodes(const Grid& g, const double (&w)[8], int ci, int cj, int ck,
+                                                  const double* __restrict__ bnode,
+                                                  const double* __restrict__ etheta, double (&f)[6]) {
+  const unsigned n0 = g.node(ci, cj, ck), nodes = g.nodes();
+  const unsigned sy = unsigned(g.nx + 1), sz = unsigned(g.nx + 1) * unsigned(g.ny + 1);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    const double* v = (c < 3 ? bnode + size_t(c) * nodes : etheta + size_t(c - 3) * nodes) + n0;
+    double value = 0.0;
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+      value += w[a] * v[unsigned(a & 1) + unsigned((a >> 1) & 1) * sy + unsigned(a >> 2) * sz];
+    f[c] = value;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // The sorted mover walks the species array in aligned blocks of 64
 // particles, not cell by cell: every record line is read once and every
 // block is one full pass of the wave (a cell walk reads the line a cell
 // shares with the next one twice and spends a second, nearly empty pass on a
 // cell holding more than 64 particles). The particles of a block lie in a few
-// consecutive bins; a pass stages the 48 corner field values of kSlots
-// consecutive bins in LDS and pushes the lanes whose key is one of them.
-constexpr unsigned kSlots = 2;
-constexpr unsigned kSlotValues = kSlots * 48;
-constexpr unsigned kSlotLoads = (kSlotValues + 63) / 64;
+// bins, in ascending order: the 48 corner field values of the first Slots
+// distinct bins are staged in LDS, and a lane reads those of its bin's slot. A
+// lane past them gathers its corners from the node fields, which costs the
+// wave a second pass: the slots follow the species' particles per cell. Two
+// slots for every species cost 228 us per 2.55M particles at 27 per cell,
+// where a block spans three or four bins; four cost about 92 us.
+// Slots lie kSlotStride doubles apart (100 words: up to ten slots at one value
+// start in distinct LDS banks).
+constexpr unsigned kSlotStride = 50;
 
 // The bin whose range holds sorted position `index` (the last bin whose
 // first index is at most `index`), or -1 when no bin's range holds it.
@@ -270,59 +311,115 @@ __device__ unsigned unpushed_flags(const Grid& g, const uint32_t* __restrict__ o
   return g.interior(i, j, k) ? unsigned(kInvalidKey) : 0u;
 }
 
-// Lane values of a pass's staged corners: value v = lane + 64 t is corner
-// v % 8 of component (v % 48) / 8 of the cell of bin base + v / 48, loaded
-// when that bin is an interior cell in base's row (others are never read).
-__device__ __forceinline__ void load_slots(const Grid& g, int32_t base, const double* __restrict__ bnode,
-                                           const double* __restrict__ etheta, unsigned lane,
-                                           double (&cv)[kSlotLoads]) {
-  int bi, bj, bk;
-  g.decode(base, bi, bj, bk);
-  const bool row = bj >= 0 && bj < g.ny && bk >= 0 && bk < g.nz;
-  const unsigned nodes = g.nodes();
-  const unsigned sy = unsigned(g.nx + 1), sz = unsigned(g.nx + 1) * unsigned(g.ny + 1);
+// Lanes that start a bin of the block: a key in range that differs from the
+// lane's below.
+__device__ __forceinline__ uint64_t head_lanes(bool candidate, int32_t key, unsigned lane) {
+  const int32_t below = __shfl_up(key, 1u, 64);
+  return __builtin_amdgcn_ballot_w64(candidate && (lane == 0 || below != key));
+}
+
+// The slot of a lane's bin: the heads at or below the lane, less one (a lane
+// below the first head is no candidate).
+__device__ __forceinline__ unsigned slot_of(uint64_t heads) {
+  const unsigned lane = threadIdx.x & 63u;
+  return __builtin_amdgcn_mbcnt_hi(unsigned(heads >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(heads), 0u)) +
+         unsigned((heads >> lane) & 1u) - 1u;
+}
+
+// The cell of a key, given the decoded cell of another key of the block:
+// most keys of a block lie in one row.
+struct BlockCell {
+  int32_t key;
+  int i, j, k;
+};
+
+__device__ __forceinline__ BlockCell block_cell(const Grid& g, int32_t key) {
+  BlockCell c{key, 0, 0, 0};
+  g.decode(key, c.i, c.j, c.k);
+  return c;
+}
+
+__device__ __forceinline__ void cell_near(const Grid& g, const BlockCell& first, int32_t key, int& i, int& j, int& k) {
+  i = first.i + (key - first.key);
+  j = first.j;
+  k = first.k;
+  if (key < first.key || i > g.nx + 1) g.decode(key, i, j, k);
+}
+
+// Lane values of a block's staged corners: value v = lane + 64 t is corner
+// v % 8 of component (v % 48) / 8 of slot v / 48, whose bin is that of the
+// block's head v / 48; loaded when the bin is an interior cell (a slot without
+// one is never read).
+template <unsigned Slots>
+struct StagedSlots {
+  static constexpr unsigned kValues = Slots * 48;
+  static constexpr unsigned kLoads = (kValues + 63) / 64;
+  double v[kLoads];
+
+  // `first` is the cell of the first head.
+  __device__ __forceinline__ void load(const Grid& g, uint64_t heads, const BlockCell& first, int32_t key,
+                                       const double* __restrict__ bnode, const double* __restrict__ etheta,
+                                       unsigned lane) {
+    const unsigned nodes = g.nodes();
+    const unsigned sy = unsigned(g.nx + 1), sz = unsigned(g.nx + 1) * unsigned(g.ny + 1);
+    // Wave-uniform: the lower node of every slot's cell, or none.
+    constexpr unsigned kNone = 0xffffffffu;
+    unsigned at[Slots];
+    uint64_t m = heads;
 #pragma unroll
-  for (unsigned t = 0; t < kSlotLoads; ++t) {
-    const unsigned v = lane + 64u * t;
-    cv[t] = 0.0;
-    const int i = bi + int(v / 48u);
-    if (v < kSlotValues && row && i >= 0 && i < g.nx) {
-      const unsigned jv = v % 48u, comp = jv >> 3, a = jv & 7u;
-      const unsigned at = g.node(i, bj, bk) + (a & 1u) + ((a >> 1) & 1u) * sy + ((a >> 2) & 1u) * sz;
-      cv[t] = comp < 3 ? bnode[size_t(comp) * nodes + at] : etheta[size_t(comp - 3) * nodes + at];
+    for (unsigned s = 0; s < Slots; ++s) {
+      at[s] = kNone;
+      if (m) {
+        const int32_t bin = __builtin_amdgcn_readlane(key, int(__builtin_ctzll(m)));
+        m &= m - 1;
+        int i, j, k;
+        cell_near(g, first, bin, i, j, k);
+        if (g.interior(i, j, k)) at[s] = g.node(i, j, k);
+      }
+    }
+#pragma unroll
+    for (unsigned t = 0; t < kLoads; ++t) {
+      const unsigned x = lane + 64u * t;
+      // Lanes of load t lie in at most three slots: first slot (64 t) / 48.
+      constexpr unsigned kLast = Slots - 1;
+      const unsigned s0 = (64u * t) / 48u;
+      const unsigned s1 = s0 + 1 < Slots ? s0 + 1 : kLast, s2 = s0 + 2 < Slots ? s0 + 2 : kLast;
+      const unsigned slot = x / 48u;
+      const unsigned node = slot == s0 ? at[s0] : (slot == s0 + 1 ? at[s1] : at[s2]);
+      v[t] = 0.0;
+      if (x < kValues && node != kNone) {
+        const unsigned jv = x % 48u, comp = jv >> 3, a = jv & 7u;
+        const unsigned n = node + (a & 1u) + ((a >> 1) & 1u) * sy + ((a >> 2) & 1u) * sz;
+        v[t] = comp < 3 ? bnode[size_t(comp) * nodes + n] : etheta[size_t(comp - 3) * nodes + n];
+      }
     }
   }
-}
 
-__device__ __forceinline__ void stage_slots(double* corner, unsigned lane, const double (&cv)[kSlotLoads]) {
+  __device__ __forceinline__ void stage(double* corner, unsigned lane) const {
 #pragma unroll
-  for (unsigned t = 0; t < kSlotLoads; ++t)
-    if (lane + 64u * t < kSlotValues) corner[lane + 64u * t] = cv[t];
-}
-
-// The first bin of a block's passes: the key of its first lane with a key in
-// range (wave-uniform), or -1 when it has none.
-__device__ __forceinline__ int32_t first_base(bool candidate, int32_t key) {
-  const uint64_t m = __builtin_amdgcn_ballot_w64(candidate);
-  if (m == 0) return -1;
-  return __builtin_amdgcn_readlane(key, int(__builtin_ctzll(m)));
-}
+    for (unsigned t = 0; t < kLoads; ++t) {
+      const unsigned x = lane + 64u * t;
+      if (x < kValues) corner[(x / 48u) * kSlotStride + x % 48u] = v[t];
+    }
+  }
+};
 
 __device__ __forceinline__ bool key_in_range(int32_t key, uint32_t bins) { return key >= 0 && uint32_t(key) < bins; }
 
 // Each wave owns a contiguous range of blocks (remapped so an XCD's waves own
 // neighbouring blocks) and walks it with a two-stage pipeline: the keys of
-// block b+2, and the records, key ranges and first-pass corner fields of
+// block b+2, and the records, key ranges and staged corner fields of
 // block b+1, are in flight while block b is pushed; block b+1's corners are
 // staged in the second LDS buffer once b is done.
-__global__ __launch_bounds__(kThreads) void k_move_blocks(Grid g, MoverParams p, ParticleView s, uint32_t n,
+template <unsigned Slots>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(Slots > 4 ? 3 : 4))) void k_move_blocks(Grid g, MoverParams p, ParticleView s, uint32_t n,
                                                           const uint32_t* __restrict__ counts,
                                                           const uint32_t* __restrict__ offsets,
                                                           const double* __restrict__ etheta,
                                                           const double* __restrict__ bnode,
                                                           unsigned* __restrict__ validation,
                                                           uint64_t* __restrict__ cross) {
-  __shared__ double s_corner[kWaves][2][kSlotValues];
+  __shared__ __align__(16) double s_corner[kWaves][2][Slots * kSlotStride];
   const unsigned lane = threadIdx.x & 63u;
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t bins = g.bins();
@@ -336,98 +433,86 @@ __global__ __launch_bounds__(kThreads) void k_move_blocks(Grid g, MoverParams p,
   unsigned flags = 0;
   unsigned buf = 0;
   // Block b_begin: records, whether each lane lies in its key's bin range,
-  // first-pass corners staged; block b_begin + 1: keys.
+  // heads and staged corners; block b_begin + 1: keys.
   Raw cur;
   cur.key = -1;
   bool cur_in_range = false;
-  int32_t base0;
+  uint64_t heads = 0;
+  BlockCell cell0{};
   {
     const uint32_t index = b_begin * 64u + lane;
-    if (index < n) load_raw(s, index, cur);
-    if (index < n && key_in_range(cur.key, bins)) cur_in_range = index - offsets[cur.key] < counts[cur.key];
-    base0 = first_base(index < n && key_in_range(cur.key, bins), cur.key);
-    if (base0 >= 0) {
-      double cv[kSlotLoads];
-      load_slots(g, base0, bnode, etheta, lane, cv);
-      stage_slots(s_corner[wave][buf], lane, cv);
+    if (index < n) load_raw(block_view(s, b_begin), lane, cur);
+    const bool ranged = index < n && key_in_range(cur.key, bins);
+    if (ranged) cur_in_range = index - offsets[cur.key] < counts[cur.key];
+    heads = head_lanes(ranged, cur.key, lane);
+    if (heads) {
+      cell0 = block_cell(g, __builtin_amdgcn_readlane(cur.key, int(__builtin_ctzll(heads))));
+      StagedSlots<Slots> cv;
+      cv.load(g, heads, cell0, cur.key, bnode, etheta, lane);
+      cv.stage(s_corner[wave][buf], lane);
     }
   }
   int32_t key1 = -1;
-  if (b_begin + 1 < b_end && (b_begin + 1) * 64u + lane < n) key1 = s.cell[(b_begin + 1) * 64u + lane];
+  if (b_begin + 1 < b_end && (b_begin + 1) * 64u + lane < n) key1 = block_view(s, b_begin + 1).cell[lane];
   for (uint32_t b = b_begin; b < b_end; ++b) {
-    // Block b + 1: records, key ranges and first-pass corners; block b + 2: keys.
+    // Block b + 1: records, key ranges and staged corners; block b + 2: keys.
     const bool more = b + 1 < b_end;
     const uint32_t index1 = (b + 1) * 64u + lane;
     Raw nxt;
     nxt.key = -1;
     uint32_t first1 = 0, count1 = 0;
-    double cv_next[kSlotLoads];
-    int32_t base1 = -1;
+    StagedSlots<Slots> cv_next;
+    uint64_t heads1 = 0;
+    BlockCell cell1{};
     if (more) {
       // The key-dependent requests first (their lane reads of key1 then wait
       // only for key1's own load, issued a block earlier), then the records:
       // all of them stay in flight while block b is pushed.
       const bool ranged = index1 < n && key_in_range(key1, bins);
-      base1 = first_base(ranged, key1);
+      heads1 = head_lanes(ranged, key1, lane);
       if (ranged) {
         first1 = offsets[key1];
         count1 = counts[key1];
       }
-      if (base1 >= 0) load_slots(g, base1, bnode, etheta, lane, cv_next);
-      if (index1 < n) load_raw(s, index1, nxt);
+      if (heads1) {
+        cell1 = block_cell(g, __builtin_amdgcn_readlane(key1, int(__builtin_ctzll(heads1))));
+        cv_next.load(g, heads1, cell1, key1, bnode, etheta, lane);
+      }
+      if (index1 < n) load_raw(block_view(s, b + 1), lane, nxt);
     }
     int32_t key2 = -1;
-    if (b + 2 < b_end && (b + 2) * 64u + lane < n) key2 = s.cell[(b + 2) * 64u + lane];
-    // Push block b: the lanes whose key is one of the kSlots staged bins from
-    // base0 in base0's row read the staged corners; any other lane (a block
-    // spanning more bins, or a row's end) gathers its corners from the node
-    // fields.
+    if (b + 2 < b_end && (b + 2) * 64u + lane < n) key2 = block_view(s, b + 2).cell[lane];
+    // Push block b: the lanes of the staged bins read the staged corners; any
+    // other lane (a block spanning more bins) gathers its corners from the
+    // node fields.
     const double* corner = s_corner[wave][buf];
     const uint32_t index = b * 64u + lane;
     const int32_t key = cur.key;
     const bool candidate = index < n && key_in_range(key, bins);
-    bool unpushed = index < n && !candidate;
-    bool gather = false;
+    bool unpushed = index < n;
     bool crossed = false;  // pushed into another cell
     __builtin_amdgcn_wave_barrier();
     asm volatile("" ::: "memory");
-    if (candidate) {
-      int bi, bj, bk;
-      g.decode(base0, bi, bj, bk);
-      const int d = key - base0;
-      if (d >= 0 && d < int(kSlots) && bi + d <= g.nx + 1) {
-        const int ci = bi + d;
-        const bool cell_ok = ci >= 0 && ci < g.nx && bj >= 0 && bj < g.ny && bk >= 0 && bk < g.nz;
-        if (cell_ok && cur_in_range) {
-          Pushed out;
-          const unsigned f = push_particle(g, p, cur, ci, bj, bk, StagedCorners{corner + d * 48}, out);
-          flags |= f;
-          if (f == 0u) {
-            store_pushed(s, index, out);
-            crossed = out.key != key;
-          }
-        } else {
-          unpushed = true;
-        }
-      } else {
-        gather = true;
-      }
-    }
-    if (__builtin_amdgcn_ballot_w64(gather) != 0 && gather) {
+    if (candidate && cur_in_range) {
       int ci, cj, ck;
-      g.decode(key, ci, cj, ck);
-      if (g.interior(ci, cj, ck) && cur_in_range) {
-        NodeCorners nc{bnode, etheta, g.nodes(), {}};
-        corner_nodes(g, ci, cj, ck, nc.at);
+      cell_near(g, cell0, key, ci, cj, ck);
+      if (g.interior(ci, cj, ck)) {
+        unpushed = false;
+        double w[8], fields[6];
+        const unsigned bad = particle_weights(cur, w);
+        const unsigned slot = slot_of(heads);
+        if (slot < Slots)
+          interpolate(w, StagedCorners{corner + slot * kSlotStride}, fields);
+        else
+          interpolate_nodes(g, w, ci, cj, ck, bnode, etheta, fields);
         Pushed out;
-        const unsigned f = push_particle(g, p, cur, ci, cj, ck, nc, out);
-        flags |= f;
+        unsigned f = push_fields(g, p, cur, ci, cj, ck, fields, out);
+        if (bad) f = bad;
         if (f == 0u) {
-          store_pushed(s, index, out);
+          store_pushed(block_view(s, b), lane, out);
           crossed = out.key != key;
         }
-      } else {
-        unpushed = true;
+        flags |= f;
       }
     }
     if (cross) {
@@ -438,10 +523,11 @@ __global__ __launch_bounds__(kThreads) void k_move_blocks(Grid g, MoverParams p,
     asm volatile("" ::: "memory");
     if (unpushed) flags |= unpushed_flags(g, offsets, counts, index, key);
     // Block b + 1 becomes current: its corners go to the other buffer.
-    if (more && base1 >= 0) stage_slots(s_corner[wave][buf ^ 1u], lane, cv_next);
+    if (heads1) cv_next.stage(s_corner[wave][buf ^ 1u], lane);
     cur = nxt;
     cur_in_range = index1 - first1 < count1;
-    base0 = base1;
+    heads = heads1;
+    cell0 = cell1;
     key1 = key2;
     buf ^= 1u;
   }
@@ -491,6 +577,9 @@ MoverParams mover_params(const Context& ctx, const SpeciesState& sp) {
   p.inverse_spacing[0] = 1.0 / ctx.grid.dx;
   p.inverse_spacing[1] = 1.0 / ctx.grid.dy;
   p.inverse_spacing[2] = 1.0 / ctx.grid.dz;
+  p.extent[0] = ctx.grid.nx;
+  p.extent[1] = ctx.grid.ny;
+  p.extent[2] = ctx.grid.nz;
   return p;
 }
 
@@ -502,6 +591,13 @@ unsigned block_walk_blocks(const Context& ctx, uint32_t n) {
   return unsigned(std::max<uint64_t>(1, want < cap ? want : cap));
 }
 
+// The sorted mover with room for Slots bins a block.
+template <unsigned Slots>
+void launch_blocks(const Context& ctx, const SpeciesState& sp, const MoverParams& p, uint64_t* cross) {
+  k_move_blocks<Slots><<<block_walk_blocks(ctx, sp.count), kThreads, 0, ctx.stream>>>(
+      ctx.grid, p, sp.view(), sp.count, sp.counts, sp.offsets, ctx.particle_field(), ctx.bn, ctx.validation, cross);
+}
+
 }  // namespace
 
 int launch_move(Context& ctx, int s, bool record_crossers) {
@@ -510,10 +606,20 @@ int launch_move(Context& ctx, int s, bool record_crossers) {
   const MoverParams p = mover_params(ctx, sp);
   phase_begin(ctx, Phase::move);
   if (sp.sorted) {
-    const unsigned blocks = block_walk_blocks(ctx, sp.count);
-    k_move_blocks<<<blocks, kThreads, 0, ctx.stream>>>(ctx.grid, p, sp.view(), sp.count, sp.counts, sp.offsets,
-                                                       ctx.particle_field(), ctx.bn, ctx.validation,
-                                                       record_crossers ? sp.cross : nullptr);
+    uint64_t* const cross = record_crossers ? sp.cross : nullptr;
+    const uint64_t cells = ctx.grid.cells();
+    // Slots by the mean count c of a cell: 64 particles span 64 / c + 1 bins
+    // and more where counts vary. From 48 on two bins hold nearly every block
+    // (four instead of two: 1.3% of the cycle slower at 64 per cell and 128^3,
+    // 3.8% at 100 per cell and 512^2); four bins hold three or four bins'
+    // blocks down to 20 (cycle at 61 x 47 x 33 with 27 per cell: 1.61 ms with
+    // two, 1.34 ms with four), ten those of 8 a cell.
+    if (sp.count >= 48 * cells)
+      launch_blocks<2>(ctx, sp, p, cross);
+    else if (sp.count >= 20 * cells)
+      launch_blocks<4>(ctx, sp, p, cross);
+    else
+      launch_blocks<10>(ctx, sp, p, cross);
   } else {
     const unsigned blocks = unsigned(std::min<uint64_t>((uint64_t(sp.count) + kThreads - 1) / kThreads,
                                                         uint64_t(ctx.cus > 0 ? ctx.cus : 256) * 32));
