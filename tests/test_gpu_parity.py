@@ -1142,6 +1142,93 @@ def test_walled_solve_projects_a_field_set_after_startup(kind):
         ref.close()
 
 
+# Grids on both sides of the line between the operator's two forms (16384
+# nodes), with a part-filled last block, one-cell axes, walls and smoothing, and
+# restarts shorter than the solve.
+SOLVER_GRIDS = {
+    "small": ((24, 24, 24), None, None, 30),
+    "small_restarted": ((13, 9, 11), None, None, 3),
+    "line": ((70, 1, 1), None, None, 4),
+    "small_walls_restarted": ((12, 11, 10), (1, R.FACE_PMC), None, 3),
+    "large": ((25, 26, 23), None, None, 30),
+    "large_restarted": ((25, 26, 23), None, None, 5),
+    "large_plane": ((40, 210, 1), None, None, 30),
+    "large_walls": ((25, 26, 23), (1, R.FACE_PEC), None, 30),
+    "large_smoothed": ((25, 26, 23), None, (R.SMOOTH_FACE7, 2, 0.5), 30),
+}
+
+
+@pytest.mark.parametrize("name", list(SOLVER_GRIDS))
+def test_operator_and_solve_on_both_forms(name):
+    """The operator within 1e-12 of the oracle's and the solve with its
+    iteration count and its E_theta to 1e-10, at the sizes where the
+    operator's form, its blocks or the solver's restarts change; a solve out
+    of iterations reports it and leaves E_theta at its guess."""
+    cells, wall, smoothing, restart = SOLVER_GRIDS[name]
+    lengths = tuple(0.25 * n for n in cells)
+    rng = np.random.default_rng(31)
+    qom = [-16.0, 1.0]
+    faces = [(R.FACE_PERIODIC,) * 2] * 3
+    periodic = [1, 1, 1]
+    if wall:
+        faces[wall[0]] = (wall[1],) * 2
+        periodic[wall[0]] = 0
+    arrays = [random_state(cells, lengths, 2, rng, vscale=0.05)[1] for _ in qom]
+    for a, q in zip(arrays, qom):
+        a["q"] = np.full(len(a["q"]), (1.0 if q > 0 else -1.0) * 0.25 ** 3 / 2 / (4 * np.pi))
+    counts = [len(a["q"]) for a in arrays]
+    b = cases.uniform_b(cells, (0.0, 0.2, 0.4), amplitude=0.3)
+    kw = dict(particle_periodic=periodic, field_faces=faces, smoothing=smoothing)
+    say("operator and solve", name)
+
+    def start(**more):
+        sim = gpu(cells, lengths, list(zip(qom, counts)), gmres_tolerance=1e-12, gmres_restart=restart, **kw, **more)
+        for s, a in enumerate(arrays):
+            sim.set_particles(s, a)
+        sim.set_field(R.FIELD_B, b)
+        sim.initialize()
+        return sim
+
+    ref = O.Sim(cells, lengths, qom, counts, 0.1, tol=1e-12, restart=restart, max_iterations=100, **kw)
+    for s, a in enumerate(arrays):
+        ref.set_particles(s, a)
+    ref.field("B")[:] = b
+    ref.initialize()
+    g = O.make_grid(cells, lengths, periodic, faces)
+    nx, ny, nz = cells
+    v = rng.normal(size=(3, nz + 1, ny + 1, nx + 1))
+    for axis, dim in ((0, 3), (1, 2), (2, 1)):
+        if not (wall and wall[0] == axis):
+            last = [slice(None)] * 4
+            first = [slice(None)] * 4
+            last[dim], first[dim] = -1, 0
+            v[tuple(last)] = v[tuple(first)]
+    ref.field("E")[:] = v.ravel()
+    ref.initialize()  # projects the constrained rows
+    v = ref.field("E").copy()
+    with start() as sim:
+        sim.set_field(R.FIELD_E, v)
+        sim.apply_operator(sim.device_field(R.FIELD_E), sim.device_field(R.FIELD_RHS))
+        out = sim.get_field(R.FIELD_RHS)
+        args = (ref.field("mass").copy(), 0.05, 4 * np.pi * 0.05, 1 / 0.25 ** 3, v)
+        want = O.maxwell_apply_smoothed(g, smoothing, *args) if smoothing else O.maxwell_apply(g, *args)
+        assert np.abs(out - want).max() <= 1e-12 * np.abs(want).max()
+        _, got = sim.solve()
+        rc, ro = ref.solve()
+        say("iterations", got["iterations"], "restart", restart)
+        assert rc == 0 and got["converged"] and got["iterations"] == ro.iterations
+        theta, want = sim.get_field(R.FIELD_ETHETA), ref.field("theta")
+        assert np.abs(theta - want).max() <= 1e-10 * np.abs(want).max()
+        assert abs(got["initial_residual"] - ro.initial_residual) <= 1e-10 * ro.initial_residual
+    limit = got["iterations"] - 1
+    with start(gmres_max_iterations=limit) as sim:
+        sim.set_field(R.FIELD_E, v)
+        rc, short = sim.solve(raise_on_failure=False)
+        assert rc == R.NOT_CONVERGED and not short["converged"] and short["iterations"] == limit
+        assert np.array_equal(sim.get_field(R.FIELD_ETHETA), v)
+    ref.close()
+
+
 @pytest.mark.parametrize("case", ["GEMHarris", "DoubleGEM"])
 def test_harris_load_matches_the_oracle(case):
     """tpic_mi_load_harris against the oracle's Harris profile: positions,

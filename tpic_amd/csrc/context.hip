@@ -137,7 +137,7 @@ void free_all(tpic_mi_context* h) {
   c.fork = c.join = nullptr;
   c.side_stream = nullptr;
   GmresWorkspace& g = c.gmres;
-  release(g.basis); release(g.x); release(g.b); release(g.r); release(g.image); release(g.values);
+  release(g.basis); release(g.x); release(g.image); release(g.arrivals);
   release(g.partials); release(g.state); release(g.curl_cells);
   if (g.controls) (void)hipHostFree(g.controls);
   if (c.host_word) (void)hipHostFree(c.host_word);
@@ -254,19 +254,17 @@ int allocate(tpic_mi_context* h) {
   }
   GmresWorkspace& gm = c.gmres;
   gm.count = unsigned(3 * nodes);
-  gm.blocks = unsigned(std::max<size_t>(1, std::min<size_t>((gm.count + 255) / 256, size_t(c.cus > 0 ? c.cus : 256) * 4)));
-  const size_t m = size_t(c.num.restart), batch = std::max<size_t>(m, 2);
+  gm.blocks = gmres_blocks(gm.count, c.cus);
+  const size_t m = size_t(c.num.restart);
   TPIC_ALLOC(gm.basis, (m + 1) * gm.count);
   TPIC_ALLOC(gm.x, gm.count);
-  TPIC_ALLOC(gm.b, gm.count);
-  TPIC_ALLOC(gm.r, gm.count);
   TPIC_ALLOC(gm.image, gm.count);
-  TPIC_ALLOC(gm.values, batch);
-  TPIC_ALLOC(gm.partials, batch * gm.blocks);
-  TPIC_ALLOC(gm.state, m * (m + 1) + 4 * m + 6);  // Hessenberg, rotations, rhs, coefficients, 5 stop words
+  TPIC_ALLOC(gm.partials, gmres_partial_words(c.num.restart, gm.blocks, operator_tail_blocks(g)));
+  TPIC_ALLOC(gm.state, gmres_state_words(c.num.restart));
+  TPIC_ALLOC(gm.arrivals, gmres_arrival_words(c.num.restart));
   TPIC_ALLOC(gm.curl_cells, 3 * cells);
 #undef TPIC_ALLOC
-  if ((rc = check_hip(c, hipHostMalloc(reinterpret_cast<void**>(&gm.controls), 8 * sizeof(double)), "pinned")))
+  if ((rc = check_hip(c, hipHostMalloc(reinterpret_cast<void**>(&gm.controls), 16 * sizeof(double)), "pinned")))
     return rc;
   if ((rc = check_hip(c, hipHostMalloc(reinterpret_cast<void**>(&c.host_word), sizeof(unsigned)), "pinned")))
     return rc;
@@ -293,6 +291,7 @@ int allocate(tpic_mi_context* h) {
   (void)hipMemsetAsync(c.mass, 0, size_t(kEntries) * g.vstride * sizeof(double), st);
   (void)hipMemsetAsync(c.cellbuf, 0, size_t(kCellRecord) * cells * sizeof(double), st);
   (void)hipMemsetAsync(c.validation, 0, sizeof(unsigned), st);
+  (void)hipMemsetAsync(gm.arrivals, 0, gmres_arrival_words(c.num.restart) * sizeof(unsigned), st);
   return check_hip(c, hipStreamSynchronize(st), "initial clear");
 }
 
@@ -730,14 +729,6 @@ int tpic_mi_solve(tpic_mi_context* h, tpic_mi_solve_result* r) {
   Context& c = h->ctx;
   int rc = launch_rhs(c);
   if (rc) return rc;
-  // The initial guess is E^n projected (enqueue_rhs_fields copies E into
-  // theta and projects it, maxwell_device.hpp:140-142): a field set with
-  // nonzero constrained rows still starts the solve in the constrained subspace.
-  if ((rc = check_hip(c, hipMemcpyAsync(c.etheta, c.e, 3 * size_t(c.grid.nodes()) * sizeof(double),
-                                        hipMemcpyDeviceToDevice, c.stream),
-                      "theta initial copy")))
-    return rc;
-  if ((rc = launch_zero_constrained(c, c.etheta))) return rc;
   tpic_mi_solve_result out{};
   rc = run_gmres(c, &out.converged, &out.iterations, &out.initial_residual, &out.residual, &out.rhs_norm,
                  &out.relative_residual);

@@ -4,24 +4,34 @@
 //
 // Algorithm of Gmres::host_blocking_solve
 // (include/tpic/ecsim/gmres/gmres_device.hpp:355-454): x0 = E^n, r = b - A x,
-// tolerance relative to |b| (scale 1 for b = 0); each restart normalises r;
+// tolerance relative to |b| (scale 1 for b = 0); each restart starts from r;
 // each Arnoldi step applies A, forms the projection dots against the basis in
 // one batch, orthogonalises by one classical Gram-Schmidt pass fused with the
-// squared norm, then one kernel normalises the new basis vector while block 0
-// thread 0 appends the column to the Hessenberg matrix and applies the Givens
-// rotations (ArnoldiLeastSquaresUpdate, :65-98). The reference's host reads
-// two control scalars per step; here that thread also tests them (the
-// estimate against the tolerance, the breakdown) and raises a stop word with
-// the step count, every kernel of a later step returns at once when the word
-// is up, and the host enqueues several steps between reads of the word: the
-// same steps run and stop where they would, with fewer host round trips.
-// After each restart the true residual |b - A x| decides
-// convergence; the solution is committed only when converged. Vectors hold
-// every interior node, periodic duplicates included (:133-137), so dots weight
-// shared nodes as the reference's compact vectors do.
+// squared norm, appends the column to the Hessenberg matrix and applies the
+// Givens rotations (ArnoldiLeastSquaresUpdate, :65-98). After each restart the
+// true residual |b - A x| decides convergence; the solution is committed only
+// when converged. Vectors hold every interior node, periodic duplicates
+// included (:133-137), so dots weight shared nodes as the reference's compact
+// vectors do.
 //
-// Reductions are deterministic: fixed block partials reduced by one block per
-// row in a fixed tree, no atomics.
+// A step is a chain of dependent passes over vectors that are small on all but
+// the largest grids, so what counts is their number. Basis vector j is kept as
+// the orthogonalised image w_j with its factor s_j = 1 / |w_j| beside it (the
+// operator's image, the dots and the update take the factor), so no pass
+// normalises. The dots are formed by the operator's kernel where it can
+// (operator_tail_blocks), else by k_dot_batch, and the last block of
+// k_orthogonalize to finish adds the squared norm and runs the Givens update. A step is two launches on small
+// grids and four on large ones (seven before; 16^3: the solve's 10 operator
+// calls and 8 steps took 340 us of kernels).
+//
+// The reference's host reads two control scalars per step. Here the Givens
+// update tests them (the estimate against the tolerance, the breakdown) and
+// raises a stop word, and the tests of the first and of the true residual are
+// kernels too: the host enqueues the first residual, a batch of steps, the
+// update, the true residual and the commit, each guarded by those words, and
+// reads the words once. The same steps run and stop where they would.
+//
+// Reductions are deterministic: fixed partials added in a fixed order.
 #include "internal.hpp"
 
 #include <cmath>
@@ -30,74 +40,153 @@ namespace tpic_mi {
 namespace {
 
 constexpr unsigned kThreads = 256;
+constexpr unsigned kWaves = kThreads / 64;
 constexpr unsigned kTile = 4;
+constexpr int kMaxColumns = 64;  // tpic_mi_config.gmres_restart's limit
+
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  return v;  // valid in lane 0
+}
 
 __device__ inline double block_reduce(double v, double* lds) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  v = wave_sum(v);
   const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   if (lane == 0) lds[wave] = v;
   __syncthreads();
   double sum = 0.0;
   if (threadIdx.x == 0)
-    for (unsigned w = 0; w < kThreads / 64; ++w) sum += lds[w];
+    for (unsigned w = 0; w < kWaves; ++w) sum += lds[w];
   __syncthreads();
   return sum;  // valid in thread 0
 }
 
-// Stop words of one Arnoldi restart cycle (after the Hessenberg state):
-// [0] residual estimate, [1] breakdown, [2] stop, [3] steps done at the stop,
-// [4] a non-finite recurrence.
-constexpr int kStatusWords = 5;
+__device__ __forceinline__ bool finite(double v) { return fabs(v) <= 1.7976931348623157e308; }
 
-__device__ inline bool stopped(const double* stop) { return stop && *stop != 0.0; }
+// The solver's words, doubles on the device read back in one copy.
+enum Word : int {
+  kEstimate,    // residual estimate of the last step
+  kBreakdown,   // 1: its image lay in the basis
+  kStop,        // 1: later steps do nothing
+  kSteps,       // steps of this restart when the stop was raised
+  kNonfinite,   // 1: a non-finite recurrence
+  kGo,          // 1: the restart's tail (update, true residual) is to run
+  kConverged,   // 1: the true residual met the tolerance
+  kTails,       // tails run
+  kDone,        // steps of the last tail
+  kDoneBreakdown,
+  kInitial2,    // |b - A x0|^2
+  kRhs2,        // |b|^2
+  kResidual2,   // |b - A x|^2 of the last tail
+  kAbsolute,    // the tolerance on the residual
+  kWords
+};
 
+// Device state of a solve: Hessenberg columns, rotations, right-hand side of
+// the least-squares problem, basis factors, words.
+struct SolverState {
+  double *h, *cosine, *sine, *g, *scale, *word;
+  int leading;  // entries of a Hessenberg column
+  double tolerance;
+};
+
+SolverState solver_state(const GmresWorkspace& w, int m, double tolerance) {
+  SolverState s;
+  s.leading = m + 1;
+  s.h = w.state;
+  s.cosine = s.h + size_t(m) * (m + 1);
+  s.sine = s.cosine + m;
+  s.g = s.sine + m;
+  s.scale = s.g + (m + 1);
+  s.word = s.scale + (m + 1);
+  s.tolerance = tolerance;
+  return s;
+}
+
+// The last block of a launch to finish adds what the others left. Only
+// `partials` values and the arrival counters (zero between launches) pass
+// between blocks within a launch: both are agent-scope accesses, which go past
+// the XCDs' caches, and a block waits for its stores of partials before it
+// arrives. (An agent-scope release instead writes back the XCD's whole L2 for
+// every block: 33 us instead of 20 for an orthogonalisation at 100,000 nodes.)
+__device__ __forceinline__ void put_partial(double* at, double v) {
+  __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_partial(const double* at) {
+  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Counters of one launch's arrivals, in words: a root, then one per kGroup
+// blocks, each on a cache line of its own. Arrivals at one address follow one
+// another at about 20 ns (1024 blocks at one counter: 20 us), so a block
+// arrives at its group's and the last of a group at the root.
+constexpr unsigned kGroup = 32, kCounterStride = 32, kMaxBlocks = 1024;
+constexpr unsigned kCounters = (1 + kMaxBlocks / kGroup) * kCounterStride;
+
+__device__ __forceinline__ bool arrive(unsigned* counter, unsigned expected) {
+  if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != expected - 1) return false;
+  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// True in every thread of the last of `blocks` blocks to get here. Thread 0's
+// wave must have stored the block's partials itself.
+__device__ __forceinline__ bool last_to_arrive(unsigned* counters, unsigned block, unsigned blocks, bool* lds) {
+  if (threadIdx.x == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned group = block / kGroup, begin = group * kGroup;
+    const unsigned size = blocks - begin < kGroup ? blocks - begin : kGroup;
+    *lds = arrive(counters + (1 + group) * kCounterStride, size) && arrive(counters, (blocks + kGroup - 1) / kGroup);
+  }
+  __syncthreads();
+  return *lds;
+}
+
+// Products of the image with the first `columns` basis vectors, kTile columns
+// per row of blocks; the last block of a row adds its partials into dots.
 __global__ __launch_bounds__(kThreads) void k_dot_batch(const double* __restrict__ basis,
-                                                        const double* __restrict__ image,
-                                                        double* __restrict__ partials, unsigned count,
-                                                        int columns, const double* __restrict__ stop) {
-  if (stopped(stop)) return;
-  __shared__ double lds[kThreads / 64];
-  for (unsigned first = blockIdx.y * kTile; first < unsigned(columns); first += gridDim.y * kTile) {
-    double sum[kTile] = {0.0, 0.0, 0.0, 0.0};
-    for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x) {
-      const double v = image[n];
-#pragma unroll
-      for (unsigned r = 0; r < kTile; ++r)
-        if (first + r < unsigned(columns)) sum[r] += basis[size_t(first + r) * count + n] * v;
-    }
+                                                        const double* __restrict__ image, double* partials,
+                                                        double* __restrict__ dots, unsigned* arrivals,
+                                                        unsigned count, unsigned columns, Guard guard) {
+  if (guard.skips()) return;
+  __shared__ double lds[kWaves][kTile];
+  __shared__ bool s_last;
+  const unsigned first = blockIdx.y * kTile;
+  double sum[kTile] = {0.0, 0.0, 0.0, 0.0};
+  for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x) {
+    const double v = image[n];
 #pragma unroll
     for (unsigned r = 0; r < kTile; ++r)
-      if (first + r < unsigned(columns)) {
-        const double total = block_reduce(sum[r], lds);
-        if (threadIdx.x == 0) partials[size_t(first + r) * gridDim.x + blockIdx.x] = total;
-      }
+      if (first + r < columns) sum[r] += basis[size_t(first + r) * count + n] * v;
   }
+  // The tile's sums with one barrier; lanes 0..3 of wave 0 store them.
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (unsigned r = 0; r < kTile; ++r) {
+    const double total = wave_sum(sum[r]);
+    if (lane == 0) lds[wave][r] = total;
+  }
+  __syncthreads();
+  if (threadIdx.x < kTile && first + threadIdx.x < columns) {
+    double total = 0.0;
+    for (unsigned w = 0; w < kWaves; ++w) total += lds[w][threadIdx.x];
+    put_partial(partials + size_t(first + threadIdx.x) * gridDim.x + blockIdx.x, total);
+  }
+  if (!last_to_arrive(arrivals + blockIdx.y * kCounters, blockIdx.x, gridDim.x, &s_last)) return;
+  const unsigned c = first + wave;  // a wave per column
+  double v = 0.0;
+  if (c < columns)
+    for (unsigned i = lane; i < gridDim.x; i += 64) v += get_partial(partials + size_t(c) * gridDim.x + i);
+  v = wave_sum(v);
+  if (c < columns && lane == 0) dots[c] = v;
 }
 
-// One block per row: sum of the row's partials; rows >= filled are zeroed.
-__global__ __launch_bounds__(kThreads) void k_reduce_rows(const double* __restrict__ partials,
-                                                          double* __restrict__ values, unsigned stride,
-                                                          unsigned count, unsigned filled,
-                                                          const double* __restrict__ stop) {
-  if (stopped(stop)) return;
-  __shared__ double lds[kThreads / 64];
-  const unsigned row = blockIdx.x;
-  if (row >= filled) {
-    if (threadIdx.x == 0) values[row] = 0.0;
-    return;
-  }
-  double s = 0.0;
-  for (unsigned i = threadIdx.x; i < count; i += blockDim.x) s += partials[size_t(row) * stride + i];
-  const double total = block_reduce(s, lds);
-  if (threadIdx.x == 0) values[row] = total;
-}
-
-// r = b - image; partial sums of |r|^2 (and |b|^2).
+// r = b - image; partial sums of |r|^2 and |b|^2 (rows 0 and 1).
 __global__ __launch_bounds__(kThreads) void k_residual(const double* __restrict__ b,
                                                        const double* __restrict__ image,
                                                        double* __restrict__ r, double* __restrict__ partials,
-                                                       unsigned count, int with_rhs) {
-  __shared__ double lds[kThreads / 64];
+                                                       unsigned count, Guard guard) {
+  if (guard.skips()) return;
+  __shared__ double lds[kWaves];
   double s0 = 0.0, s1 = 0.0;
   for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x) {
     const double bv = b[n];
@@ -106,128 +195,224 @@ __global__ __launch_bounds__(kThreads) void k_residual(const double* __restrict_
     s0 += v * v;
     s1 += bv * bv;
   }
-  const double t0 = block_reduce(s0, lds);
-  if (threadIdx.x == 0) partials[blockIdx.x] = t0;
-  if (with_rhs) {
-    const double t1 = block_reduce(s1, lds);
-    if (threadIdx.x == 0) partials[gridDim.x + blockIdx.x] = t1;
+  const double t0 = block_reduce(s0, lds), t1 = block_reduce(s1, lds);
+  if (threadIdx.x == 0) {
+    partials[blockIdx.x] = t0;
+    partials[gridDim.x + blockIdx.x] = t1;
   }
 }
 
-// Classical Gram-Schmidt against the first `columns` basis vectors with the
-// reduced dots; stores the image and its squared-norm partial; block 0 copies
-// the dots into the Hessenberg column.
-__global__ __launch_bounds__(kThreads) void k_orthogonalize(const double* __restrict__ basis,
-                                                            const double* __restrict__ dots,
-                                                            double* __restrict__ image,
-                                                            double* __restrict__ hcol,
-                                                            double* __restrict__ partials, unsigned count,
-                                                            int columns, const double* __restrict__ stop) {
-  if (stopped(stop)) return;
-  __shared__ double lds[kThreads / 64];
-  __shared__ double s_dots[64];
-  if (threadIdx.x < unsigned(columns) && threadIdx.x < 64) s_dots[threadIdx.x] = dots[threadIdx.x];
-  __syncthreads();
-  double norm2 = 0.0;
-  for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x) {
-    double value = image[n];
-    for (int c = 0; c < columns; ++c) value -= s_dots[c] * basis[size_t(c) * count + n];
-    image[n] = value;
-    norm2 += value * value;
+// One block: the residual's squared norm from its partials, the convergence
+// test, and the start of the next restart (its first basis vector is the
+// residual). `first` is the residual of the initial guess, whose right-hand
+// side norm also sets the tolerance; else the residual after a restart.
+__global__ __launch_bounds__(kThreads) void k_residual_test(const double* __restrict__ partials, unsigned blocks,
+                                                            SolverState s, int first, Guard guard) {
+  if (guard.skips()) return;
+  __shared__ double lds[kWaves];
+  double s0 = 0.0, s1 = 0.0;
+  for (unsigned i = threadIdx.x; i < blocks; i += kThreads) {
+    s0 += partials[i];
+    s1 += partials[blocks + i];
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0)
-    for (int row = 0; row < columns; ++row) hcol[row] = s_dots[row];
-  const double total = block_reduce(norm2, lds);
-  if (threadIdx.x == 0) partials[blockIdx.x] = total;
+  const double r2 = block_reduce(s0, lds), b2 = block_reduce(s1, lds);
+  if (threadIdx.x != 0) return;
+  double* w = s.word;
+  double absolute = w[kAbsolute];
+  bool good = finite(r2);
+  if (first) {
+    absolute = (b2 == 0.0 ? 1.0 : sqrt(b2)) * s.tolerance;
+    good = good && finite(b2);
+    w[kInitial2] = r2;
+    w[kRhs2] = b2;
+    w[kAbsolute] = absolute;
+    w[kNonfinite] = 0.0;
+    w[kTails] = 0.0;
+    w[kDone] = 0.0;
+    w[kDoneBreakdown] = 0.0;
+  } else {
+    w[kTails] += 1.0;
+    w[kDone] = w[kSteps];
+    w[kDoneBreakdown] = w[kBreakdown];
+  }
+  const double r = sqrt(r2);
+  const bool converged = good && r <= absolute;
+  w[kResidual2] = r2;
+  w[kConverged] = converged ? 1.0 : 0.0;
+  w[kStop] = converged || !good || (!first && w[kBreakdown] != 0.0) ? 1.0 : 0.0;
+  w[kGo] = 0.0;
+  w[kSteps] = 0.0;
+  w[kBreakdown] = 0.0;
+  s.g[0] = r;
+  s.scale[0] = r2 > 0.0 ? 1.0 / r : 0.0;
 }
 
-struct GivensTail {
-  int mode;  // 0: restart (rhs[0] = |r|), 1: Arnoldi update of column `step`
-  double* column;
-  double* cosine;
-  double* sine;
-  double* rhs;
-  double* status;  // kStatusWords stop words
-  int step;
-  double absolute;  // the tolerance on the residual estimate
-};
-
-__device__ void run_tail(const GivensTail& t, double norm2) {
-  if (t.mode == 0) {
-    t.rhs[0] = sqrt(norm2);
-    return;
-  }
-  const int step = t.step;
-  double* column = t.column;
+// The Givens update of column `step` with the squared norm of its
+// orthogonalised image (ArnoldiLeastSquaresUpdate, gmres_device.hpp:65-98) and
+// the host's test of the two controls (:431-441). `column` holds the column's
+// dots, `cosine` and `sine` the earlier rotations, all in LDS; `upper` is the
+// last entry of the rotated right-hand side so far.
+__device__ void append_column(const SolverState& s, int step, bool last, double norm2, double upper, double absolute,
+                              double* column, const double* cosine, const double* sine) {
   const double sub = sqrt(norm2);
-  column[step + 1] = sub;
   for (int row = 0; row < step; ++row) {
-    const double upper = column[row], lower = column[row + 1];
-    column[row] = t.cosine[row] * upper + t.sine[row] * lower;
-    column[row + 1] = -t.sine[row] * upper + t.cosine[row] * lower;
+    const double above = column[row], below = column[row + 1];
+    column[row] = cosine[row] * above + sine[row] * below;
+    column[row + 1] = -sine[row] * above + cosine[row] * below;
   }
   const double diagonal = column[step];
   const double den = hypot(diagonal, sub);
   const double c = den != 0.0 ? diagonal / den : 1.0;
-  const double s = den != 0.0 ? sub / den : 0.0;
-  t.cosine[step] = c;
-  t.sine[step] = s;
-  column[step] = c * diagonal + s * sub;
-  column[step + 1] = 0.0;
-  const double upper = t.rhs[step], lower = t.rhs[step + 1];
-  t.rhs[step] = c * upper + s * lower;
-  t.rhs[step + 1] = -s * upper + c * lower;
-  t.status[0] = fabs(t.rhs[step + 1]);
-  t.status[1] = sub == 0.0 ? 1.0 : 0.0;
-  // The host's test of the two controls (gmres_device.hpp:431-441).
-  const bool finite = t.status[0] <= 1.7976931348623157e308;
-  if (!finite || t.status[0] <= t.absolute || t.status[1] != 0.0) {
-    t.status[4] = finite ? 0.0 : 1.0;
-    t.status[3] = double(step + 1);
-    t.status[2] = 1.0;
+  const double sn = den != 0.0 ? sub / den : 0.0;
+  s.cosine[step] = c;
+  s.sine[step] = sn;
+  column[step] = c * diagonal + sn * sub;
+  s.g[step] = c * upper;
+  s.g[step + 1] = -sn * upper;
+  s.scale[step + 1] = sub > 0.0 ? 1.0 / sub : 0.0;
+  const double estimate = fabs(sn * upper);
+  const bool good = finite(estimate), breakdown = sub == 0.0;
+  s.word[kEstimate] = estimate;
+  if (!good || breakdown || estimate <= absolute || last) {
+    s.word[kNonfinite] = good ? 0.0 : 1.0;
+    s.word[kBreakdown] = breakdown ? 1.0 : 0.0;
+    s.word[kSteps] = double(step + 1);
+    s.word[kGo] = good ? 1.0 : 0.0;
+    s.word[kStop] = 1.0;
   }
 }
 
-// target = source / sqrt(norm2) (zero for a zero norm); block 0 thread 0 runs
-// the Givens tail first.
-__global__ __launch_bounds__(kThreads) void k_normalize(const double* __restrict__ source,
-                                                        const double* __restrict__ norm2,
-                                                        double* __restrict__ target, unsigned count,
-                                                        GivensTail tail, const double* __restrict__ stop) {
-  // A block that finds the word already up (raised by an earlier step, or by
-  // this step's tail) skips: the vector of a step past the stop is unused.
-  if (stopped(stop)) return;
-  const double n2 = norm2[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) run_tail(tail, n2);
-  const double scale = n2 > 0.0 ? 1.0 / sqrt(n2) : 0.0;
-  for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x)
-    target[n] = source[n] * scale;
-}
-
-__global__ void k_back_substitute(const double* __restrict__ h, const double* __restrict__ rhs,
-                                  double* __restrict__ y, int leading, int columns) {
-  for (int row = columns - 1; row >= 0; --row) {
-    double sum = 0.0;
-    for (int col = row + 1; col < columns; ++col) sum += h[size_t(col) * leading + row] * y[col];
-    const double d = h[size_t(row) * leading + row];
-    y[row] = d != 0.0 ? (rhs[row] - sum) / d : 0.0;
+// Classical Gram-Schmidt of the image against the basis vectors 0 .. step:
+// w_{step+1} = image - sum_c (s_c dot_c) s_c w_c, the dots added here from
+// `rows` partials per column. The last block to arrive adds the blocks'
+// squared norms and appends the column. The vectors' first values are
+// requested before the dots.
+__global__ __launch_bounds__(kThreads) void k_orthogonalize(const double* __restrict__ basis,
+                                                            const double* __restrict__ image,
+                                                            double* __restrict__ target,
+                                                            const double* __restrict__ dots, unsigned rows,
+                                                            double* norms, unsigned* arrivals, unsigned count,
+                                                            int step, int last, SolverState s, Guard guard) {
+  __shared__ double lds[kWaves];
+  __shared__ double s_column[kMaxColumns + 1], s_weight[kMaxColumns], s_cosine[kMaxColumns], s_sine[kMaxColumns];
+  __shared__ bool s_last;
+  const int columns = step + 1;
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const unsigned n0 = blockIdx.x * blockDim.x + threadIdx.x;
+  // What does not wait for the dots is requested first: the first values of
+  // the image and of up to kAhead basis vectors, the factors, the tail's state.
+  constexpr int kAhead = 8;
+  double value = 0.0, ahead[kAhead];
+#pragma unroll
+  for (int c = 0; c < kAhead; ++c) ahead[c] = c < columns && n0 < count ? basis[size_t(c) * count + n0] : 0.0;
+  if (n0 < count) value = image[n0];
+  const double scale = int(lane) < columns ? s.scale[lane] : 0.0;
+  const double upper = s.g[step], absolute = s.word[kAbsolute];
+  const bool skip = guard.skips();
+  double dot[kMaxColumns / kWaves];
+#pragma unroll
+  for (int t = 0; t < int(kMaxColumns / kWaves); ++t) {
+    const int c = int(wave) + t * int(kWaves);
+    dot[t] = 0.0;
+    if (c < columns)
+      for (unsigned i = lane; i < rows; i += 64) dot[t] += dots[size_t(c) * rows + i];
   }
+  if (int(threadIdx.x) < step) {
+    s_cosine[threadIdx.x] = s.cosine[threadIdx.x];
+    s_sine[threadIdx.x] = s.sine[threadIdx.x];
+  }
+  if (skip) return;
+#pragma unroll
+  for (int t = 0; t < int(kMaxColumns / kWaves); ++t) {
+    const int c = int(wave) + t * int(kWaves);
+    if (c < columns) {
+      const double v = rows > 1 ? wave_sum(dot[t]) : dot[t], by = __shfl(scale, c, 64);
+      if (lane == 0) {
+        s_column[c] = by * v;
+        s_weight[c] = by * (by * v);
+      }
+    }
+  }
+  __syncthreads();
+  double norm2 = 0.0;
+  if (n0 < count) {
+#pragma unroll
+    for (int c = 0; c < kAhead; ++c)
+      if (c < columns) value -= s_weight[c] * ahead[c];
+    for (int c = kAhead; c < columns; ++c) value -= s_weight[c] * basis[size_t(c) * count + n0];
+    target[n0] = value;
+    norm2 = value * value;
+  }
+  for (unsigned n = n0 + gridDim.x * blockDim.x; n < count; n += gridDim.x * blockDim.x) {
+    value = image[n];
+#pragma unroll 4
+    for (int c = 0; c < columns; ++c) value -= s_weight[c] * basis[size_t(c) * count + n];
+    target[n] = value;
+    norm2 += value * value;
+  }
+  const double total = block_reduce(norm2, lds);
+  if (threadIdx.x == 0) put_partial(norms + blockIdx.x, total);
+  if (!last_to_arrive(arrivals, blockIdx.x, gridDim.x, &s_last)) return;
+  double v = 0.0;
+  for (unsigned i = threadIdx.x; i < gridDim.x; i += kThreads) v += get_partial(norms + i);
+  const double sum = block_reduce(v, lds);
+  if (threadIdx.x == 0) append_column(s, step, last != 0, sum, upper, absolute, s_column, s_cosine, s_sine);
+  __syncthreads();
+  double* const column = s.h + size_t(step) * s.leading;
+  if (int(threadIdx.x) <= step) column[threadIdx.x] = s_column[threadIdx.x];
 }
 
-__global__ __launch_bounds__(kThreads) void k_update(const double* __restrict__ basis,
-                                                     const double* __restrict__ y, double* __restrict__ x,
-                                                     unsigned count, int columns) {
-  __shared__ double s_y[64];
-  if (threadIdx.x < unsigned(columns) && threadIdx.x < 64) s_y[threadIdx.x] = y[threadIdx.x];
+// x_out = x_in + sum_c y_c s_c w_c with the least-squares solution y of the
+// restart's steps, which every block solves for by itself: the triangle goes
+// to LDS and a lane per row takes the back substitution.
+__global__ __launch_bounds__(kThreads) void k_update(const double* __restrict__ basis, const double* x_in,
+                                                     double* x_out, unsigned count, SolverState s, Guard guard) {
+  if (guard.skips()) return;
+  __shared__ double s_h[kMaxColumns * kMaxColumns];
+  __shared__ double s_y[kMaxColumns];
+  const int columns = int(s.word[kSteps]);
+  for (int t = int(threadIdx.x); t < columns * columns; t += int(kThreads))
+    s_h[t] = s.h[size_t(t / columns) * s.leading + t % columns];
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int row = int(threadIdx.x);
+    double rhs = row < columns ? s.g[row] : 0.0;
+    for (int col = columns - 1; col >= 0; --col) {
+      const double d = s_h[col * columns + col];
+      const double y = d != 0.0 ? __shfl(rhs, col, 64) / d : 0.0;
+      if (row < col) rhs -= s_h[col * columns + row] * y;
+      if (row == col) s_y[col] = y * s.scale[col];
+    }
+  }
   __syncthreads();
   for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x) {
-    double value = x[n];
+    double value = x_in[n];
+#pragma unroll 4
     for (int c = 0; c < columns; ++c) value += s_y[c] * basis[size_t(c) * count + n];
-    x[n] = value;
+    x_out[n] = value;
   }
+}
+
+__global__ __launch_bounds__(kThreads) void k_commit(const double* __restrict__ x, double* __restrict__ solution,
+                                                     unsigned count, Guard guard) {
+  if (guard.skips()) return;
+  for (unsigned n = blockIdx.x * blockDim.x + threadIdx.x; n < count; n += gridDim.x * blockDim.x) solution[n] = x[n];
 }
 
 }  // namespace
+
+// Words of GmresWorkspace::arrivals: the orthogonalisation's counters, then
+// those of each row of k_dot_batch's blocks; and the blocks of both.
+size_t gmres_arrival_words(int m) { return (1 + size_t(m + kTile - 1) / kTile) * kCounters; }
+unsigned gmres_blocks(unsigned count, int cus) {
+  return std::max(1u, std::min({(count + kThreads - 1) / kThreads, unsigned(cus > 0 ? cus : 256) * 4, kMaxBlocks}));
+}
+// Doubles of GmresWorkspace::partials: dots per block, norms per block, dots.
+size_t gmres_partial_words(int m, unsigned blocks, unsigned tail_blocks) {
+  return size_t(std::max(m, 2)) * std::max(blocks, tail_blocks) + blocks + size_t(m);
+}
+// Doubles of GmresWorkspace::state.
+size_t gmres_state_words(int m) { return size_t(m) * (m + 1) + 4 * size_t(m) + 2 + kWords; }
 
 int run_gmres(Context& ctx, int* converged_out, int* iterations_out, double* initial_out, double* residual_out,
               double* rhs_norm_out, double* relative_out) {
@@ -241,118 +426,106 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
   hipStream_t st = ctx.stream;
   const unsigned n = w.count;
   const int m = ctx.num.restart;
-  const unsigned blocks = w.blocks;
-  const unsigned batch = unsigned(m > 2 ? m : 2);
-  double* h = w.state;
-  double* cs = h + size_t(m) * (m + 1);
-  double* sn = cs + m;
-  double* g = sn + m;
-  double* y = g + (m + 1);
-  double* status = y + m;
+  const SolverState s = solver_state(w, m, ctx.num.gmres_tol);
+  const unsigned tail_blocks = operator_tail_blocks(ctx.grid);
+  const unsigned rows = tail_blocks ? tail_blocks : w.blocks;  // partials per dot or norm
+  double* const basis = w.basis;
+  double* const norms = w.partials + size_t(std::max(m, 2)) * rows;
+  double* const dots = norms + w.blocks;
   int rc = 0;
 #define TPIC_TRY(expr, what)             \
   do {                                  \
     rc = check_hip(ctx, (expr), what);  \
     if (rc) return rc;                  \
   } while (0)
-  auto read_words = [&](const double* src, int words, double* out) -> int {
-    int e = check_hip(ctx, hipMemcpyAsync(w.controls, src, size_t(words) * sizeof(double), hipMemcpyDeviceToHost, st),
-                      "gmres readback");
-    if (e) return e;
-    e = check_hip(ctx, hipStreamSynchronize(st), "gmres readback");
-    if (e) return e;
-    for (int k = 0; k < words; ++k) out[k] = w.controls[k];
-    return 0;
+  // The first basis vector and the test of the residual b - A x.
+  auto residual = [&](const double* x, int first, Guard guard) -> int {
+    OperatorCall call;
+    call.guard = guard;
+    if (tail_blocks) {
+      call.epilogue = OperatorEpilogue::residual;
+      call.tail.rhs = rhs_in;
+      call.tail.partials = w.partials;
+      if (int e = launch_operator(ctx, x, basis, call)) return e;
+    } else {
+      if (int e = launch_operator(ctx, x, w.image, call)) return e;
+      k_residual<<<w.blocks, kThreads, 0, st>>>(rhs_in, w.image, basis, w.partials, n, guard);
+      if (int e = check_hip(ctx, hipGetLastError(), "gmres residual")) return e;
+    }
+    k_residual_test<<<1, kThreads, 0, st>>>(w.partials, rows, s, first, guard);
+    return check_hip(ctx, hipGetLastError(), "gmres residual test");
   };
-  auto read_two = [&](const double* src, double out[2]) -> int { return read_words(src, 2, out); };
-  auto residual = [&](bool with_rhs, double out[2]) -> int {
-    int e = launch_operator(ctx, w.x, w.image);
-    if (e) return e;
-    k_residual<<<blocks, kThreads, 0, st>>>(w.b, w.image, w.r, w.partials, n, with_rhs ? 1 : 0);
-    if ((e = check_hip(ctx, hipGetLastError(), "gmres residual"))) return e;
-    k_reduce_rows<<<batch, kThreads, 0, st>>>(w.partials, w.values, blocks, blocks, with_rhs ? 2u : 1u, nullptr);
-    if ((e = check_hip(ctx, hipGetLastError(), "gmres reduce"))) return e;
-    return read_two(w.values, out);
+  auto arnoldi = [&](int col, bool last) -> int {
+    const Guard running{s.word + kStop, 1.0};
+    OperatorCall call;
+    call.scale = s.scale + col;
+    call.guard = running;
+    if (tail_blocks) {
+      call.epilogue = OperatorEpilogue::dots;
+      call.tail.basis = basis;
+      call.tail.columns = unsigned(col + 1);
+      call.tail.partials = w.partials;
+    }
+    if (int e = launch_operator(ctx, basis + size_t(col) * n, w.image, call)) return e;
+    if (!tail_blocks) {
+      const dim3 dgrid(w.blocks, unsigned((col + 1 + kTile - 1) / kTile));
+      k_dot_batch<<<dgrid, kThreads, 0, st>>>(basis, w.image, w.partials, dots, w.arrivals + kCounters, n, unsigned(col + 1),
+                                              running);
+      if (int e = check_hip(ctx, hipGetLastError(), "gmres dots")) return e;
+    }
+    k_orthogonalize<<<w.blocks, kThreads, 0, st>>>(basis, w.image, basis + size_t(col + 1) * n,
+                                                   tail_blocks ? w.partials : dots, tail_blocks ? rows : 1u, norms,
+                                                   w.arrivals, n, col, last ? 1 : 0, s, running);
+    return check_hip(ctx, hipGetLastError(), "gmres orthogonalize");
+  };
+  // A restart's end, done once its stop word is up: update, true residual
+  // (into the next restart's first basis vector), commit.
+  auto finish = [&](const double* x) -> int {
+    const Guard going{s.word + kGo, 0.0};
+    k_update<<<w.blocks, kThreads, 0, st>>>(basis, x, w.x, n, s, going);
+    if (int e = check_hip(ctx, hipGetLastError(), "gmres update")) return e;
+    if (int e = residual(w.x, 0, going)) return e;
+    k_commit<<<w.blocks, kThreads, 0, st>>>(w.x, solution, n, Guard{s.word + kConverged, 0.0});
+    return check_hip(ctx, hipGetLastError(), "gmres commit");
   };
   phase_begin(ctx, Phase::solve);
-  TPIC_TRY(hipMemcpyAsync(w.x, solution, n * sizeof(double), hipMemcpyDeviceToDevice, st), "gmres x");
-  TPIC_TRY(hipMemcpyAsync(w.b, rhs_in, n * sizeof(double), hipMemcpyDeviceToDevice, st), "gmres b");
-  double two[2];
-  if ((rc = residual(true, two))) return rc;
-  if (!std::isfinite(two[0]) || !std::isfinite(two[1]) || two[0] < 0 || two[1] < 0)
-    return fail(ctx, -3, "GMRES: nonfinite initial residual");
-  double res = std::sqrt(two[0]);
-  const double initial = res, rhs_norm = std::sqrt(two[1]);
-  const double scale = rhs_norm == 0.0 ? 1.0 : rhs_norm;
-  const double absolute = scale * ctx.num.gmres_tol;
-  bool converged = res <= absolute;
-  int iterations = 0;
-  const size_t state_words = size_t(m) * (m + 1) + 4 * size_t(m) + 1 + kStatusWords;
-  // Steps enqueued between two reads of the stop word (one by one with
-  // smoothing, whose kernels do not see the word).
-  const int steps_per_read = ctx.num.smoothing ? 1 : 8;
-  double* basis = w.basis;
+  if ((rc = residual(solution, 1, Guard{}))) return rc;
+  // Steps enqueued between two reads of the words.
+  constexpr int kStepsPerRead = 8;
+  bool converged = false, first_read = true;
+  int iterations = 0, enqueued = 0, tails = 0;
+  double word[kWords];
   while (!converged && iterations < ctx.num.max_iterations) {
-    TPIC_TRY(hipMemsetAsync(w.state, 0, state_words * sizeof(double), st), "gmres state");
-    // Restart: basis 0 = r / |r| with |r|^2 still in values[0]; rhs[0] = |r|.
-    GivensTail restart{0, nullptr, nullptr, nullptr, g, nullptr, 0, 0.0};
-    k_normalize<<<blocks, kThreads, 0, st>>>(w.r, w.values, basis, n, restart, nullptr);
-    TPIC_TRY(hipGetLastError(), "gmres restart");
     const int columns = std::min(m, ctx.num.max_iterations - iterations);
-    const double* stop = steps_per_read > 1 ? status + 2 : nullptr;
-    int completed = 0;
-    bool breakdown = false;
-    int enqueued = 0;
-    while (enqueued < columns) {
-      const int upto = std::min(columns, enqueued + steps_per_read);
-      for (int col = enqueued; col < upto; ++col) {
-        if ((rc = launch_operator(ctx, basis + size_t(col) * n, w.image, stop))) return rc;
-        const dim3 dgrid(blocks, unsigned((col + 1 + kTile - 1) / kTile));
-        k_dot_batch<<<dgrid, kThreads, 0, st>>>(basis, w.image, w.partials, n, col + 1, stop);
-        TPIC_TRY(hipGetLastError(), "gmres dots");
-        k_reduce_rows<<<batch, kThreads, 0, st>>>(w.partials, w.values, blocks, blocks, unsigned(col + 1), stop);
-        TPIC_TRY(hipGetLastError(), "gmres reduce");
-        double* hcol = h + size_t(col) * (m + 1);
-        k_orthogonalize<<<blocks, kThreads, 0, st>>>(basis, w.values, w.image, hcol, w.partials, n, col + 1, stop);
-        TPIC_TRY(hipGetLastError(), "gmres orthogonalize");
-        k_reduce_rows<<<batch, kThreads, 0, st>>>(w.partials, w.values, blocks, blocks, 1u, stop);
-        TPIC_TRY(hipGetLastError(), "gmres reduce");
-        GivensTail arnoldi{1, hcol, cs, sn, g, status, col, absolute};
-        k_normalize<<<blocks, kThreads, 0, st>>>(w.image, w.values, basis + size_t(col + 1) * n, n, arnoldi, stop);
-        TPIC_TRY(hipGetLastError(), "gmres normalize");
-      }
-      enqueued = upto;
-      double word[kStatusWords];
-      if ((rc = read_words(status, kStatusWords, word))) return rc;
-      if (word[4] != 0.0) return fail(ctx, -3, "GMRES: nonfinite Arnoldi recurrence");
-      if (word[2] != 0.0) {
-        completed = int(word[3]);
-        breakdown = word[1] != 0.0;
-        break;
-      }
-      completed = enqueued;
-    }
-    k_back_substitute<<<1, 1, 0, st>>>(h, g, y, m + 1, completed);
-    TPIC_TRY(hipGetLastError(), "gmres back substitution");
-    k_update<<<blocks, kThreads, 0, st>>>(basis, y, w.x, n, completed);
-    TPIC_TRY(hipGetLastError(), "gmres update");
-    iterations += completed;
-    // Always verify b - A x after an accepted update.
-    if ((rc = residual(false, two))) return rc;
-    if (!std::isfinite(two[0]) || two[0] < 0) return fail(ctx, -3, "GMRES: nonfinite residual");
-    res = std::sqrt(two[0]);
-    converged = res <= absolute;
-    if (breakdown && !converged) break;
+    const int upto = std::min(columns, enqueued + kStepsPerRead);
+    for (int col = enqueued; col < upto; ++col)
+      if ((rc = arnoldi(col, col + 1 == columns))) return rc;
+    enqueued = upto;
+    if ((rc = finish(tails ? w.x : solution))) return rc;
+    TPIC_TRY(hipMemcpyAsync(w.controls, s.word, kWords * sizeof(double), hipMemcpyDeviceToHost, st),
+             "gmres readback");
+    TPIC_TRY(hipStreamSynchronize(st), "gmres readback");
+    for (int k = 0; k < kWords; ++k) word[k] = w.controls[k];
+    if (first_read && (!std::isfinite(word[kInitial2]) || !std::isfinite(word[kRhs2])))
+      return fail(ctx, -3, "GMRES: nonfinite initial residual");
+    first_read = false;
+    if (word[kNonfinite] != 0.0) return fail(ctx, -3, "GMRES: nonfinite Arnoldi recurrence");
+    converged = word[kConverged] != 0.0;
+    if (int(word[kTails]) == tails) continue;  // converged from the start, or the restart goes on
+    tails = int(word[kTails]);
+    iterations += int(word[kDone]);
+    enqueued = 0;
+    if (!std::isfinite(word[kResidual2])) return fail(ctx, -3, "GMRES: nonfinite residual");
+    if (word[kDoneBreakdown] != 0.0) break;
   }
-  if (converged)
-    TPIC_TRY(hipMemcpyAsync(solution, w.x, n * sizeof(double), hipMemcpyDeviceToDevice, st), "gmres commit");
   phase_end(ctx, Phase::solve);
+  const double res = std::sqrt(word[kResidual2]), rhs_norm = std::sqrt(word[kRhs2]);
   *converged_out = converged ? 1 : 0;
   *iterations_out = iterations;
-  *initial_out = initial;
+  *initial_out = std::sqrt(word[kInitial2]);
   *residual_out = res;
   *rhs_norm_out = rhs_norm;
-  *relative_out = res / scale;
+  *relative_out = res / (rhs_norm == 0.0 ? 1.0 : rhs_norm);
   return 0;
 #undef TPIC_TRY
 }

@@ -75,13 +75,11 @@ struct GmresWorkspace {
   unsigned blocks = 0;      // reduction blocks
   double* basis = nullptr;  // [(restart + 1) * count]
   double* x = nullptr;      // solution being updated
-  double* b = nullptr;      // right-hand side
-  double* r = nullptr;      // residual
   double* image = nullptr;  // operator image
-  double* values = nullptr;    // [max(restart, 2)] reduced batch
-  double* partials = nullptr;  // [max(restart, 2) * blocks]
-  double* state = nullptr;     // Hessenberg, cos, sin, rhs, coefficients, status
-  double* controls = nullptr;  // pinned host [8]
+  double* partials = nullptr;  // gmres_partial_words
+  double* state = nullptr;     // Hessenberg, rotations, right-hand side, basis factors, words
+  unsigned* arrivals = nullptr;  // blocks of a running launch that are done (0 between launches)
+  double* controls = nullptr;  // pinned host copy of the words
   double* curl_cells = nullptr;   // [3 * cells] scratch of the operator
 };
 
@@ -200,19 +198,49 @@ int launch_assemble(Context& ctx);
 int launch_cell_to_node(Context& ctx);
 int launch_zero_constrained(Context& ctx, double* v);  // no-op without walls
 int launch_rhs(Context& ctx);
-// stop: a device word that, once nonzero, makes the launch do nothing (the
-// GMRES stop word; ignored with smoothing).
-int launch_operator(Context& ctx, const double* in, double* out, const double* stop = nullptr);
+// A device word that decides whether a launch does anything: it returns at
+// once while the word holds `skip` (the solver's words are 0 or 1).
+struct Guard {
+  const double* word = nullptr;
+  double skip = 0.0;
+  __device__ bool skips() const { return word && *word == skip; }
+};
+// What the solver wants of an operator image: products with `columns` basis
+// vectors of 3 nodes() values (kDots: row c of partials holds one value per
+// block), or rhs - image in its place with the blocks' parts of its squared
+// norm and of rhs's in rows 0 and 1 (kResidual).
+struct OperatorTail {
+  const double* basis = nullptr;
+  unsigned columns = 0;
+  const double* rhs = nullptr;
+  double* partials = nullptr;
+};
+enum class OperatorEpilogue : int { plain = 0, dots = 1, residual = 2 };
+struct OperatorCall {
+  const double* scale = nullptr;  // device factor of the image, or null
+  Guard guard{};
+  OperatorEpilogue epilogue = OperatorEpilogue::plain;
+  OperatorTail tail{};
+};
+// Blocks (values per row of partials) of an operator whose kernel takes the
+// epilogue, or 0 on grids whose kernel does not: the caller then works on
+// the plain image.
+unsigned operator_tail_blocks(const Grid& g);
+int launch_operator(Context& ctx, const double* in, double* out, const OperatorCall& call = {});
 // The configured smoothing S(src) of a node vector (ctx.num.smoothing must be
 // set; constrained rows of src read as zero, those of every pass zeroed): the
 // passes alternate between smooth_a and smooth_b, starting with the one src
 // is not, and the last writes into dst when dst is given. *result: where the
 // result is.
-int launch_smooth(Context& ctx, const double* src, double* dst, const double** result);
+int launch_smooth(Context& ctx, const double* src, double* dst, const double** result, Guard guard = {});
 int launch_next_fields(Context& ctx);
 int launch_energy(Context& ctx, double* out);  // out: W_E, W_B, K per species
 int launch_scalars(Context& ctx, double* out);
 int launch_moments(Context& ctx, int species, unsigned selected, double* out);  // out: 10 x nodes, device  // out: W_E, W_B, then K, charge, momentum x y z per species
+size_t gmres_state_words(int restart);
+size_t gmres_arrival_words(int restart);
+unsigned gmres_blocks(unsigned count, int cus);
+size_t gmres_partial_words(int restart, unsigned blocks, unsigned tail_blocks);
 int run_gmres(Context& ctx, int* converged, int* iterations, double* initial_residual,
               double* residual, double* rhs_norm, double* relative);
 // GMRES on A x = rhs (A^T with ctx.transposed_operator): x holds the initial

@@ -56,13 +56,12 @@ __device__ __forceinline__ void curl_of(const Samples* s, const Grid& g, double&
   z = derivative<NodeSource>(s[1], 0, g.ix) - derivative<NodeSource>(s[0], 1, g.iy);
 }
 
-// Cell (i,j,k) from its 8 nodes (all interior, no wrap needed).
-__device__ __forceinline__ void n2c_at(const Grid& g, const double* __restrict__ v, int i, int j, int k, double& x,
-                                       double& y, double& z) {
+// The 8 nodes of cell (i,j,k), all interior (no wrap needed).
+__device__ __forceinline__ void load_cell_nodes(const Grid& g, const double* __restrict__ v, int i, int j, int k,
+                                                Samples (&s)[3]) {
   const unsigned nodes = g.nodes();
   const unsigned sy = unsigned(g.nx + 1), sz = sy * unsigned(g.ny + 1);
   const unsigned n0 = g.node(i, j, k);
-  Samples s[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const double* f = v + size_t(c) * nodes;
@@ -75,6 +74,12 @@ __device__ __forceinline__ void n2c_at(const Grid& g, const double* __restrict__
     s[c].yz = f[n0 + sz + sy];
     s[c].xyz = f[n0 + sz + sy + 1];
   }
+}
+
+__device__ __forceinline__ void n2c_at(const Grid& g, const double* __restrict__ v, int i, int j, int k, double& x,
+                                       double& y, double& z) {
+  Samples s[3];
+  load_cell_nodes(g, v, i, j, k, s);
   curl_of<true>(s, g, x, y, z);
 }
 
@@ -128,8 +133,8 @@ __device__ __forceinline__ void c2n_at(const Grid& g, const double* __restrict__
 }
 
 __global__ __launch_bounds__(kThreads) void k_curl_n2c(Grid g, const double* __restrict__ v,
-                                                       double* __restrict__ out, const double* __restrict__ stop) {
-  if (stop && *stop != 0.0) return;
+                                                       double* __restrict__ out, Guard guard) {
+  if (guard.skips()) return;
   const unsigned cells = g.cells();
   for (unsigned c = blockIdx.x * blockDim.x + threadIdx.x; c < cells; c += gridDim.x * blockDim.x) {
     const int i = int(c % unsigned(g.nx)), j = int((c / unsigned(g.nx)) % unsigned(g.ny)),
@@ -266,7 +271,8 @@ __device__ __forceinline__ AxisImages axis_images(const Grid& g, int axis, int i
 template <int Op, bool Walls>
 __global__ __launch_bounds__(kThreads) void k_smooth(Grid g, const double* __restrict__ src,
                                                      double* __restrict__ dst, double alpha, double beta,
-                                                     unsigned* __restrict__ validation) {
+                                                     unsigned* __restrict__ validation, Guard guard) {
+  if (guard.skips()) return;
   const unsigned nodes = g.nodes();
   const unsigned sx = unsigned(g.nx + 1), sy = unsigned(g.ny + 1);
   unsigned flags = 0;
@@ -305,11 +311,15 @@ __global__ __launch_bounds__(kThreads) void k_smooth(Grid g, const double* __res
   if (flags) atomicOr(validation, flags);
 }
 
+// The right-hand side, and the solve's initial guess E^n with its constrained
+// rows zeroed (enqueue_rhs_fields copies E into theta and projects it,
+// maxwell_device.hpp:140-142): a field set with nonzero constrained rows
+// still starts the solve in the constrained subspace.
 template <bool Walls>
 __global__ __launch_bounds__(kThreads) void k_rhs(Grid g, const double* __restrict__ e, const double* __restrict__ b,
                                                   const double* __restrict__ current, double delta,
                                                   double current_factor, double* __restrict__ rhs,
-                                                  unsigned* __restrict__ validation) {
+                                                  double* __restrict__ theta, unsigned* __restrict__ validation) {
   const unsigned nodes = g.nodes();
   const unsigned sx = unsigned(g.nx + 1), sy = unsigned(g.ny + 1);
   unsigned flags = 0;
@@ -320,18 +330,21 @@ __global__ __launch_bounds__(kThreads) void k_rhs(Grid g, const double* __restri
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const size_t at = size_t(c) * nodes + n;
-      double value = 1.0 * e[at] + delta * cv[c] + (-current_factor) * current[at];
-      if (Walls && g.constrained_row(c, i, j, k)) value = 0.0;
+      const double start = e[at];
+      double value = 1.0 * start + delta * cv[c] + (-current_factor) * current[at];
+      const bool held = Walls && g.constrained_row(c, i, j, k);
+      if (held) value = 0.0;
       rhs[at] = value;
+      theta[at] = held ? 0.0 : start;
       if (!finite_value(value)) flags |= kInvalidField;
     }
   }
   if (flags) atomicOr(validation, flags);
 }
 
-__constant__ int c_offsets[kStencils][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 0},
-                                            {1, -1, 0}, {1, 0, 1}, {1, 0, -1}, {0, 1, 1}, {0, 1, -1},
-                                            {1, -1, 1}, {1, 1, -1}, {-1, 1, 1}, {1, 1, 1}};
+constexpr int c_offsets[kStencils][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 0},
+                                         {1, -1, 0}, {1, 0, 1}, {1, 0, -1}, {0, 1, 1}, {0, 1, -1},
+                                         {1, -1, 1}, {1, 1, -1}, {-1, 1, 1}, {1, 1, 1}};
 
 // image = 1*v + d2*curl_C2N(curl_cells) + k*(1/V)*M v at every interior node.
 // M is read in its storage type (double, or float for the mixed forms); the
@@ -340,72 +353,114 @@ __constant__ int c_offsets[kStencils][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0,
 // 32 rows are 6% faster than plane order for the FP64 matrix, 4% for FP32).
 constexpr unsigned kApplyTileRows = 16;
 
-// (1/V) f_g (M v) at node (i, j, kk) = n: the centre block, then per stencil
-// the forward block times v(i + o) and the backward block of the neighbour
-// vertex (not transposed) times v(i - o); FP64 products and sums.
-// With Transposed every 3 x 3 block enters transposed: (1/V) M^T v, the mass
-// part of the adjoint operator (the backward blocks are the forward pair's,
-// not transposed, so M^T needs the transpose of every block).
+// Node images of the neighbours of a node along each axis (offsets -1, 0,
+// +1): on a wall axis the reflection through the wall node, else the periodic
+// image.
+struct NodeImages {
+  int x[3], y[3], z[3];
+};
+
+template <bool Walls>
+__device__ __forceinline__ NodeImages node_images(const Grid& g, int i, int j, int k) {
+  NodeImages m;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    m.x[d] = d == 1 ? i : (Walls ? node_image(g, 0, i + d - 1, g.nx) : wrap_node(i + d - 1, g.nx));
+    m.y[d] = d == 1 ? j : (Walls ? node_image(g, 1, j + d - 1, g.ny) : wrap_node(j + d - 1, g.ny));
+    m.z[d] = d == 1 ? k : (Walls ? node_image(g, 2, k + d - 1, g.nz) : wrap_node(k + d - 1, g.nz));
+  }
+  return m;
+}
+
+// The vertex of a node and the vertex strides of its axes. Along an axis of
+// one cell all four stored vertices are images of vertex 0 (the assembly sums
+// the same cells in the same order for each), so the axis is read at vertex 0
+// alone: the matrix of a plane is one plane's records, not four (the apply of
+// a 512 x 512 x 1 grid took 179 us through all the images).
+struct VertexWalk {
+  int v0, sx, sy, sz;
+};
+
+__device__ __forceinline__ VertexWalk vertex_walk(const Grid& g, int i, int j, int k) {
+  VertexWalk w;
+  w.sx = g.nx == 1 ? 0 : 1;
+  w.sy = g.ny == 1 ? 0 : g.nx + 3;
+  w.sz = g.nz == 1 ? 0 : (g.nx + 3) * (g.ny + 3);
+  w.v0 = int(g.vertex(g.nx == 1 ? 0 : i, g.ny == 1 ? 0 : j, g.nz == 1 ? 0 : k));
+  return w;
+}
+
+// Stencils First .. Last - 1 of M v at a node: per stencil the forward block
+// times v(i + o) and the backward block of the neighbour vertex (not
+// transposed) times v(i - o); stencil 0 is the centre block alone. FP64
+// products and sums. With Transposed every 3 x 3 block enters transposed: the
+// mass part of the adjoint operator (the backward blocks are the forward
+// pair's, not transposed, so M^T needs the transpose of every block). The
+// values are loaded in one go and multiplied in another.
+template <class MassT, bool Transposed, int First, int Last>
+struct MassStencils {
+  static constexpr int kBlocks = 2 * (Last - First) - (First == 0 ? 1 : 0);
+  double a[kBlocks][3];
+  MassT b[kBlocks][9];
+
+  __device__ __forceinline__ void load_block(int t, const Grid& g, const double* __restrict__ v,
+                                             const MassT* __restrict__ at, unsigned node) {
+    const unsigned nodes = g.nodes();
+    const size_t vs = g.vstride;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) b[t][e] = at[size_t(e) * vs];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) a[t][c] = v[size_t(c) * nodes + node];
+  }
+
+  __device__ __forceinline__ void load(const Grid& g, const double* __restrict__ v, const MassT* __restrict__ mass,
+                                       const NodeImages& im, const VertexWalk& w) {
+    int t = 0;
+#pragma unroll
+    for (int s = First; s < Last; ++s) {
+      const int ox = c_offsets[s][0], oy = c_offsets[s][1], oz = c_offsets[s][2];
+      const MassT* rows = mass + size_t(s) * 9 * g.vstride + w.v0;
+      load_block(t++, g, v, rows, g.node(im.x[1 + ox], im.y[1 + oy], im.z[1 + oz]));
+      if (s != 0)
+        load_block(t++, g, v, rows - (ox * w.sx + oy * w.sy + oz * w.sz),
+                   g.node(im.x[1 - ox], im.y[1 - oy], im.z[1 - oz]));
+    }
+  }
+
+  __device__ __forceinline__ void add(double (&m)[3]) const {
+#pragma unroll
+    for (int t = 0; t < kBlocks; ++t)
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+        m[r] += a[t][0] * double(b[t][Transposed ? r : 3 * r]) +
+                a[t][1] * double(b[t][Transposed ? 3 + r : 3 * r + 1]) +
+                a[t][2] * double(b[t][Transposed ? 6 + r : 3 * r + 2]);
+  }
+};
+
+// Stencils First and on, one after the other.
+template <class MassT, bool Transposed, int First>
+__device__ __forceinline__ void add_stencils(const Grid& g, const double* __restrict__ v,
+                                             const MassT* __restrict__ mass, const NodeImages& im,
+                                             const VertexWalk& w, double (&m)[3]) {
+  MassStencils<MassT, Transposed, First, First + 1> one;
+  one.load(g, v, mass, im, w);
+  one.add(m);
+  if constexpr (First + 1 < kStencils) add_stencils<MassT, Transposed, First + 1>(g, v, mass, im, w, m);
+}
+
+// (1/V) f_g (M v) at node (i, j, kk).
 template <class MassT, bool Walls, bool Transposed = false>
 __device__ __forceinline__ void mass_rows(const Grid& g, const double* __restrict__ v,
                                           const MassT* __restrict__ mass, double inverse_volume, int i, int j,
-                                          int kk, unsigned n, double& mx, double& my, double& mz) {
-  // Entry (row, column) of a block sits at (3 row + column) vs, or at
-  // (3 column + row) vs transposed.
-  constexpr int e01 = Transposed ? 3 : 1, e02 = Transposed ? 6 : 2, e10 = Transposed ? 1 : 3;
-  constexpr int e12 = Transposed ? 7 : 5, e20 = Transposed ? 2 : 6, e21 = Transposed ? 5 : 7;
-  const unsigned nodes = g.nodes();
-  const unsigned ex = unsigned(g.nx + 3), exy = ex * unsigned(g.ny + 3);
-  const size_t vs = g.vstride;
-  const double* vx = v;
-  const double* vy = v + nodes;
-  const double* vz = v + 2 * size_t(nodes);
-  const unsigned v0 = g.vertex(i, j, kk);
-  // Node images of the neighbours along each axis (offsets -1, 0, +1): on a
-  // wall axis the reflection through the wall node, else the periodic image.
-  int xi[3], yi[3], zi[3];
-  if (Walls) {
-    xi[0] = node_image(g, 0, i - 1, g.nx), xi[1] = i, xi[2] = node_image(g, 0, i + 1, g.nx);
-    yi[0] = node_image(g, 1, j - 1, g.ny), yi[1] = j, yi[2] = node_image(g, 1, j + 1, g.ny);
-    zi[0] = node_image(g, 2, kk - 1, g.nz), zi[1] = kk, zi[2] = node_image(g, 2, kk + 1, g.nz);
-  }
-  {
-    const double ax = vx[n], ay = vy[n], az = vz[n];
-    const MassT* b = mass + v0;
-    mx = ax * double(b[0]) + ay * double(b[e01 * vs]) + az * double(b[e02 * vs]);
-    my = ax * double(b[e10 * vs]) + ay * double(b[4 * vs]) + az * double(b[e12 * vs]);
-    mz = ax * double(b[e20 * vs]) + ay * double(b[e21 * vs]) + az * double(b[8 * vs]);
-  }
-#pragma unroll
-  for (int s = 1; s < kStencils; ++s) {
-    const int ox = c_offsets[s][0], oy = c_offsets[s][1], oz = c_offsets[s][2];
-    // Forward: this vertex's block times v(i + o).
-    {
-      const unsigned at = Walls ? g.node(xi[1 + ox], yi[1 + oy], zi[1 + oz])
-                                : g.node(wrap_node(i + ox, g.nx), wrap_node(j + oy, g.ny), wrap_node(kk + oz, g.nz));
-      const double ax = vx[at], ay = vy[at], az = vz[at];
-      const MassT* b = mass + size_t(s) * 9 * vs + v0;
-      mx += ax * double(b[0]) + ay * double(b[e01 * vs]) + az * double(b[e02 * vs]);
-      my += ax * double(b[e10 * vs]) + ay * double(b[4 * vs]) + az * double(b[e12 * vs]);
-      mz += ax * double(b[e20 * vs]) + ay * double(b[e21 * vs]) + az * double(b[8 * vs]);
-    }
-    // Backward: the neighbour vertex's block (not transposed) times v(i - o).
-    {
-      const unsigned at = Walls ? g.node(xi[1 - ox], yi[1 - oy], zi[1 - oz])
-                                : g.node(wrap_node(i - ox, g.nx), wrap_node(j - oy, g.ny), wrap_node(kk - oz, g.nz));
-      const double ax = vx[at], ay = vy[at], az = vz[at];
-      const unsigned vb = unsigned(int(v0) - ox - oy * int(ex) - oz * int(exy));
-      const MassT* b = mass + size_t(s) * 9 * vs + vb;
-      mx += ax * double(b[0]) + ay * double(b[e01 * vs]) + az * double(b[e02 * vs]);
-      my += ax * double(b[e10 * vs]) + ay * double(b[4 * vs]) + az * double(b[e12 * vs]);
-      mz += ax * double(b[e20 * vs]) + ay * double(b[e21 * vs]) + az * double(b[8 * vs]);
-    }
-  }
+                                          int kk, double& mx, double& my, double& mz) {
+  double m[3] = {0.0, 0.0, 0.0};
+  add_stencils<MassT, Transposed, 0>(g, v, mass, node_images<Walls>(g, i, j, kk), vertex_walk(g, i, j, kk), m);
   // mass_matrix_apply_device.hpp:34-35: the row scale (1/V) f_g.
   const double row_scale = Walls ? inverse_volume * double(g.dual_factor(i, j, kk)) : inverse_volume;
-  mx *= row_scale;
-  my *= row_scale;
-  mz *= row_scale;
+  mx = m[0] * row_scale;
+  my = m[1] * row_scale;
+  mz = m[2] * row_scale;
 }
 
 // Stages of k_apply: the fused image; with smoothing, the mass response
@@ -419,9 +474,10 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
                                                     const MassT* __restrict__ mass,
                                                     const double* __restrict__ response, double d2, double k,
                                                     double inverse_volume, double* __restrict__ out,
-                                                    unsigned tile_rows, const double* __restrict__ stop) {
+                                                    unsigned tile_rows, const double* __restrict__ scale,
+                                                    Guard guard) {
   // A launch of a GMRES step after the solver stopped does nothing.
-  if (stop && *stop != 0.0) return;
+  if (guard.skips()) return;
   const unsigned nodes = g.nodes();
   const unsigned sx = unsigned(g.nx + 1), sy = unsigned(g.ny + 1), sz = unsigned(g.nz + 1);
   const unsigned L = xcd_logical_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
@@ -453,7 +509,7 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
     my = response[nodes + n];
     mz = response[2 * size_t(nodes) + n];
   } else {
-    mass_rows<MassT, Walls, Transposed>(g, v, mass, inverse_volume, i, j, kk, n, mx, my, mz);
+    mass_rows<MassT, Walls, Transposed>(g, v, mass, inverse_volume, i, j, kk, mx, my, mz);
   }
   double cx = 0, cy = 0, cz = 0;
   if (Stage != kMassResponse) c2n_at<Walls>(g, curl_cells, i, j, kk, cx, cy, cz);
@@ -472,9 +528,186 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
     if (g.constrained_row(1, i, j, kk)) oy = vy[n];
     if (g.constrained_row(2, i, j, kk)) oz = vz[n];
   }
+  if (scale) {
+    const double by = *scale;
+    ox *= by;
+    oy *= by;
+    oz *= by;
+  }
   out[n] = ox;
   out[nodes + n] = oy;
   out[2 * size_t(nodes) + n] = oz;
+}
+
+// The operator on a grid too small to fill the chip with a thread per node:
+// a block takes 64 nodes (a lane each) and its eight waves share the work of
+// every node: two stencils of M and one of the eight cells around the node,
+// whose curl is formed in place (no curl pass). Each wave loads all it needs
+// (up to 36 matrix entries and 36 vector values a lane) before it multiplies,
+// and the eight parts meet in LDS. At 16^3 a thread per node leaves 20 blocks,
+// whose lanes wait for their 27 x 12 loads in many turns: 14.6 us, and 3.6 us
+// for the curl pass before it.
+// With the image in registers the block goes on to what the solver reads it
+// for: Epilogue kDots forms the block's part of the image's products with
+// `columns` basis vectors, kResidual writes rhs - image instead of the image
+// and the block's parts of its squared norm and of rhs's.
+constexpr int kPlain = 0, kDots = 1, kResidual = 2;
+constexpr unsigned kParts = 8;
+
+// One cell's part of curl_C2N(curl_N2C v) at node (i, j, k): the cell at
+// offset (-Ax, -Ay, -Az) from the node.
+template <bool Walls, int Ax, int Ay, int Az>
+struct CurlCell {
+  Samples s[3];
+  double sign[3];
+
+  __device__ __forceinline__ void load(const Grid& g, const double* __restrict__ v, int i, int j, int k) {
+    int ci, cj, ck;
+    if constexpr (!Walls) {
+      ci = wrap_cell(i - Ax, g.nx), cj = wrap_cell(j - Ay, g.ny), ck = wrap_cell(k - Az, g.nz);
+    } else {
+      int fx, fy, fz;
+      ci = cell_image(g, 0, i - Ax, g.nx, fx), cj = cell_image(g, 1, j - Ay, g.ny, fy);
+      ck = cell_image(g, 2, k - Az, g.nz, fz);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) sign[c] = b_ghost_sign(g, c, fx, fy, fz);
+    }
+    load_cell_nodes(g, v, ci, cj, ck, s);
+  }
+
+  __device__ __forceinline__ void add(const Grid& g, double d2, double (&sum)[3]) const {
+    constexpr double dx = Ax ? -0.25 : 0.25, dy = Ay ? -0.25 : 0.25, dz = Az ? -0.25 : 0.25;
+    double b[3];
+    curl_of<true>(s, g, b[0], b[1], b[2]);
+    if constexpr (Walls)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) b[c] *= sign[c];
+    sum[0] += d2 * (dy * g.iy * b[2] - dz * g.iz * b[1]);
+    sum[1] += d2 * (dz * g.iz * b[0] - dx * g.ix * b[2]);
+    sum[2] += d2 * (dx * g.ix * b[1] - dy * g.iy * b[0]);
+  }
+};
+
+// Wave `Part`'s share of the operator at a node: stencils 2 Part and
+// 2 Part + 1 (the last two waves one each), weighted by `f`, and cell Part.
+template <class MassT, bool Walls, int Stage, bool Transposed, int Part>
+__device__ __forceinline__ void operator_share(const Grid& g, const double* __restrict__ v,
+                                               const MassT* __restrict__ mass, double f, double d2, int i, int j,
+                                               int k, double (&sum)[3]) {
+  constexpr int kFirst = Part < 6 ? 2 * Part : Part + 6, kLast = Part < 6 ? kFirst + 2 : kFirst + 1;
+  MassStencils<MassT, Transposed, kFirst, kLast> stencils;
+  CurlCell<Walls, (Part & 1), ((Part >> 1) & 1), (Part >> 2)> cell;
+  if constexpr (Stage != kCombine) stencils.load(g, v, mass, node_images<Walls>(g, i, j, k), vertex_walk(g, i, j, k));
+  if constexpr (Stage != kMassResponse) cell.load(g, v, i, j, k);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (Stage != kCombine) {
+    double m[3] = {0.0, 0.0, 0.0};
+    stencils.add(m);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) sum[c] = f * m[c];
+  }
+  if constexpr (Stage != kMassResponse) cell.add(g, d2, sum);
+}
+
+// Sum over the wave, in lane 0.
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  return v;
+}
+
+template <class MassT, bool Walls, int Stage, bool Transposed, int Epilogue>
+__global__ __launch_bounds__(64 * kParts) __attribute__((amdgpu_waves_per_eu(2, 3))) void k_apply_split(Grid g, const double* __restrict__ v,
+                                                             const MassT* __restrict__ mass,
+                                                             const double* __restrict__ response, double d2, double k,
+                                                             double inverse_volume, double* __restrict__ out,
+                                                             const double* __restrict__ scale, OperatorTail tail,
+                                                             Guard guard) {
+  if (guard.skips()) return;
+  __shared__ double s_part[kParts][3][64];
+  const unsigned lane = threadIdx.x & 63u;
+  const unsigned part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned nodes = g.nodes();
+  const unsigned L = blockIdx.x * 64u + lane;
+  const bool present = L < nodes;
+  const unsigned n = present ? L : nodes - 1;
+  const unsigned sx = unsigned(g.nx + 1), sy = unsigned(g.ny + 1);
+  const int i = int(n % sx), j = int((n / sx) % sy), kk = int(n / (sx * sy));
+  // The columns this wave multiplies, requested before the operator's loads.
+  constexpr unsigned kAhead = 2;
+  double ahead[kAhead][3];
+  if constexpr (Epilogue == kDots) {
+#pragma unroll
+    for (unsigned t = 0; t < kAhead; ++t) {
+      const unsigned col = part + t * kParts;
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        ahead[t][c] = col < tail.columns ? tail.basis[(3 * size_t(col) + c) * nodes + n] : 0.0;
+    }
+  }
+  double f = inverse_volume;
+  if (Walls) f *= double(g.dual_factor(i, j, kk));
+  if (Stage == kFused) f *= k;
+  double sum[3] = {0.0, 0.0, 0.0};
+  switch (part) {
+    case 0: operator_share<MassT, Walls, Stage, Transposed, 0>(g, v, mass, f, d2, i, j, kk, sum); break;
+    case 1: operator_share<MassT, Walls, Stage, Transposed, 1>(g, v, mass, f, d2, i, j, kk, sum); break;
+    case 2: operator_share<MassT, Walls, Stage, Transposed, 2>(g, v, mass, f, d2, i, j, kk, sum); break;
+    case 3: operator_share<MassT, Walls, Stage, Transposed, 3>(g, v, mass, f, d2, i, j, kk, sum); break;
+    case 4: operator_share<MassT, Walls, Stage, Transposed, 4>(g, v, mass, f, d2, i, j, kk, sum); break;
+    case 5: operator_share<MassT, Walls, Stage, Transposed, 5>(g, v, mass, f, d2, i, j, kk, sum); break;
+    case 6: operator_share<MassT, Walls, Stage, Transposed, 6>(g, v, mass, f, d2, i, j, kk, sum); break;
+    default: operator_share<MassT, Walls, Stage, Transposed, 7>(g, v, mass, f, d2, i, j, kk, sum); break;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) s_part[part][c][lane] = sum[c];
+  __syncthreads();
+  double image[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    image[c] = ((s_part[0][c][lane] + s_part[1][c][lane]) + (s_part[2][c][lane] + s_part[3][c][lane])) +
+               ((s_part[4][c][lane] + s_part[5][c][lane]) + (s_part[6][c][lane] + s_part[7][c][lane]));
+  if constexpr (Stage != kMassResponse) {
+    const double by = scale ? *scale : 1.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const size_t at = size_t(c) * nodes + n;
+      if (Stage == kCombine) image[c] += k * response[at];
+      image[c] += v[at];
+      // Constrained image rows take the (projected) input rows.
+      if (Walls && g.constrained_row(c, i, j, kk)) image[c] = v[at];
+      image[c] *= by;
+    }
+  }
+  if constexpr (Epilogue == kResidual) {
+    double r2 = 0.0, b2 = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double rhs = tail.rhs[size_t(c) * nodes + n];
+      image[c] = rhs - image[c];
+      r2 += image[c] * image[c];
+      b2 += rhs * rhs;
+    }
+    const double total = wave_sum(present ? (part == 0 ? r2 : b2) : 0.0);
+    if (part < 2 && lane == 0) tail.partials[size_t(part) * gridDim.x + blockIdx.x] = total;
+  }
+  if (part == 0 && present)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) out[size_t(c) * nodes + n] = image[c];
+  if constexpr (Epilogue == kDots) {
+    auto dot = [&](unsigned col, const double (&w)[3]) {
+      const double total = wave_sum(present ? w[0] * image[0] + w[1] * image[1] + w[2] * image[2] : 0.0);
+      if (lane == 0) tail.partials[size_t(col) * gridDim.x + blockIdx.x] = total;
+    };
+#pragma unroll
+    for (unsigned t = 0; t < kAhead; ++t)
+      if (part + t * kParts < tail.columns) dot(part + t * kParts, ahead[t]);
+    for (unsigned col = part + kAhead * kParts; col < tail.columns; col += kParts) {
+      double w[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) w[c] = tail.basis[(3 * size_t(col) + c) * nodes + n];
+      dot(col, w);
+    }
+  }
 }
 
 __global__ __launch_bounds__(kThreads) void k_next_e(unsigned count, const double* __restrict__ etheta,
@@ -532,7 +765,7 @@ int launch_zero_constrained(Context& ctx, double* v) {
   return check_hip(ctx, hipGetLastError(), "constrained rows");
 }
 
-int launch_smooth(Context& ctx, const double* src, double* dst, const double** result) {
+int launch_smooth(Context& ctx, const double* src, double* dst, const double** result, Guard guard) {
   const Grid& g = ctx.grid;
   const Numerics& k = ctx.num;
   if (!k.smoothing || !ctx.smooth_a || !ctx.smooth_b)
@@ -546,16 +779,16 @@ int launch_smooth(Context& ctx, const double* src, double* dst, const double** r
     double* to = last && dst ? dst : buffers[next];
     if (k.smooth_operator == TPIC_MI_SMOOTH_FACE7 && g.walls)
       k_smooth<kFace7, true><<<blocks, kThreads, 0, ctx.stream>>>(g, from, to, k.smooth_alpha, k.smooth_beta,
-                                                                 ctx.validation);
+                                                                 ctx.validation, guard);
     else if (k.smooth_operator == TPIC_MI_SMOOTH_FACE7)
       k_smooth<kFace7, false><<<blocks, kThreads, 0, ctx.stream>>>(g, from, to, k.smooth_alpha, k.smooth_beta,
-                                                                  ctx.validation);
+                                                                  ctx.validation, guard);
     else if (g.walls)
       k_smooth<kBinomial27, true><<<blocks, kThreads, 0, ctx.stream>>>(
-          g, from, to, k.smooth_alpha, k.smooth_beta, ctx.validation);
+          g, from, to, k.smooth_alpha, k.smooth_beta, ctx.validation, guard);
     else
       k_smooth<kBinomial27, false><<<blocks, kThreads, 0, ctx.stream>>>(
-          g, from, to, k.smooth_alpha, k.smooth_beta, ctx.validation);
+          g, from, to, k.smooth_alpha, k.smooth_beta, ctx.validation, guard);
     if (int rc = check_hip(ctx, hipGetLastError(), "node smoothing")) return rc;
     from = to;
     next ^= 1;
@@ -572,113 +805,149 @@ int launch_rhs(Context& ctx) {
     if (int rc = launch_smooth(ctx, ctx.current, nullptr, &current)) return rc;
   if (ctx.grid.walls)
     k_rhs<true><<<blocks_for(ctx, ctx.grid.nodes()), kThreads, 0, ctx.stream>>>(
-        ctx.grid, ctx.e, ctx.b, current, ctx.delta, ctx.current_factor, ctx.rhs, ctx.validation);
+        ctx.grid, ctx.e, ctx.b, current, ctx.delta, ctx.current_factor, ctx.rhs, ctx.etheta, ctx.validation);
   else
     k_rhs<false><<<blocks_for(ctx, ctx.grid.nodes()), kThreads, 0, ctx.stream>>>(
-        ctx.grid, ctx.e, ctx.b, current, ctx.delta, ctx.current_factor, ctx.rhs, ctx.validation);
+        ctx.grid, ctx.e, ctx.b, current, ctx.delta, ctx.current_factor, ctx.rhs, ctx.etheta, ctx.validation);
   return check_hip(ctx, hipGetLastError(), "rhs");
 }
 
 namespace {
 
-// complete_apply_smoothed (maxwell_device.hpp:389-417): x = S(v),
-// r = (1/V) f_g M x, y = S(r), image = 1*v + d2*curl_C2N(curl_cells) + k*y
-// with the constrained rows of v.
+// Grids up to this many nodes take k_apply_split, larger ones the curl pass
+// and a thread per node.
+constexpr unsigned kSplitNodes = 16384;
+
+struct OperatorArgs {
+  const Grid& g;
+  hipStream_t stream;
+  double d2, k, inverse_volume;
+  const double* scale;
+  Guard guard;
+  OperatorTail tail;
+};
+
+template <class MassT, bool Walls, int Stage, bool Transposed, int Epilogue>
+void split_kernel(const OperatorArgs& a, const double* in, const MassT* mass, const double* response, double* out) {
+  k_apply_split<MassT, Walls, Stage, Transposed, Epilogue>
+      <<<(a.g.nodes() + 63u) / 64u, 64 * kParts, 0, a.stream>>>(a.g, in, mass, response, a.d2, a.k, a.inverse_volume,
+                                                                out, a.scale, a.tail, a.guard);
+}
+
+template <class MassT, bool Walls, int Stage, bool Transposed>
+void split_stage(const OperatorArgs& a, int epilogue, const double* in, const MassT* mass, const double* response,
+                 double* out) {
+  if constexpr (Stage != kMassResponse) {  // whose image is not the operator's
+    if (epilogue == kDots) return split_kernel<MassT, Walls, Stage, Transposed, kDots>(a, in, mass, response, out);
+    if (epilogue == kResidual)
+      return split_kernel<MassT, Walls, Stage, Transposed, kResidual>(a, in, mass, response, out);
+  }
+  split_kernel<MassT, Walls, Stage, Transposed, kPlain>(a, in, mass, response, out);
+}
+
+// Rows per traversal tile: kApplyTileRows, fewer where a row is so long that a
+// tile's matrix records of one plane (16 rows at 128^3: 2.1 MB) would not
+// stay in an XCD's L2 until the next plane reads them.
 template <class MassT>
-int smoothed_apply(Context& ctx, const double* in, const MassT* mass, double* out, unsigned blocks, unsigned rows) {
-  const Grid& g = ctx.grid;
-  const double d2 = ctx.delta * ctx.delta;
-  const double* x = nullptr;
-  if (int rc = launch_smooth(ctx, in, nullptr, &x)) return rc;
-  double* r = x == ctx.smooth_a ? ctx.smooth_b : ctx.smooth_a;
-  if (g.walls)
-    k_apply<MassT, true, kMassResponse><<<blocks, kThreads, 0, ctx.stream>>>(
-        g, x, nullptr, mass, nullptr, d2, ctx.current_factor, ctx.inverse_volume, r, rows, nullptr);
+unsigned apply_tile_rows(const Grid& g) {
+  const unsigned row_bytes = unsigned(g.nx + 3) * unsigned(kEntries * sizeof(MassT));
+  const unsigned fit = std::max(1u, 2200000u / row_bytes);
+  return std::min({kApplyTileRows, fit, unsigned(g.ny + 1)});
+}
+
+template <class MassT, bool Walls, int Stage, bool Transposed = false>
+void node_stage(const OperatorArgs& a, const double* in, const double* curl, const MassT* mass,
+                const double* response, double* out) {
+  const unsigned rows = apply_tile_rows<MassT>(a.g);
+  k_apply<MassT, Walls, Stage, Transposed><<<(a.g.nodes() + kThreads - 1) / kThreads, kThreads, 0, a.stream>>>(
+      a.g, in, curl, mass, response, a.d2, a.k, a.inverse_volume, out, rows, a.scale, a.guard);
+}
+
+// image = A in by either form. Walls and smoothing take the mass response by
+// itself: smoothing between two passes of S (complete_apply_smoothed,
+// maxwell_device.hpp:389-417: x = S(v), r = (1/V) f_g M x, y = S(r),
+// image = 1*v + d2*curl_C2N(curl_cells) + k*y with the constrained rows of v);
+// with walls a thread per node would hold the kernel that does both to one
+// wave per SIMD (256 registers). The sums are those of the fused form.
+template <class MassT, bool Walls>
+int operator_image(Context& ctx, const OperatorArgs& a, bool split, int epilogue, const double* in, double* out) {
+  const MassT* mass = static_cast<const MassT*>(ctx.mass);
+  const double* const curl = ctx.gmres.curl_cells;
+  const double* response = ctx.mass_response;
+  if (ctx.num.smoothing) {
+    const double* x = nullptr;
+    if (int rc = launch_smooth(ctx, in, nullptr, &x, a.guard)) return rc;
+    double* r = x == ctx.smooth_a ? ctx.smooth_b : ctx.smooth_a;
+    OperatorArgs plain = a;
+    plain.scale = nullptr;
+    if (split)
+      split_stage<MassT, Walls, kMassResponse, false>(plain, kPlain, x, mass, nullptr, r);
+    else
+      node_stage<MassT, Walls, kMassResponse>(plain, x, nullptr, mass, nullptr, r);
+    if (int rc = check_hip(ctx, hipGetLastError(), "mass response")) return rc;
+    if (int rc = launch_smooth(ctx, r, nullptr, &response, a.guard)) return rc;
+  } else if (Walls && !split) {
+    if (!ctx.mass_response)
+      return fail(ctx, TPIC_MI_INVALID_STATE, "walled operator without its mass response buffer");
+    OperatorArgs plain = a;
+    plain.scale = nullptr;
+    node_stage<MassT, Walls, kMassResponse>(plain, in, nullptr, mass, nullptr, ctx.mass_response);
+    if (int rc = check_hip(ctx, hipGetLastError(), "walled mass response")) return rc;
+  } else {
+    if (split)
+      split_stage<MassT, Walls, kFused, false>(a, epilogue, in, mass, nullptr, out);
+    else if constexpr (!Walls)
+      node_stage<MassT, Walls, kFused>(a, in, curl, mass, nullptr, out);
+    return check_hip(ctx, hipGetLastError(), "operator apply");
+  }
+  if (split)
+    split_stage<double, Walls, kCombine, false>(a, epilogue, in, nullptr, response, out);
   else
-    k_apply<MassT, false, kMassResponse><<<blocks, kThreads, 0, ctx.stream>>>(
-        g, x, nullptr, mass, nullptr, d2, ctx.current_factor, ctx.inverse_volume, r, rows, nullptr);
-  if (int rc = check_hip(ctx, hipGetLastError(), "mass response")) return rc;
-  const double* y = nullptr;
-  if (int rc = launch_smooth(ctx, r, nullptr, &y)) return rc;
-  if (g.walls)
-    k_apply<double, true, kCombine><<<blocks, kThreads, 0, ctx.stream>>>(
-        g, in, ctx.gmres.curl_cells, nullptr, y, d2, ctx.current_factor, ctx.inverse_volume, out, rows, nullptr);
-  else
-    k_apply<double, false, kCombine><<<blocks, kThreads, 0, ctx.stream>>>(
-        g, in, ctx.gmres.curl_cells, nullptr, y, d2, ctx.current_factor, ctx.inverse_volume, out, rows, nullptr);
+    node_stage<double, Walls, kCombine>(a, in, curl, nullptr, response, out);
   return check_hip(ctx, hipGetLastError(), "operator combination");
+}
+
+// The adjoint operator of a periodic box: curl-curl is symmetric over the
+// unique nodes, the mass blocks enter transposed.
+template <class MassT>
+int transposed_image(Context& ctx, const OperatorArgs& a, bool split, int epilogue, const double* in, double* out) {
+  const MassT* mass = static_cast<const MassT*>(ctx.mass);
+  if (split)
+    split_stage<MassT, false, kFused, true>(a, epilogue, in, mass, nullptr, out);
+  else
+    node_stage<MassT, false, kFused, true>(a, in, ctx.gmres.curl_cells, mass, nullptr, out);
+  return check_hip(ctx, hipGetLastError(), "transposed operator apply");
 }
 
 }  // namespace
 
-int launch_operator(Context& ctx, const double* in, double* out, const double* stop) {
+unsigned operator_tail_blocks(const Grid& g) { return g.nodes() <= kSplitNodes ? (g.nodes() + 63u) / 64u : 0u; }
+
+int launch_operator(Context& ctx, const double* in, double* out, const OperatorCall& call) {
   const Grid& g = ctx.grid;
+  const bool split = operator_tail_blocks(g) != 0;
+  const OperatorArgs a{g, ctx.stream, ctx.delta * ctx.delta, ctx.current_factor, ctx.inverse_volume, call.scale,
+                       call.guard, call.tail};
+  const int epilogue = split ? int(call.epilogue) : kPlain;
   phase_begin(ctx, Phase::spmv);
-  // The stop word reaches the kernels of the unsmoothed operator only.
-  if (ctx.num.smoothing) stop = nullptr;
-  k_curl_n2c<<<blocks_for(ctx, g.cells()), kThreads, 0, ctx.stream>>>(g, in, ctx.gmres.curl_cells, stop);
-  int rc = check_hip(ctx, hipGetLastError(), "operator curl");
-  if (rc) return rc;
-  const unsigned blocks = (g.nodes() + kThreads - 1) / kThreads;
-  const unsigned rows = std::min(kApplyTileRows, unsigned(g.ny + 1));
-  const double d2 = ctx.delta * ctx.delta;
-  const float* mf = static_cast<const float*>(ctx.mass);
-  const double* md = static_cast<const double*>(ctx.mass);
-  if (ctx.transposed_operator) {
-    // The adjoint operator of a periodic box: curl-curl is symmetric over
-    // the unique nodes, the mass blocks enter transposed.
-    if (g.walls || ctx.num.smoothing) {
-      phase_end(ctx, Phase::spmv);
-      return fail(ctx, TPIC_MI_INVALID_STATE, "the transposed operator is built for periodic fields without smoothing");
-    }
-    if (ctx.mass_single)
-      k_apply<float, false, kFused, true><<<blocks, kThreads, 0, ctx.stream>>>(
-          g, in, ctx.gmres.curl_cells, mf, nullptr, d2, ctx.current_factor, ctx.inverse_volume, out, rows, stop);
-    else
-      k_apply<double, false, kFused, true><<<blocks, kThreads, 0, ctx.stream>>>(
-          g, in, ctx.gmres.curl_cells, md, nullptr, d2, ctx.current_factor, ctx.inverse_volume, out, rows, stop);
-    rc = check_hip(ctx, hipGetLastError(), "transposed operator apply");
-    phase_end(ctx, Phase::spmv);
-    return rc;
+  int rc = 0;
+  if (!split) {
+    k_curl_n2c<<<blocks_for(ctx, g.cells()), kThreads, 0, ctx.stream>>>(g, in, ctx.gmres.curl_cells, call.guard);
+    rc = check_hip(ctx, hipGetLastError(), "operator curl");
   }
-  if (ctx.num.smoothing) {
-    rc = ctx.mass_single ? smoothed_apply(ctx, in, mf, out, blocks, rows) : smoothed_apply(ctx, in, md, out, blocks, rows);
-    phase_end(ctx, Phase::spmv);
-    return rc;
+  if (rc) {
+  } else if (ctx.transposed_operator && (g.walls || ctx.num.smoothing)) {
+    rc = fail(ctx, TPIC_MI_INVALID_STATE, "the transposed operator is built for periodic fields without smoothing");
+  } else if (ctx.transposed_operator) {
+    rc = ctx.mass_single ? transposed_image<float>(ctx, a, split, epilogue, in, out)
+                         : transposed_image<double>(ctx, a, split, epilogue, in, out);
+  } else if (g.walls) {
+    rc = ctx.mass_single ? operator_image<float, true>(ctx, a, split, epilogue, in, out)
+                         : operator_image<double, true>(ctx, a, split, epilogue, in, out);
+  } else {
+    rc = ctx.mass_single ? operator_image<float, false>(ctx, a, split, epilogue, in, out)
+                         : operator_image<double, false>(ctx, a, split, epilogue, in, out);
   }
-  if (g.walls) {
-    // Two stages, the mass response (1/V) f_g M v into a node buffer, then
-    // the image with the curl term: fused, the wall images and ghost signs of
-    // both terms held the kernel to one wave per SIMD (256 registers). The
-    // sums are those of the fused form.
-    double* r = ctx.mass_response;
-    if (!r) {
-      phase_end(ctx, Phase::spmv);
-      return fail(ctx, TPIC_MI_INVALID_STATE, "walled operator without its mass response buffer");
-    }
-    if (ctx.mass_single)
-      k_apply<float, true, kMassResponse><<<blocks, kThreads, 0, ctx.stream>>>(
-          g, in, nullptr, mf, nullptr, d2, ctx.current_factor, ctx.inverse_volume, r, rows, stop);
-    else
-      k_apply<double, true, kMassResponse><<<blocks, kThreads, 0, ctx.stream>>>(
-          g, in, nullptr, md, nullptr, d2, ctx.current_factor, ctx.inverse_volume, r, rows, stop);
-    if ((rc = check_hip(ctx, hipGetLastError(), "walled mass response"))) {
-      phase_end(ctx, Phase::spmv);
-      return rc;
-    }
-    k_apply<double, true, kCombine><<<blocks, kThreads, 0, ctx.stream>>>(
-        g, in, ctx.gmres.curl_cells, nullptr, r, d2, ctx.current_factor, ctx.inverse_volume, out, rows, stop);
-    rc = check_hip(ctx, hipGetLastError(), "walled operator combination");
-    phase_end(ctx, Phase::spmv);
-    return rc;
-  }
-  if (ctx.mass_single)
-    k_apply<float, false><<<blocks, kThreads, 0, ctx.stream>>>(g, in, ctx.gmres.curl_cells, mf, nullptr, d2,
-                                                               ctx.current_factor, ctx.inverse_volume, out, rows, stop);
-  else
-    k_apply<double, false><<<blocks, kThreads, 0, ctx.stream>>>(g, in, ctx.gmres.curl_cells, md, nullptr, d2,
-                                                                ctx.current_factor, ctx.inverse_volume, out, rows, stop);
-  rc = check_hip(ctx, hipGetLastError(), "operator apply");
   phase_end(ctx, Phase::spmv);
   return rc;
 }
@@ -691,7 +960,7 @@ int launch_curl_c2n(Context& ctx, const double* cells_in, double* nodes_out) {
 
 int launch_curl_n2c(Context& ctx, const double* nodes_in, double* cells_out) {
   k_curl_n2c<<<blocks_for(ctx, ctx.grid.cells()), kThreads, 0, ctx.stream>>>(ctx.grid, nodes_in, cells_out,
-                                                                              nullptr);
+                                                                              Guard{});
   return check_hip(ctx, hipGetLastError(), "cell curl");
 }
 
