@@ -731,8 +731,7 @@ def test_cycle_incremental_plan_equals_the_run_based_plan(case):
     matrix, the bins and every particle attribute are equal bit for bit:
     for a two-species uniform plasma (the crosser plan throughout), for a
     slab whose column-2 particles all cross into column 3 in the first step
-    (about 400 arrivals per bin: the crosser plan hands the species to the
-    run-based plan), and after a sort failed on an invalid key (the crosser plan finds
+    (about 400 arrivals per bin), and after a sort failed on an invalid key (the crosser plan finds
     the old bins inconsistent and hands over as well)."""
     rng = np.random.default_rng(43)
     if case == "converging":
@@ -779,6 +778,46 @@ def test_cycle_incremental_plan_equals_the_run_based_plan(case):
             assert sims[0].validation() & R.INVALID_SORT
         if case == "uniform":
             assert sims[0].validation() == 0
+    finally:
+        for sim in sims:
+            sim.close()
+
+
+@pytest.mark.parametrize("arrivals", [2, 12, 13, 64, 65, 130, 1100])
+def test_cycle_plan_at_every_arrival_count(arrivals):
+    """Bins that receive few to many particles in one step (a thread's list, a
+    wave's, several rounds of one, and more than the crosser plan orders) in
+    the first and the last of three species (planned as a pair and alone),
+    one of them without particles in turn: as the run-based plan, bit for
+    bit."""
+    rng = np.random.default_rng(47 + arrivals)
+    cells = lengths = (8, 4, 3)
+    empty = {k: v[:0] for k, v in converging_slab(cells, 1, 10.0, rng).items()}
+    arrays = [converging_slab(cells, arrivals, 10.0, rng),
+              empty if arrivals % 2 else cases.uniform_maxwellian(cells, lengths, (2, 2, 2), 1.0, thermal=(0.3,) * 3,
+                                                                  seed=5),
+              converging_slab(cells, max(1, arrivals // 3), 10.0, rng)]
+    spec = [(q, len(a["cell"])) for q, a in zip((-1.0, 1.0, -2.0), arrays)]
+    b = cases.uniform_b(cells, (0.01, 0.02, 0.05), amplitude=0.2)
+    say("arrivals", arrivals, "particles", [n for _, n in spec])
+    sims = [gpu(cells, lengths, spec, dt=0.1, gmres_tolerance=1e-12) for _ in range(2)]
+    try:
+        sims[1].record_permutation(True)
+        for sim in sims:
+            for s, a in enumerate(arrays):
+                sim.set_particles(s, a)
+            sim.set_field(R.FIELD_B, b)
+            sim.initialize()
+        for _ in range(3):
+            for sim in sims:
+                sim.cycle(1)
+            for s in range(3):
+                g0, g1 = sims[0].get_particles(s), sims[1].get_particles(s)
+                for k in R.ATTRIBUTES:
+                    assert np.array_equal(g0[k], g1[k]), (s, k)
+                for x, y in zip(sims[0].get_bins(s), sims[1].get_bins(s)):
+                    assert np.array_equal(x, y), s
+        assert sims[0].validation() == sims[1].validation()
     finally:
         for sim in sims:
             sim.close()

@@ -93,6 +93,9 @@ void release(T*& p) {
   p = nullptr;
 }
 
+// Particles from which a cycle plans species 0's sort beside the other moves.
+constexpr uint64_t kForkParticles = 40000000;
+
 size_t scan_scratch_words(size_t n) {
   size_t words = 0;
   while (n > 2048) {
@@ -131,6 +134,8 @@ void free_all(tpic_mi_context* h) {
     release(w.block_base); release(w.bin_base); release(w.bin_lower);
   }
   release(c.plan_status);
+  if (c.planned) (void)hipEventDestroy(c.planned);
+  c.planned = nullptr;
   if (c.fork) (void)hipEventDestroy(c.fork);
   if (c.join) (void)hipEventDestroy(c.join);
   if (c.side_stream) (void)hipStreamDestroy(c.side_stream);
@@ -242,9 +247,11 @@ int allocate(tpic_mi_context* h) {
     TPIC_ALLOC(w.block_base, blocks + 1);
     TPIC_ALLOC(w.bin_base, bins);
     TPIC_ALLOC(w.bin_lower, bins);
-    w.scan_scratch_words = scan_scratch_words(std::max({bins, size_t(w.tiles) + 1, blocks + 1}));
+    w.scan_scratch_words = std::max(scan_scratch_words(std::max({bins, size_t(w.tiles) + 1, blocks + 1})),
+                                    cross_plan_words(blocks, bins));
     TPIC_ALLOC(w.scan_scratch, w.scan_scratch_words);
   }
+  if ((rc = check_hip(c, hipEventCreateWithFlags(&c.planned, hipEventDisableTiming), "plan event"))) return rc;
   if (side) {
     // Default priority, like the context stream.
     if ((rc = check_hip(c, hipStreamCreateWithFlags(&c.side_stream, hipStreamNonBlocking), "side stream")) ||
@@ -786,42 +793,58 @@ int tpic_mi_cycle(tpic_mi_context* h, int cycles, tpic_mi_solve_result* last) {
     if (rc) return rc;
     // Move, advance, sort (the reference's order); the sort's record copy is
     // fused into the deposition, whose sums are those of the separate calls.
-    // With two or more species (and no permutation record), species 0's sort
-    // plan runs on the side stream while the other species move: the plan
-    // from the crossers is light in HBM traffic, the mover bound by it.
     // A species sorted before its move gets the incremental plan (from the
     // crossers the block mover records); a species whose incremental plan
     // reports a bin it cannot order, or an inconsistent previous plan, then
     // gets the run-based plan (one host read of the plan words per cycle).
     uint32_t* saved = c.sort.permutation;
     if (!h->record_permutation) c.sort.permutation = nullptr;
-    const bool fork = c.side_stream && !h->record_permutation;
+    const bool side = c.side_stream && !h->record_permutation;
     bool incremental[kMaxSpecies] = {};
     bool any_incremental = false;
+    uint64_t particles = 0;
     for (int s = 0; s < ns; ++s) {
       incremental[s] = !h->record_permutation && c.species[size_t(s)].sorted && c.species[size_t(s)].count > 0;
       any_incremental = any_incremental || incremental[s];
+      particles += c.species[size_t(s)].count;
     }
+    // Large runs move species 0 first and plan its sort on the side stream
+    // while the others move: the plan from the crossers is light in HBM
+    // traffic, the mover bound by it. Below kForkParticles a cycle waits for
+    // launches more than for memory, so every species moves in one launch and
+    // the first two plans share theirs.
+    const bool fork = side && particles >= kForkParticles;
+    const bool paired = side && !fork && incremental[0] && incremental[1];
     auto plan = [&](int s, SortWorkspace& ws, hipStream_t st) {
-      return incremental[s] ? launch_sort_plan_incremental(c, s, ws, st) : launch_sort_plan(c, s, ws, st);
+      SortWorkspace* const one[] = {&ws};
+      return incremental[s] ? launch_sort_plan_incremental(c, s, 1, one, st) : launch_sort_plan(c, s, ws, st);
     };
-    for (int s = 0; s < ns && !rc; ++s) {
-      rc = launch_move(c, s, incremental[s]);
-      if (!rc && s == 0 && fork) {
-        if (!(rc = check_hip(c, hipEventRecord(c.fork, c.stream), "fork")) &&
-            !(rc = check_hip(c, hipStreamWaitEvent(c.side_stream, c.fork, 0), "fork")) &&
-            !(rc = plan(0, c.sort_side, c.side_stream)))
-          rc = check_hip(c, hipEventRecord(c.join, c.side_stream), "join");
-      }
+    if (fork) {
+      rc = launch_moves(c, 0, 1, incremental);
+      if (!rc && !(rc = check_hip(c, hipEventRecord(c.fork, c.stream), "fork")) &&
+          !(rc = check_hip(c, hipStreamWaitEvent(c.side_stream, c.fork, 0), "fork")) &&
+          !(rc = plan(0, c.sort_side, c.side_stream)))
+        rc = check_hip(c, hipEventRecord(c.join, c.side_stream), "join");
+      if (!rc) rc = launch_moves(c, 1, ns, incremental + 1);
+    } else {
+      rc = launch_moves(c, 0, ns, incremental);
     }
-    if (!rc) rc = launch_next_fields(c);
-    for (int s = fork ? 1 : 0; s < ns && !rc; ++s) rc = plan(s, c.sort, c.stream);
+    if (!rc && paired) {
+      SortWorkspace* const both[] = {&c.sort_side, &c.sort};
+      rc = launch_sort_plan_incremental(c, 0, 2, both, c.stream);
+    }
+    for (int s = fork ? 1 : (paired ? 2 : 0); s < ns && !rc; ++s) rc = plan(s, c.sort, c.stream);
     if (!rc && fork) rc = check_hip(c, hipStreamWaitEvent(c.stream, c.join, 0), "join");
+    // The plan words travel to the host while the fields advance (the plans
+    // and the fields do not meet before the deposition).
+    if (!rc && any_incremental &&
+        !(rc = check_hip(c, hipMemcpyAsync(c.host_status, c.plan_status, size_t(ns) * sizeof(uint32_t),
+                                           hipMemcpyDeviceToHost, c.stream),
+                         "plan status")))
+      rc = check_hip(c, hipEventRecord(c.planned, c.stream), "plan status");
+    if (!rc) rc = launch_next_fields(c);
     if (!rc && any_incremental) {
-      rc = check_hip(c, hipMemcpyAsync(c.host_status, c.plan_status, size_t(ns) * sizeof(uint32_t),
-                                       hipMemcpyDeviceToHost, c.stream),
-                     "plan status");
-      if (!rc) rc = check_hip(c, hipStreamSynchronize(c.stream), "plan status");
+      rc = check_hip(c, hipEventSynchronize(c.planned), "plan status");
       for (int s = 0; s < ns && !rc; ++s)
         if (incremental[s] && c.host_status[s] != 0) rc = launch_sort_plan(c, s);
     }

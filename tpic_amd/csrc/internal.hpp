@@ -134,6 +134,7 @@ struct Context {
   SortWorkspace sort_side;
   hipStream_t side_stream = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
+  hipEvent_t planned = nullptr;  // the cycle's plan words are on the host
   GmresWorkspace gmres;
   // Timing (hipEvents around phases when enabled)
   bool timing = false;
@@ -183,10 +184,15 @@ int launch_sort_plan(Context& ctx, int species, SortWorkspace& ws, hipStream_t s
 // sources as the run-based plan). It sets ctx.plan_status[species] nonzero
 // when the run-based plan must be run instead (a bin with many arrivals, or
 // a previous plan that failed).
-int launch_sort_plan_incremental(Context& ctx, int species, SortWorkspace& ws, hipStream_t stream);
+// One or two species from `first` on in the same launches, each with a
+// workspace of its own and at least one particle.
+int launch_sort_plan_incremental(Context& ctx, int first, int species, SortWorkspace* const* ws, hipStream_t stream);
+size_t cross_plan_words(size_t blocks, size_t bins);
 // With record_crossers (a sorted species) the block mover also writes the
 // species' crosser masks for launch_sort_plan_incremental.
 int launch_move(Context& ctx, int species, bool record_crossers = false);
+// Species [first, last) in as few launches as their particles per cell allow.
+int launch_moves(Context& ctx, int first, int last, const bool* record_crossers);
 int launch_deposit(Context& ctx, int first_species, int last_species, bool accumulate);
 // Every species' planned sort fused with the deposition: each destination
 // record is gathered from its source, stored in the scratch slot and

@@ -411,14 +411,31 @@ __device__ __forceinline__ bool key_in_range(int32_t key, uint32_t bins) { retur
 // block b+2, and the records, key ranges and staged corner fields of
 // block b+1, are in flight while block b is pushed; block b+1's corners are
 // staged in the second LDS buffer once b is done.
+struct MoveSpecies {
+  MoverParams p;
+  ParticleView s;
+  uint32_t n;
+  const uint32_t* counts;
+  const uint32_t* offsets;
+  uint64_t* cross;  // or null
+};
+
+// The species of a launch, blockIdx.y.
+struct MoveBatch {
+  MoveSpecies species[kMaxSpecies];
+};
+
 template <unsigned Slots>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(Slots > 4 ? 3 : 4))) void k_move_blocks(Grid g, MoverParams p, ParticleView s, uint32_t n,
-                                                          const uint32_t* __restrict__ counts,
-                                                          const uint32_t* __restrict__ offsets,
-                                                          const double* __restrict__ etheta,
-                                                          const double* __restrict__ bnode,
-                                                          unsigned* __restrict__ validation,
-                                                          uint64_t* __restrict__ cross) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(Slots > 4 ? 3 : 4))) void k_move_blocks(
+    Grid g, MoveBatch batch, const double* __restrict__ etheta, const double* __restrict__ bnode,
+    unsigned* __restrict__ validation) {
+  const MoveSpecies& sp = batch.species[blockIdx.y];
+  const MoverParams& p = sp.p;
+  const ParticleView s = sp.s;
+  const uint32_t n = sp.n;
+  const uint32_t* __restrict__ counts = sp.counts;
+  const uint32_t* __restrict__ offsets = sp.offsets;
+  uint64_t* __restrict__ cross = sp.cross;
   __shared__ __align__(16) double s_corner[kWaves][2][Slots * kSlotStride];
   const unsigned lane = threadIdx.x & 63u;
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -591,45 +608,61 @@ unsigned block_walk_blocks(const Context& ctx, uint32_t n) {
   return unsigned(std::max<uint64_t>(1, want < cap ? want : cap));
 }
 
-// The sorted mover with room for Slots bins a block.
-template <unsigned Slots>
-void launch_blocks(const Context& ctx, const SpeciesState& sp, const MoverParams& p, uint64_t* cross) {
-  k_move_blocks<Slots><<<block_walk_blocks(ctx, sp.count), kThreads, 0, ctx.stream>>>(
-      ctx.grid, p, sp.view(), sp.count, sp.counts, sp.offsets, ctx.particle_field(), ctx.bn, ctx.validation, cross);
+// Slots by the mean count c of a cell: 64 particles span 64 / c + 1 bins and
+// more where counts vary. From 48 on two bins hold nearly every block (four
+// instead of two: 1.3% of the cycle slower at 64 per cell and 128^3, 3.8% at
+// 100 per cell and 512^2); four bins hold three or four bins' blocks down to
+// 20 (cycle at 61 x 47 x 33 with 27 per cell: 1.61 ms with two, 1.34 ms with
+// four), ten those of 8 a cell.
+unsigned slots_for(const Context& ctx, const SpeciesState& sp) {
+  const uint64_t cells = ctx.grid.cells();
+  return sp.count >= 48 * cells ? 2u : (sp.count >= 20 * cells ? 4u : 10u);
 }
 
 }  // namespace
 
-int launch_move(Context& ctx, int s, bool record_crossers) {
-  SpeciesState& sp = ctx.species[size_t(s)];
-  if (sp.count == 0) return 0;
-  const MoverParams p = mover_params(ctx, sp);
+int launch_move(Context& ctx, int s, bool record_crossers) { return launch_moves(ctx, s, s + 1, &record_crossers); }
+
+int launch_moves(Context& ctx, int first, int last, const bool* record_crossers) {
+  bool any = false;
+  for (int s = first; s < last; ++s) any = any || ctx.species[size_t(s)].count != 0;
+  if (!any) return 0;
   phase_begin(ctx, Phase::move);
-  if (sp.sorted) {
-    uint64_t* const cross = record_crossers ? sp.cross : nullptr;
-    const uint64_t cells = ctx.grid.cells();
-    // Slots by the mean count c of a cell: 64 particles span 64 / c + 1 bins
-    // and more where counts vary. From 48 on two bins hold nearly every block
-    // (four instead of two: 1.3% of the cycle slower at 64 per cell and 128^3,
-    // 3.8% at 100 per cell and 512^2); four bins hold three or four bins'
-    // blocks down to 20 (cycle at 61 x 47 x 33 with 27 per cell: 1.61 ms with
-    // two, 1.34 ms with four), ten those of 8 a cell.
-    if (sp.count >= 48 * cells)
-      launch_blocks<2>(ctx, sp, p, cross);
-    else if (sp.count >= 20 * cells)
-      launch_blocks<4>(ctx, sp, p, cross);
-    else
-      launch_blocks<10>(ctx, sp, p, cross);
-  } else {
+  const double* e = ctx.particle_field();
+  for (int s = first; s < last; ++s) {
+    const SpeciesState& sp = ctx.species[size_t(s)];
+    if (sp.count == 0 || sp.sorted) continue;
     const unsigned blocks = unsigned(std::min<uint64_t>((uint64_t(sp.count) + kThreads - 1) / kThreads,
                                                         uint64_t(ctx.cus > 0 ? ctx.cus : 256) * 32));
-    k_move<<<blocks, kThreads, 0, ctx.stream>>>(ctx.grid, p, sp.view(), sp.count, ctx.particle_field(), ctx.bn,
+    k_move<<<blocks, kThreads, 0, ctx.stream>>>(ctx.grid, mover_params(ctx, sp), sp.view(), sp.count, e, ctx.bn,
                                                 ctx.validation);
+    if (int rc = check_hip(ctx, hipGetLastError(), "mover")) return rc;
   }
-  const int rc = check_hip(ctx, hipGetLastError(), "mover");
+  // The sorted species, one launch per number of slots.
+  for (unsigned slots : {2u, 4u, 10u}) {
+    MoveBatch batch{};
+    unsigned species = 0, blocks = 0;
+    for (int s = first; s < last; ++s) {
+      const SpeciesState& sp = ctx.species[size_t(s)];
+      if (sp.count == 0 || !sp.sorted || slots_for(ctx, sp) != slots) continue;
+      batch.species[species++] = MoveSpecies{mover_params(ctx, sp), sp.view(), sp.count, sp.counts, sp.offsets,
+                                             record_crossers[s - first] ? sp.cross : nullptr};
+      blocks = std::max(blocks, block_walk_blocks(ctx, sp.count));
+    }
+    if (species == 0) continue;
+    const dim3 grid(blocks, species);
+    if (slots == 2)
+      k_move_blocks<2><<<grid, kThreads, 0, ctx.stream>>>(ctx.grid, batch, e, ctx.bn, ctx.validation);
+    else if (slots == 4)
+      k_move_blocks<4><<<grid, kThreads, 0, ctx.stream>>>(ctx.grid, batch, e, ctx.bn, ctx.validation);
+    else
+      k_move_blocks<10><<<grid, kThreads, 0, ctx.stream>>>(ctx.grid, batch, e, ctx.bn, ctx.validation);
+    if (int rc = check_hip(ctx, hipGetLastError(), "mover")) return rc;
+  }
   phase_end(ctx, Phase::move);
-  sp.sorted = false;
-  return rc;
+  for (int s = first; s < last; ++s)
+    if (ctx.species[size_t(s)].count != 0) ctx.species[size_t(s)].sorted = false;
+  return 0;
 }
 
 }  // namespace tpic_mi

@@ -506,12 +506,72 @@ __global__ __launch_bounds__(kThreads) void k_scan_apply(const uint32_t* __restr
 // earlier positions (lower bins), in position order; its stayers, in position
 // order; its arrivals from later positions. Every stayer's destination is its
 // bin's base plus its position less the crossers before it; each bin orders
-// its few arrivals by position. A bin with more than kArrivalsMax arrivals,
-// or an old state in which the stayers and crossers do not add up to the
-// particles (a previous plan that failed), sets the species' plan status: the
-// run-based plan is then run instead.
-constexpr uint32_t kArrivalsMax = 64;
-constexpr uint32_t kArrivalsInRegisters = 16;
+// its arrivals by position. A bin with more than kArrivalsMax arrivals, or an
+// old state in which the stayers and crossers do not add up to the particles
+// (a previous plan that failed), sets the species' plan status: the run-based
+// plan is then run instead.
+//
+// Seven launches for one or two species (blockIdx.y), each with what it needs
+// cleared, counted or scanned folded in: a scan over tiles is two passes, the
+// second of which adds the tiles before its own by itself. As clears, counts
+// and three-launch scans of their own they were nineteen a species, 130 us of
+// launches a cycle at 16^3.
+constexpr uint32_t kArrivalsMax = 1024;
+constexpr uint32_t kArrivalsInRegisters = 12;
+
+struct CrossPlan {
+  const int32_t* keys;
+  const uint64_t* cross;
+  uint32_t n, blocks;       // particles, 64-particle blocks
+  uint32_t* block_base;     // [blocks + 1] crossers before each block
+  uint32_t* arrivals;       // [bins]
+  uint32_t* arrival_offset; // [bins + 1]
+  uint32_t* lower;          // [bins] arrivals from lower bins
+  uint32_t* slot;           // per crosser: its index among its bin's arrivals
+  uint32_t* shift;          // [bins] crossers before the old range less its start
+  uint32_t* bin_base;       // [bins] stayer destination base
+  uint32_t* bin_arrivals;   // positions of the arrivals, by bin
+  uint32_t* tile_a;         // tile sums: crossers, then counts
+  uint32_t* tile_b;         // tile sums: arrivals
+  uint32_t* counts;
+  uint32_t* offsets;
+  uint32_t* source;
+  uint32_t* status;
+  ParticleView src, dst;
+};
+
+struct CrossPlans {
+  CrossPlan species[2];
+};
+
+// Bins and 64-particle blocks per tile of the plan's scans: two a thread, so a
+// small grid's few thousand still spread over the chip (eight a thread: 15 us
+// instead of 5 for the new counts at 16^3).
+constexpr unsigned kPlanItems = 2;
+constexpr unsigned kPlanTile = kThreads * kPlanItems;
+
+// Sum of tiles[0 .. last), in every thread.
+__device__ inline uint32_t tiles_before(const uint32_t* __restrict__ tiles, uint32_t last, uint32_t* lds) {
+  uint32_t v = 0;
+  for (uint32_t t = threadIdx.x; t < last; t += kThreads) v += tiles[t];
+  return block_sum(v, lds);
+}
+
+// Exclusive prefix of a value per thread over the block.
+__device__ inline uint32_t block_exclusive(uint32_t v, uint32_t* lds) {
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint32_t inc = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t t = __shfl_up(inc, off, 64);
+    if (int(lane) >= off) inc += t;
+  }
+  if (lane == 63) lds[wave] = inc;
+  __syncthreads();
+  uint32_t before = 0;
+  for (unsigned w = 0; w < kThreads / 64; ++w) before += w < wave ? lds[w] : 0u;
+  __syncthreads();
+  return before + inc - v;
+}
 
 __device__ __forceinline__ uint32_t crossers_before(const uint64_t* __restrict__ cross,
                                                     const uint32_t* __restrict__ block_base, uint32_t blocks,
@@ -522,10 +582,46 @@ __device__ __forceinline__ uint32_t crossers_before(const uint64_t* __restrict__
   return block_base[blk] + below;
 }
 
-__global__ __launch_bounds__(kThreads) void k_cross_counts(const uint64_t* __restrict__ cross, uint32_t blocks,
-                                                           uint32_t* __restrict__ out) {
-  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < blocks; b += gridDim.x * blockDim.x)
-    out[b] = uint32_t(__popcll(cross[b]));
+// Crossers per tile of kPlanTile blocks, the bins' arrival counts cleared.
+__global__ __launch_bounds__(kThreads) void k_cross_begin(CrossPlans plans, uint32_t bins) {
+  const CrossPlan& s = plans.species[blockIdx.y];
+  __shared__ uint32_t lds[kThreads / 64];
+  const uint32_t base = blockIdx.x * kPlanTile + threadIdx.x;
+  if (base == 0) *s.status = 0;
+  uint32_t sum = 0;
+#pragma unroll
+  for (unsigned r = 0; r < kPlanItems; ++r) {
+    const uint32_t i = base + r * kThreads;
+    if (i < s.blocks) sum += uint32_t(__popcll(s.cross[i]));
+    if (i < bins) {
+      s.arrivals[i] = 0;
+      s.lower[i] = 0;
+    }
+  }
+  const uint32_t total = block_sum(sum, lds);
+  if (threadIdx.x == 0 && blockIdx.x * kPlanTile < s.blocks) s.tile_a[blockIdx.x] = total;
+}
+
+// Crossers before each block.
+__global__ __launch_bounds__(kThreads) void k_cross_bases(CrossPlans plans) {
+  const CrossPlan& s = plans.species[blockIdx.y];
+  if (blockIdx.x * kPlanTile >= s.blocks) return;
+  __shared__ uint32_t lds[kThreads / 64];
+  const uint32_t first = blockIdx.x * kPlanTile + threadIdx.x * kPlanItems;
+  uint32_t v[kPlanItems], sum = 0;
+#pragma unroll
+  for (unsigned r = 0; r < kPlanItems; ++r) {
+    v[r] = first + r < s.blocks ? uint32_t(__popcll(s.cross[first + r])) : 0u;
+    sum += v[r];
+  }
+  uint32_t running = tiles_before(s.tile_a, blockIdx.x, lds);
+  running += block_exclusive(sum, lds);
+#pragma unroll
+  for (unsigned r = 0; r < kPlanItems; ++r) {
+    if (first + r < s.blocks) s.block_base[first + r] = running;
+    running += v[r];
+    if (first + r + 1 == s.blocks) s.block_base[s.blocks] = running;
+  }
 }
 
 // Per crosser one arrival in its new bin (integer atomics: crosser t of the
@@ -534,21 +630,15 @@ __global__ __launch_bounds__(kThreads) void k_cross_counts(const uint64_t* __res
 // from a lower bin when its position precedes the bin's old range. Tiles of
 // kTile particles: the crosser words of a wave span and every crosser's key
 // are loaded first, then the atomics and range starts, then the stores.
-__global__ __launch_bounds__(kThreads) void k_cross_arrivals(const uint64_t* __restrict__ cross, uint32_t n,
-                                                             const uint32_t* __restrict__ block_base,
-                                                             const int32_t* __restrict__ keys, uint32_t bins,
-                                                             const uint32_t* __restrict__ old_offsets,
-                                                             uint32_t* __restrict__ arrivals,
-                                                             uint32_t* __restrict__ lower,
-                                                             uint32_t* __restrict__ slot,
-                                                             uint32_t* __restrict__ status) {
+__global__ __launch_bounds__(kThreads) void k_cross_arrivals(CrossPlans plans, uint32_t bins) {
+  const CrossPlan& s = plans.species[blockIdx.y];
   const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t sub = blockIdx.x * kTile + wave * kWaveSpan;
-  if (sub >= n) return;
+  if (sub >= s.n) return;
   const uint32_t blk0 = sub >> 6;  // sub is a multiple of 64
-  const bool item_lane = lane < kWaveItems && sub + lane * 64u < n;
-  const uint64_t words = item_lane ? cross[blk0 + lane] : 0ull;
-  const uint32_t bases = item_lane ? block_base[blk0 + lane] : 0u;
+  const bool item_lane = lane < kWaveItems && sub + lane * 64u < s.n;
+  const uint64_t words = item_lane ? s.cross[blk0 + lane] : 0ull;
+  const uint32_t bases = item_lane ? s.block_base[blk0 + lane] : 0u;
   uint32_t crossers = 0;  // bit r: the lane's particle of item r is a crosser
   uint32_t list[kWaveItems];  // its index in the crosser list
   int32_t key[kWaveItems];
@@ -559,7 +649,7 @@ __global__ __launch_bounds__(kThreads) void k_cross_arrivals(const uint64_t* __r
     const bool crosser = ((lane < 32u ? lo : hi) >> (lane & 31u)) & 1u;
     crossers |= uint32_t(crosser) << r;
     list[r] = uint32_t(__builtin_amdgcn_readlane(int(bases), int(r))) + bits_below(lo, hi);
-    key[r] = crosser ? keys[sub + r * 64 + lane] : -1;
+    key[r] = crosser ? s.keys[sub + r * 64 + lane] : -1;
   }
   if (crossers == 0) return;
   wait_loads();
@@ -568,8 +658,8 @@ __global__ __launch_bounds__(kThreads) void k_cross_arrivals(const uint64_t* __r
   for (unsigned r = 0; r < kWaveItems; ++r) {
     const int32_t k = key[r];
     const bool ok = ((crossers >> r) & 1u) && k >= 0 && uint32_t(k) < bins;
-    j[r] = ok ? atomicAdd(arrivals + k, 1u) : 0u;
-    start[r] = ok ? old_offsets[k] : 0u;
+    j[r] = ok ? atomicAdd(s.arrivals + k, 1u) : 0u;
+    start[r] = ok ? s.offsets[k] : 0u;
   }
   wait_loads();
 #pragma unroll
@@ -577,89 +667,116 @@ __global__ __launch_bounds__(kThreads) void k_cross_arrivals(const uint64_t* __r
     if (!((crossers >> r) & 1u)) continue;
     const int32_t k = key[r];
     if (k < 0 || uint32_t(k) >= bins) {
-      atomicOr(status, 4u);
+      atomicOr(s.status, 4u);
       continue;
     }
-    slot[list[r]] = j[r];
-    if (sub + r * 64 + lane < start[r]) atomicAdd(lower + k, 1u);
+    s.slot[list[r]] = j[r];
+    if (sub + r * 64 + lane < start[r]) atomicAdd(s.lower + k, 1u);
   }
 }
 
 // Per bin: new count (old count less the bin's crossers plus its arrivals)
 // and `shift`, the crossers before the old range less the range's start (the
-// stayer base less the new offset and the arrivals from lower bins). Reads
-// the previous plan's offsets, before the scan of the new counts replaces
-// them.
-__global__ __launch_bounds__(kThreads) void k_cross_counts_new(uint32_t bins, const uint32_t* __restrict__ old_offsets,
-                                                               const uint64_t* __restrict__ cross,
-                                                               const uint32_t* __restrict__ block_base,
-                                                               uint32_t blocks,
-                                                               const uint32_t* __restrict__ arrivals,
-                                                               uint32_t* __restrict__ counts,
-                                                               uint32_t* __restrict__ shift,
-                                                               uint32_t* __restrict__ status) {
-  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < bins; b += gridDim.x * blockDim.x) {
-    const uint32_t o = old_offsets[b], e = old_offsets[b + 1];
-    const uint32_t lo = crossers_before(cross, block_base, blocks, o);
-    const uint32_t hi = crossers_before(cross, block_base, blocks, e);
-    const uint32_t arrive = arrivals[b];
-    if (arrive > kArrivalsMax) atomicOr(status, 1u);
-    counts[b] = (e - o) - (hi - lo) + arrive;
-    shift[b] = lo - o;
+// stayer base less the new offset and the arrivals from lower bins), and the
+// tiles' sums of counts and arrivals. Reads the previous plan's offsets,
+// before the scan of the new counts replaces them.
+__global__ __launch_bounds__(kThreads) void k_cross_counts_new(CrossPlans plans, uint32_t bins) {
+  const CrossPlan& s = plans.species[blockIdx.y];
+  __shared__ uint32_t lds[kThreads / 64];
+  uint32_t count_sum = 0, arrival_sum = 0;
+  bool many = false;
+#pragma unroll
+  for (unsigned r = 0; r < kPlanItems; ++r) {
+    const uint32_t b = blockIdx.x * kPlanTile + r * kThreads + threadIdx.x;
+    if (b >= bins) continue;
+    const uint32_t o = s.offsets[b], e = s.offsets[b + 1];
+    const uint32_t lo = crossers_before(s.cross, s.block_base, s.blocks, o);
+    const uint32_t hi = crossers_before(s.cross, s.block_base, s.blocks, e);
+    const uint32_t arrive = s.arrivals[b], count = (e - o) - (hi - lo) + arrive;
+    many |= arrive > kArrivalsMax;
+    s.counts[b] = count;
+    s.shift[b] = lo - o;
+    count_sum += count;
+    arrival_sum += arrive;
+  }
+  if (many) atomicOr(s.status, 1u);
+  count_sum = block_sum(count_sum, lds);
+  arrival_sum = block_sum(arrival_sum, lds);
+  if (threadIdx.x == 0) {
+    s.tile_a[blockIdx.x] = count_sum;
+    s.tile_b[blockIdx.x] = arrival_sum;
   }
 }
 
-// Per bin: the stayer base (stayer p of the bin lands at base + p -
-// crossers_before(p)), after the scans. With a consistent old state (the new
-// counts add up to the particles) a non-empty halo bin is flagged as by the
-// run-based plan.
-__global__ __launch_bounds__(kThreads) void k_cross_base(Grid g, uint32_t n, const uint32_t* __restrict__ counts,
-                                                         const uint32_t* __restrict__ offsets,
-                                                         const uint32_t* __restrict__ shift,
-                                                         const uint32_t* __restrict__ lower,
-                                                         uint32_t* __restrict__ bin_base,
-                                                         uint32_t* __restrict__ status,
-                                                         unsigned* __restrict__ validation) {
-  const uint32_t bins = g.bins();
-  const bool consistent = offsets[bins] == n;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && !consistent) atomicOr(status, 2u);
-  if (!consistent) return;
-  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < bins; b += gridDim.x * blockDim.x) {
-    if (counts[b] != 0) {
-      int i, j, k;
-      g.decode(int32_t(b), i, j, k);
-      if (!g.interior(i, j, k)) atomicOr(validation, kInvalidHalo);
+// The scans of counts and arrivals, and per bin the stayer base (stayer p of
+// the bin lands at base + p - crossers_before(p)). With a consistent old state
+// (the new counts add up to the particles) a non-empty halo bin is flagged as
+// by the run-based plan.
+__global__ __launch_bounds__(kThreads) void k_cross_offsets(CrossPlans plans, Grid g,
+                                                            unsigned* __restrict__ validation) {
+  const CrossPlan& s = plans.species[blockIdx.y];
+  __shared__ uint32_t lds[kThreads / 64];
+  const uint32_t bins = g.bins(), tiles = (bins + kPlanTile - 1) / kPlanTile;
+  const uint32_t first = blockIdx.x * kPlanTile + threadIdx.x * kPlanItems;
+  uint32_t count[kPlanItems], arrive[kPlanItems], base[kPlanItems], count_sum = 0, arrival_sum = 0;
+#pragma unroll
+  for (unsigned r = 0; r < kPlanItems; ++r) {
+    const bool in = first + r < bins;
+    count[r] = in ? s.counts[first + r] : 0u;
+    arrive[r] = in ? s.arrivals[first + r] : 0u;
+    base[r] = in ? s.lower[first + r] + s.shift[first + r] : 0u;
+    count_sum += count[r];
+    arrival_sum += arrive[r];
+  }
+  const uint32_t total = tiles_before(s.tile_a, tiles, lds);
+  uint32_t at = tiles_before(s.tile_a, blockIdx.x, lds);
+  uint32_t arrival_at = tiles_before(s.tile_b, blockIdx.x, lds);
+  at += block_exclusive(count_sum, lds);
+  arrival_at += block_exclusive(arrival_sum, lds);
+  const bool consistent = total == s.n;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && !consistent) atomicOr(s.status, 2u);
+#pragma unroll
+  for (unsigned r = 0; r < kPlanItems; ++r) {
+    const uint32_t b = first + r;
+    if (b < bins) {
+      s.offsets[b] = at;
+      s.arrival_offset[b] = arrival_at;
+      s.bin_base[b] = at + base[r];
+      if (consistent && count[r] != 0) {
+        int i, j, k;
+        g.decode(int32_t(b), i, j, k);
+        if (!g.interior(i, j, k)) atomicOr(validation, kInvalidHalo);
+      }
     }
-    bin_base[b] = offsets[b] + lower[b] + shift[b];
+    at += count[r];
+    arrival_at += arrive[r];
+    if (b + 1 == bins) {
+      s.offsets[bins] = at;
+      s.arrival_offset[bins] = arrival_at;
+    }
   }
 }
 
 // Source-ordered pass over tiles of kTile particles: a stayer writes its own
 // source entry; a crosser is listed among its new bin's arrivals (at its
 // index j within the bin).
-__global__ __launch_bounds__(kThreads) void k_cross_sources(const int32_t* __restrict__ keys, uint32_t n, uint32_t bins,
-                                                            const uint64_t* __restrict__ cross,
-                                                            const uint32_t* __restrict__ block_base,
-                                                            const uint32_t* __restrict__ bin_base,
-                                                            const uint32_t* __restrict__ arr_off,
-                                                            const uint32_t* __restrict__ slot,
-                                                            uint32_t* __restrict__ bin_arrivals,
-                                                            const uint32_t* __restrict__ status,
-                                                            uint32_t* __restrict__ source) {
-  if (*status) return;
+__global__ __launch_bounds__(kThreads) void k_cross_sources(CrossPlans plans, uint32_t bins) {
+  const CrossPlan& s = plans.species[blockIdx.y];
+  const uint32_t n = s.n;
+  if (*s.status) return;
   const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t sub = blockIdx.x * kTile + wave * kWaveSpan;
   if (sub >= n) return;
   // Lane r < kWaveItems holds the crosser word and crossers-before of item r.
   const uint32_t blk0 = sub >> 6;  // sub is a multiple of 64
   const bool item_lane = lane < kWaveItems && sub + lane * 64u < n;
-  const uint64_t words = item_lane ? cross[blk0 + lane] : 0ull;
-  const uint32_t bases = item_lane ? block_base[blk0 + lane] : 0u;
+  const uint64_t words = item_lane ? s.cross[blk0 + lane] : 0ull;
+  const uint32_t bases = item_lane ? s.block_base[blk0 + lane] : 0u;
   int32_t key[kWaveItems];
 #pragma unroll
   for (unsigned r = 0; r < kWaveItems; ++r) {
     const uint32_t i = sub + r * 64 + lane;
-    key[r] = i < n ? keys[i] : -1;
+    key[r] = i < n ? s.keys[i] : -1;
   }
   // Every item's crosser bit and crossers-before first (lane reads only), so
   // the gathers below are issued back to back.
@@ -679,9 +796,9 @@ __global__ __launch_bounds__(kThreads) void k_cross_sources(const int32_t* __res
   for (unsigned r = 0; r < kWaveItems; ++r) {
     const bool valid = key[r] >= 0 && uint32_t(key[r]) < bins;
     const bool crosser = (crossers >> r) & 1u;
-    const uint32_t* table = crosser ? arr_off : bin_base;
+    const uint32_t* table = crosser ? s.arrival_offset : s.bin_base;
     const uint32_t base_or_offset = valid ? table[key[r]] : 0u;
-    const uint32_t j = (valid && crosser) ? slot[before[r]] : 0u;
+    const uint32_t j = (valid && crosser) ? s.slot[before[r]] : 0u;
     target[r] = crosser ? base_or_offset + j : base_or_offset - before[r];
   }
   wait_loads();
@@ -690,53 +807,102 @@ __global__ __launch_bounds__(kThreads) void k_cross_sources(const int32_t* __res
     const uint32_t i = sub + r * 64 + lane;
     if (key[r] < 0 || uint32_t(key[r]) >= bins) continue;
     if ((crossers >> r) & 1u) {
-      bin_arrivals[target[r]] = i;
+      s.bin_arrivals[target[r]] = i;
     } else {
       const uint32_t dest = target[r] + i;
-      if (dest < n) source[dest] = i;
+      if (dest < n) s.source[dest] = i;
     }
   }
 }
 
+// One bin's arrivals: where they lie in bin_arrivals, the bin's first
+// destination, those from lower bins and the stayers.
+struct Arrivals {
+  uint32_t k, at, first, below, stay;
+  // Destination of the arrival of rank r in position order: before the stayers
+  // those from lower bins, after them the others.
+  __device__ __forceinline__ uint32_t destination(uint32_t r) const { return first + r + (r >= below ? stay : 0u); }
+};
+
+__device__ __forceinline__ Arrivals bin_arrivals_of(const CrossPlan& s, uint32_t b) {
+  Arrivals a;
+  a.k = s.arrivals[b];
+  a.at = s.arrival_offset[b];
+  a.first = s.offsets[b];
+  a.below = s.lower[b];
+  a.stay = s.counts[b] - a.k;
+  return a;
+}
+
 // Per bin: the arrivals in position order (rank = arrivals at smaller
-// positions; positions are distinct) at their destinations: before the
-// stayers those from lower bins, after them the others.
-__global__ __launch_bounds__(kThreads) void k_cross_bins(uint32_t bins, uint32_t n,
-                                                         const uint32_t* __restrict__ counts,
-                                                         const uint32_t* __restrict__ offsets,
-                                                         const uint32_t* __restrict__ arrivals,
-                                                         const uint32_t* __restrict__ arr_off,
-                                                         const uint32_t* __restrict__ bin_arrivals,
-                                                         const uint32_t* __restrict__ lower,
-                                                         const uint32_t* __restrict__ status,
-                                                         uint32_t* __restrict__ source) {
-  if (*status) return;
-  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < bins; b += gridDim.x * blockDim.x) {
-    const uint32_t k = arrivals[b];
-    if (k == 0 || k > kArrivalsMax) continue;
-    const uint32_t a0 = arr_off[b], d0 = offsets[b], below = lower[b], stay = counts[b] - k;
-    if (k <= kArrivalsInRegisters) {
+// positions; positions are distinct) at their destinations. A thread takes a
+// bin of up to kArrivalsInRegisters arrivals; the block's waves share the
+// others, a lane per arrival (100 particles a cell with a sixth of them
+// crossing: a thread per such bin read them k^2 times, 186 us per species of a
+// 512 x 512 plane). The halo bins' records are then copied, as after the
+// run-based plan (the fused gather and deposition visits interior cells only).
+// A block takes `per_block` bins (at most its threads): fewer where most bins
+// have more arrivals than a thread orders.
+__global__ __launch_bounds__(kThreads) void k_cross_bins(CrossPlans plans, Grid g, uint32_t per_block) {
+  const CrossPlan& s = plans.species[blockIdx.y];
+  if (*s.status) return;
+  __shared__ uint32_t s_listed, s_list[kThreads];
+  const uint32_t n = s.n, end = (blockIdx.x + 1) * per_block;
+  const uint32_t bins = end < g.bins() ? end : g.bins();  // of this block and those before it
+  const uint32_t b = threadIdx.x < per_block ? blockIdx.x * per_block + threadIdx.x : bins;
+  if (threadIdx.x == 0) s_listed = 0;
+  __syncthreads();
+  if (b < bins) {
+    const Arrivals a = bin_arrivals_of(s, b);
+    if (a.k > kArrivalsInRegisters) {
+      s_list[atomicAdd(&s_listed, 1u)] = b;
+    } else if (a.k != 0) {
       uint32_t pos[kArrivalsInRegisters];
 #pragma unroll
-      for (uint32_t r = 0; r < kArrivalsInRegisters; ++r) pos[r] = r < k ? bin_arrivals[a0 + r] : 0xffffffffu;
+      for (uint32_t r = 0; r < kArrivalsInRegisters; ++r) pos[r] = r < a.k ? s.bin_arrivals[a.at + r] : 0xffffffffu;
 #pragma unroll
       for (uint32_t r = 0; r < kArrivalsInRegisters; ++r) {
-        if (r >= k) break;
+        if (r >= a.k) break;
         uint32_t rank = 0;
 #pragma unroll
         for (uint32_t q = 0; q < kArrivalsInRegisters; ++q) rank += pos[q] < pos[r] ? 1u : 0u;
-        const uint32_t dest = d0 + rank + (rank >= below ? stay : 0u);
-        if (dest < n) source[dest] = pos[r];
-      }
-    } else {
-      for (uint32_t r = 0; r < k; ++r) {
-        const uint32_t p = bin_arrivals[a0 + r];
-        uint32_t rank = 0;
-        for (uint32_t q = 0; q < k; ++q) rank += bin_arrivals[a0 + q] < p ? 1u : 0u;
-        const uint32_t dest = d0 + rank + (rank >= below ? stay : 0u);
-        if (dest < n) source[dest] = p;
+        const uint32_t dest = a.destination(rank);
+        if (dest < n) s.source[dest] = pos[r];
       }
     }
+  }
+  __syncthreads();
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t listed = s_listed;
+  for (uint32_t l = wave; l < listed; l += kThreads / 64) {
+    const Arrivals a = bin_arrivals_of(s, uint32_t(__builtin_amdgcn_readfirstlane(int(s_list[l]))));
+    for (uint32_t r0 = 0; r0 < a.k; r0 += 64) {
+      const uint32_t pos = r0 + lane < a.k ? s.bin_arrivals[a.at + r0 + lane] : 0xffffffffu;
+      uint32_t rank = 0;
+      for (uint32_t q0 = 0; q0 < a.k; q0 += 64) {
+        const uint32_t other = q0 == r0 ? pos : (q0 + lane < a.k ? s.bin_arrivals[a.at + q0 + lane] : 0xffffffffu);
+        const uint32_t m = a.k - q0 < 64u ? a.k - q0 : 64u;
+        for (uint32_t t = 0; t < m; ++t)
+          rank += uint32_t(__builtin_amdgcn_readlane(int(other), int(t))) < pos ? 1u : 0u;
+      }
+      const uint32_t dest = a.destination(rank);
+      if (r0 + lane < a.k && dest < n) s.source[dest] = pos;
+    }
+  }
+  // The halo bins of this block: their sources are complete now (a listed
+  // bin's were written by another wave of the block).
+  __threadfence_block();
+  __syncthreads();
+  if (b >= bins) return;
+  const uint32_t count = s.counts[b];
+  if (count == 0) return;
+  int i, j, k;
+  g.decode(int32_t(b), i, j, k);
+  if (g.interior(i, j, k)) return;
+  for (uint32_t d = s.offsets[b]; d < s.offsets[b] + count; ++d) {
+    Record rec;
+    load_record(s.src, s.source[d], rec);
+    store_record(s.dst, d, rec);
   }
 }
 
@@ -898,65 +1064,66 @@ int launch_sort_plan(Context& ctx, int s, SortWorkspace& ws, hipStream_t st) {
   return 0;
 }
 
-int launch_sort_plan_incremental(Context& ctx, int s, SortWorkspace& ws, hipStream_t st) {
-  SpeciesState& sp = ctx.species[size_t(s)];
-  const uint32_t n = sp.count;
+int launch_sort_plan_incremental(Context& ctx, int first, int species, SortWorkspace* const* ws, hipStream_t st) {
   const Grid& g = ctx.grid;
   const uint32_t bins = g.bins();
-  uint32_t* status = ctx.plan_status + s;
   const bool timed = st == ctx.stream;
   if (timed) phase_begin(ctx, Phase::sort);
-  int rc = 0;
-#define TPIC_TRY(expr, what)            \
-  do {                                 \
-    rc = check_hip(ctx, (expr), what); \
-    if (rc) return rc;                 \
-  } while (0)
-  TPIC_TRY(hipMemsetAsync(status, 0, sizeof(uint32_t), st), "plan clear");
-  if (n == 0) {
-    TPIC_TRY(hipMemsetAsync(sp.counts, 0, bins * sizeof(uint32_t), st), "sort clear");
-    TPIC_TRY(hipMemsetAsync(sp.offsets, 0, (bins + 1) * sizeof(uint32_t), st), "sort clear");
-    if (timed) phase_end(ctx, Phase::sort);
-    return 0;
+  CrossPlans plans{};
+  uint32_t blocks = 0, tiles = 0;
+  for (int t = 0; t < species; ++t) {
+    SpeciesState& sp = ctx.species[size_t(first + t)];
+    SortWorkspace& w = *ws[t];
+    if (sp.count > w.capacity || !sp.cross || sp.count == 0) return fail(ctx, -3, "plan workspace too small");
+    CrossPlan& p = plans.species[t];
+    p.src = sp.view();
+    p.dst = sp.scratch();
+    p.keys = p.src.cell;
+    p.cross = sp.cross;
+    p.n = sp.count;
+    p.blocks = (p.n + 63u) / 64u;
+    p.block_base = w.block_base;
+    // Arrays of the run-based plan's table.
+    p.arrivals = w.rcounts;
+    p.arrival_offset = w.roffsets;
+    p.slot = w.run_start;
+    p.shift = w.large;
+    p.bin_arrivals = w.bin_runs;
+    p.lower = w.bin_lower;
+    p.bin_base = w.bin_base;
+    const uint32_t sums = (std::max(p.blocks, bins) + kPlanTile - 1) / kPlanTile;
+    if (2 * size_t(sums) > w.scan_scratch_words) return fail(ctx, -3, "scan scratch too small");
+    p.tile_a = w.scan_scratch;
+    p.tile_b = w.scan_scratch + sums;
+    p.counts = sp.counts;
+    p.offsets = sp.offsets;
+    p.source = sp.source;
+    p.status = ctx.plan_status + first + t;
+    blocks = std::max(blocks, p.blocks);
+    tiles = std::max(tiles, (p.n + kTile - 1) / kTile);
   }
-  if (n > ws.capacity || !sp.cross) return fail(ctx, -3, "plan workspace too small");
-  const uint32_t blocks = (n + 63u) / 64u;
-  TPIC_TRY(hipMemsetAsync(ws.rcounts, 0, bins * sizeof(uint32_t), st), "plan clear");
-  TPIC_TRY(hipMemsetAsync(ws.bin_lower, 0, bins * sizeof(uint32_t), st), "plan clear");
-  const unsigned bin_blocks = (bins + kThreads - 1) / kThreads;
-  const ParticleView src = sp.view(), dst = sp.scratch();
-  // Run-table arrays reused: run_dest the crossers per block, run_start (by
-  // crosser list index) each crosser's index among its bin's arrivals,
-  // rcounts and roffsets the
-  // arrivals per bin and their offsets, large each bin's shift, bin_runs the
-  // arrivals by bin.
-  const uint32_t tiles = (n + kTile - 1) / kTile;
-  k_cross_counts<<<(blocks + kThreads - 1) / kThreads, kThreads, 0, st>>>(sp.cross, blocks, ws.run_dest);
-  TPIC_TRY(hipGetLastError(), "plan crossers");
-  if ((rc = exclusive_scan(ctx, ws, st, ws.run_dest, ws.block_base, blocks))) return rc;
-  k_cross_arrivals<<<tiles, kThreads, 0, st>>>(sp.cross, n, ws.block_base, src.cell, bins, sp.offsets, ws.rcounts,
-                                               ws.bin_lower, ws.run_start, status);
-  TPIC_TRY(hipGetLastError(), "plan arrivals");
-  k_cross_counts_new<<<bin_blocks, kThreads, 0, st>>>(bins, sp.offsets, sp.cross, ws.block_base, blocks,
-                                                      ws.rcounts, sp.counts, ws.large, status);
-  TPIC_TRY(hipGetLastError(), "plan counts");
-  if ((rc = exclusive_scan(ctx, ws, st, sp.counts, sp.offsets, bins))) return rc;
-  if ((rc = exclusive_scan(ctx, ws, st, ws.rcounts, ws.roffsets, bins))) return rc;
-  k_cross_base<<<bin_blocks, kThreads, 0, st>>>(g, n, sp.counts, sp.offsets, ws.large, ws.bin_lower, ws.bin_base,
-                                                status, ctx.validation);
-  TPIC_TRY(hipGetLastError(), "plan bases");
-  k_cross_sources<<<tiles, kThreads, 0, st>>>(src.cell, n, bins, sp.cross, ws.block_base, ws.bin_base, ws.roffsets,
-                                               ws.run_start, ws.bin_runs, status, sp.source);
-  TPIC_TRY(hipGetLastError(), "plan sources");
-  k_cross_bins<<<bin_blocks, kThreads, 0, st>>>(bins, n, sp.counts, sp.offsets, ws.rcounts, ws.roffsets, ws.bin_runs,
-                                                ws.bin_lower, status, sp.source);
-  TPIC_TRY(hipGetLastError(), "plan arrival order");
-  k_copy_halo_bins<<<bin_blocks, kThreads, 0, st>>>(g, src, dst, sp.counts, sp.offsets, sp.source, status);
-  TPIC_TRY(hipGetLastError(), "plan halo copy");
-#undef TPIC_TRY
+  const unsigned y = unsigned(species);
+  const unsigned block_tiles = (blocks + kPlanTile - 1) / kPlanTile, bin_tiles = (bins + kPlanTile - 1) / kPlanTile;
+  k_cross_begin<<<dim3(std::max(block_tiles, bin_tiles), y), kThreads, 0, st>>>(plans, bins);
+  k_cross_bases<<<dim3(block_tiles, y), kThreads, 0, st>>>(plans);
+  k_cross_arrivals<<<dim3(tiles, y), kThreads, 0, st>>>(plans, bins);
+  k_cross_counts_new<<<dim3(bin_tiles, y), kThreads, 0, st>>>(plans, bins);
+  k_cross_offsets<<<dim3(bin_tiles, y), kThreads, 0, st>>>(plans, g, ctx.validation);
+  k_cross_sources<<<dim3(tiles, y), kThreads, 0, st>>>(plans, bins);
+  // A species' arrivals a bin grow with its particles a cell (a few percent to
+  // a sixth of them): at 1000 a cell nearly every bin is listed, and 256 bins
+  // a block leave four waves 64 lists each (479 us for a 1024-cell line).
+  uint64_t particles = 0;
+  for (int t = 0; t < species; ++t) particles = std::max<uint64_t>(particles, plans.species[t].n);
+  const uint32_t per_block = particles >= 256ull * g.cells() ? 4u : (particles >= 80ull * g.cells() ? 64u : kThreads);
+  k_cross_bins<<<dim3((bins + per_block - 1) / per_block, y), kThreads, 0, st>>>(plans, g, per_block);
+  const int rc = check_hip(ctx, hipGetLastError(), "sort plan from crossers");
   if (timed) phase_end(ctx, Phase::sort);
-  return 0;
+  return rc;
 }
+
+// Words of scan scratch that the plan from the crossers needs (two tile sums).
+size_t cross_plan_words(size_t blocks, size_t bins) { return 2 * ((std::max(blocks, bins) + kPlanTile - 1) / kPlanTile); }
 
 int launch_sort_plan(Context& ctx, int s) { return launch_sort_plan(ctx, s, ctx.sort, ctx.stream); }
 
