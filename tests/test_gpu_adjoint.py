@@ -188,6 +188,51 @@ def test_adjoint_cycles_match_the_oracle_adjoint():
             assert np.abs(g_ - exp[key]).max() <= 1e-8 * np.abs(exp[key]).max(), (s, key)
 
 
+@pytest.mark.parametrize("ppc", [1, 7, 18, 19, 36, 37, 71])
+def test_adjoint_cycle_at_every_lane_group(ppc):
+    """Two adjoint cycles at the particles per cell on both sides of the lines
+    between the particle passes' lane groups (and odd particle counts, whose
+    checkpoint copies end in part words), cells not a multiple of a block's
+    groups: against the oracle's adjoint within 1e-8."""
+    rng = np.random.default_rng(60 + ppc)
+    cells, lengths, qoms, dt, cycles = (5, 3, 1), (2.5, 1.5, 0.5), (-8.0, 1.0), 0.2, 2
+    g, arrays = case(rng, cells, lengths, ppc=ppc, qoms=qoms)
+    box = AD.Box(g)
+    nc = O.cell_count(g)
+    e0 = box.expand(rng.normal(size=3 * box.unique) * 0.01)
+    b0 = rng.normal(size=3 * nc) * 0.05 + np.repeat([0.1, 0.0, 0.2], nc)
+    counts = [len(a["q"]) for a in arrays]
+    say("adjoint cycles, particles per cell", ppc)
+    with started(cells, lengths, arrays, qoms, e0, b0, dt=dt) as sim:
+        sim.checkpoint_reserve(cycles)
+        for n in range(cycles):
+            sim.checkpoint_save(n)
+            sim.cycle(1)
+        with sim.adjoint() as adj:
+            adj.seed_field_energy(1.0, 0.5, [0, 100000])
+            for n in range(cycles - 1, -1, -1):
+                sim.checkpoint_restore(n)
+                adj.cycle()
+            ebar, bbar = adj.field(R.FIELD_E), adj.field(R.FIELD_B)
+            parts = [adj.particles(s) for s in range(2)]
+    osim = O.Sim(cells, lengths, list(qoms), counts, dt, tol=1e-14, restart=60, max_iterations=400)
+    for s, a in enumerate(arrays):
+        osim.set_particles(s, a)
+    osim.field("E")[:] = e0
+    osim.field("B")[:] = b0
+    osim.initialize()
+    want = AD.gradient_of_field_energy(osim, box, AD.run_forward(osim, cycles), dt, 0.5, 1.0, 0.5)
+    osim.close()
+    assert np.abs(box.reduce(ebar) - want.ebar).max() <= 1e-8 * np.abs(want.ebar).max()
+    assert np.abs(bbar - want.bbar).max() <= 1e-8 * np.abs(want.bbar).max()
+    for s in range(2):
+        at = {int(x): n for n, x in enumerate(parts[s]["ids"])}
+        idx = np.array([at[int(x)] for x in want.particles[s]["ids"]])
+        for key in ("rbar", "vbar", "qbar"):
+            exp = want.particles[s][key]
+            assert np.abs(parts[s][key][..., idx] - exp).max() <= 1e-8 * np.abs(exp).max(), (s, key)
+
+
 def _oracle_two_stream_energy(model, v0, eps, cycles):
     """W_E after `cycles` of the oracle on the model's initial state at (v0, eps)."""
     v, q, e, b = (t.numpy() for t in model.state(v0, eps))

@@ -53,19 +53,22 @@ Context* context_of(tpic_mi_context* h);
 namespace {
 
 constexpr unsigned kThreads = 256;
-constexpr unsigned kWaves = kThreads / 64;
 
-// One species' adjoint arrays.
+// One species' adjoint arrays. The particle adjoints and the ids of the order
+// they are held in lie in two slots: a permutation writes the other slot,
+// which then becomes the current one.
 struct AdjointArrays {
   uint32_t count = 0;
   uint64_t first_id = 0;
-  double* rbar = nullptr;  // [3][count] dL/d(fraction)
-  double* vbar = nullptr;  // [3][count]
-  double* qbar = nullptr;  // [count]
+  double* slot[2]{};     // [7][count]: rbar (3), vbar (3), qbar
+  uint64_t* id_slot[2]{};
+  int current = 0;
   double* wbar = nullptr;  // [3][count] omega adjoint between the two particle passes
-  uint64_t* ids = nullptr; // [count] ids of the order the adjoint is held in
-  double* stage = nullptr; // [7][count] permutation staging
   uint32_t* inverse = nullptr;  // [count] position of id first + d in the context's order
+  double* rbar() const { return slot[current]; }                       // [3][count] dL/d(fraction)
+  double* vbar() const { return slot[current] + 3 * size_t(count); }   // [3][count]
+  double* qbar() const { return slot[current] + 6 * size_t(count); }   // [count]
+  uint64_t* ids() const { return id_slot[current]; }
 };
 
 // Per-particle parameters of a species in the particle passes.
@@ -87,18 +90,21 @@ struct PassConstants {
   double k;               // 4 pi theta dt
 };
 
-__device__ __forceinline__ void cic(double fx, double fy, double fz, double (&w)[8], double (&dw)[8][3]) {
-  const double wx[2] = {1.0 - fx, fx}, wy[2] = {1.0 - fy, fy}, wz[2] = {1.0 - fz, fz};
-  const double sx[2] = {-1.0, 1.0};
-#pragma unroll
-  for (int a = 0; a < 8; ++a) {
-    const int ax = a & 1, ay = (a >> 1) & 1, az = (a >> 2) & 1;
-    w[a] = (wx[ax] * wy[ay]) * wz[az];
-    dw[a][0] = sx[ax] * wy[ay] * wz[az];
-    dw[a][1] = sx[ay] * wx[ax] * wz[az];
-    dw[a][2] = sx[az] * wx[ax] * wy[ay];
+// CIC weights of a particle and their derivatives, formed per corner from the
+// six factors (32 values held at once took a lane's registers).
+struct Cic {
+  double x[2], y[2], z[2];
+  __device__ __forceinline__ Cic(double fx, double fy, double fz)
+      : x{1.0 - fx, fx}, y{1.0 - fy, fy}, z{1.0 - fz, fz} {}
+  __device__ __forceinline__ double w(int a) const { return (x[a & 1] * y[(a >> 1) & 1]) * z[a >> 2]; }
+  // r += s dW_a.
+  __device__ __forceinline__ void add_gradient(int a, double s, double (&r)[3]) const {
+    const int ax = a & 1, ay = (a >> 1) & 1, az = a >> 2;
+    r[0] += (ax ? s : -s) * (y[ay] * z[az]);
+    r[1] += (ay ? s : -s) * (x[ax] * z[az]);
+    r[2] += (az ? s : -s) * (x[ax] * y[ay]);
   }
-}
+};
 
 // alpha (row-major) of omega.
 __device__ __forceinline__ void response(const double (&om)[3], double (&al)[9], double& d) {
@@ -150,41 +156,57 @@ struct CellWalk {
   uint32_t first, count;
 };
 
+template <unsigned Group>
 __device__ __forceinline__ void stage_corners(const Grid& g, const CellWalk& c, const double* const* fields,
                                               int nfields, unsigned lane, double* lds) {
   const unsigned nodes = g.nodes();
-  for (unsigned t = lane; t < unsigned(24 * nfields); t += 64) {
+  for (unsigned t = lane; t < unsigned(24 * nfields); t += Group) {
     const unsigned f = t / 24, comp = (t / 8) % 3, a = t % 8;
     const unsigned n = g.node(c.i + int(a & 1), c.j + int((a >> 1) & 1), c.k + int((a >> 2) & 1));
     lds[t] = fields[f][size_t(comp) * nodes + n];
   }
+}
+
+__device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
   asm volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ void gather(const double (&w)[8], const double* lds, int field, double (&out)[3]) {
+__device__ __forceinline__ void gather(const Cic& w, const double* lds, int field, double (&out)[3]) {
+  out[0] = out[1] = out[2] = 0.0;
 #pragma unroll
-  for (int comp = 0; comp < 3; ++comp) {
-    double s = 0.0;
+  for (int a = 0; a < 8; ++a) {
+    const double v = w.w(a);
 #pragma unroll
-    for (int a = 0; a < 8; ++a) s += w[a] * lds[field * 24 + comp * 8 + a];
-    out[comp] = s;
+    for (int comp = 0; comp < 3; ++comp) out[comp] += v * lds[field * 24 + comp * 8 + a];
   }
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// Sum over the wave of the 24 corner accumulators; lane 0 writes the cell's
-// record [corner * 3 + component][cells].
-__device__ __forceinline__ void flush_corners(double (&acc)[24], unsigned lane, unsigned cell, unsigned cells,
-                                              double* __restrict__ record) {
+// Sum over a group's lanes of the 24 corner accumulators into the cell's
+// record [corner * 3 + component][cells]. The first three exchanges halve the
+// values a lane carries (12, 6, then 3), so a group of 32 exchanges 27 values,
+// not 24 x 5; eight lanes then hold three sums each.
+template <unsigned Group>
+__device__ __forceinline__ void flush_corners(double (&acc)[24], unsigned lane, bool active, unsigned cell,
+                                              unsigned cells, double* __restrict__ record) {
+  unsigned first = 0;
 #pragma unroll
-  for (int t = 0; t < 24; ++t) {
-    double v = acc[t];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    acc[t] = v;
+  for (int half = 12, mask = int(Group) / 2; half >= 3; half /= 2, mask /= 2) {
+    const bool upper = (lane & unsigned(mask)) != 0;
+#pragma unroll
+    for (int t = 0; t < half; ++t) {
+      const double send = upper ? acc[t] : acc[t + half], keep = upper ? acc[t + half] : acc[t];
+      acc[t] = keep + __shfl_xor(send, mask, 64);
+    }
+    first += upper ? unsigned(half) : 0u;
   }
-  if (lane == 0) {
 #pragma unroll
-    for (int t = 0; t < 24; ++t) record[size_t(t) * cells + cell] = acc[t];
+  for (int t = 0; t < 3; ++t)
+    for (int mask = int(Group) / 16; mask > 0; mask /= 2) acc[t] += __shfl_xor(acc[t], mask, 64);
+  if (active && (lane & (Group / 8 - 1)) == 0) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) record[size_t(first + unsigned(t)) * cells + cell] = acc[t];
   }
 }
 
@@ -199,31 +221,40 @@ __device__ __forceinline__ bool next_cell(const Grid& g, const uint32_t* counts,
   return c.count != 0;
 }
 
+// Both particle passes give a cell to a group of Group lanes (16, 32 or 64, by
+// the species' particles per cell): with a wave per cell, 25 particles a cell
+// left 39 of its lanes idle and every cell paid 144 lane exchanges (222 and
+// 247 us per species of 192 x 160 cells).
+
 // Pass 1: the push's part. Reads rbar', vbar' (this order) and writes the
 // partial rbar, vbar, the omega adjoint, and per cell the scattered
 // E_theta adjoint.
-__global__ __launch_bounds__(kThreads) void k_adjoint_push(Grid g, SpeciesPass sp, PassConstants pc,
+template <unsigned Group>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_adjoint_push(Grid g, SpeciesPass sp, PassConstants pc,
                                                            const double* __restrict__ bnode,
                                                            const double* __restrict__ etheta,
                                                            double* __restrict__ record) {
-  __shared__ double s_stage[kWaves][48];
-  const unsigned lane = threadIdx.x & 63u;
-  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  double* lds = s_stage[wave];
+  constexpr unsigned kGroups = kThreads / Group;
+  __shared__ double s_stage[kGroups][48];
+  const unsigned lane = threadIdx.x % Group, group = threadIdx.x / Group;
+  double* lds = s_stage[group];
   const unsigned cells = g.cells();
   const double* fields[2] = {bnode, etheta};
-  for (unsigned cell = blockIdx.x * kWaves + wave; cell < cells; cell += gridDim.x * kWaves) {
+  for (unsigned base = blockIdx.x * kGroups; base < cells; base += gridDim.x * kGroups) {
+    const unsigned cell = base + group;
+    const bool active = cell < cells;
     CellWalk c;
     double acc[24];
 #pragma unroll
     for (int t = 0; t < 24; ++t) acc[t] = 0.0;
-    if (next_cell(g, sp.counts, sp.offsets, cell, c)) {
-      stage_corners(g, c, fields, 2, lane, lds);
-      for (uint32_t o = lane; o < c.count; o += 64) {
+    const bool populated = active && next_cell(g, sp.counts, sp.offsets, cell, c);
+    if (populated) stage_corners<Group>(g, c, fields, 2, lane, lds);
+    wave_sync();
+    if (populated) {
+      for (uint32_t o = lane; o < c.count; o += Group) {
         const uint32_t at = c.first + o;
         const size_t n = sp.count;
-        double w[8], dw[8][3];
-        cic(sp.p.rx[at], sp.p.ry[at], sp.p.rz[at], w, dw);
+        const Cic w(sp.p.rx[at], sp.p.ry[at], sp.p.rz[at]);
         double bp[3], ep[3];
         gather(w, lds, 0, bp);
         gather(w, lds, 1, ep);
@@ -247,12 +278,12 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_push(Grid g, SpeciesPass s
         for (int a = 0; a < 8; ++a) {
           const double ea[3] = {lds[24 + a], lds[32 + a], lds[40 + a]};
           const double s = dot3(ebar_p, ea);
-          rb[0] += dw[a][0] * s;
-          rb[1] += dw[a][1] * s;
-          rb[2] += dw[a][2] * s;
-          acc[a * 3 + 0] += w[a] * ebar_p[0];
-          acc[a * 3 + 1] += w[a] * ebar_p[1];
-          acc[a * 3 + 2] += w[a] * ebar_p[2];
+          w.add_gradient(a, s, rb);
+          const double wa = w.w(a);
+          acc[a * 3 + 0] += wa * ebar_p[0];
+          acc[a * 3 + 1] += wa * ebar_p[1];
+          acc[a * 3 + 2] += wa * ebar_p[2];
+          if (a & 1) __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int c3 = 0; c3 < 3; ++c3) {
@@ -261,39 +292,42 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_push(Grid g, SpeciesPass s
           sp.wbar[c3 * n + at] = wb[c3];
         }
       }
-      __builtin_amdgcn_wave_barrier();
-      asm volatile("" ::: "memory");
     }
-    flush_corners(acc, lane, cell, cells, record);
+    wave_sync();
+    flush_corners<Group>(acc, lane, active, cell, cells, record);
   }
 }
 
 // Pass 2: the deposition's part (J and M) with mu, then the whole omega
 // adjoint scattered into Bnbar; writes the state-n rbar, vbar, qbar.
-__global__ __launch_bounds__(kThreads) void k_adjoint_deposit(Grid g, SpeciesPass sp, PassConstants pc,
+template <unsigned Group>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_adjoint_deposit(Grid g, SpeciesPass sp, PassConstants pc,
                                                               const double* __restrict__ bnode,
                                                               const double* __restrict__ etheta,
                                                               const double* __restrict__ mu,
                                                               double* __restrict__ record) {
-  __shared__ double s_stage[kWaves][72];
-  const unsigned lane = threadIdx.x & 63u;
-  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  double* lds = s_stage[wave];
+  constexpr unsigned kGroups = kThreads / Group;
+  __shared__ double s_stage[kGroups][72];
+  const unsigned lane = threadIdx.x % Group, group = threadIdx.x / Group;
+  double* lds = s_stage[group];
   const unsigned cells = g.cells();
   const double* fields[3] = {bnode, etheta, mu};
   const double t_mass = -(pc.k * pc.inverse_volume) * sp.beta_over_c;
-  for (unsigned cell = blockIdx.x * kWaves + wave; cell < cells; cell += gridDim.x * kWaves) {
+  for (unsigned base = blockIdx.x * kGroups; base < cells; base += gridDim.x * kGroups) {
+    const unsigned cell = base + group;
+    const bool active = cell < cells;
     CellWalk c;
     double acc[24];
 #pragma unroll
     for (int t = 0; t < 24; ++t) acc[t] = 0.0;
-    if (next_cell(g, sp.counts, sp.offsets, cell, c)) {
-      stage_corners(g, c, fields, 3, lane, lds);
-      for (uint32_t o = lane; o < c.count; o += 64) {
+    const bool populated = active && next_cell(g, sp.counts, sp.offsets, cell, c);
+    if (populated) stage_corners<Group>(g, c, fields, 3, lane, lds);
+    wave_sync();
+    if (populated) {
+      for (uint32_t o = lane; o < c.count; o += Group) {
         const uint32_t at = c.first + o;
         const size_t n = sp.count;
-        double w[8], dw[8][3];
-        cic(sp.p.rx[at], sp.p.ry[at], sp.p.rz[at], w, dw);
+        const Cic w(sp.p.rx[at], sp.p.ry[at], sp.p.rz[at]);
         double bp[3], ep[3], m[3];
         gather(w, lds, 0, bp);
         gather(w, lds, 1, ep);
@@ -335,12 +369,12 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_deposit(Grid g, SpeciesPas
           const double ba[3] = {lds[a], lds[8 + a], lds[16 + a]};
           const double s = sj * (-pc.k) * dot3(mua, av) + t_mass * q * (dot3(mua, ae) + dot3(atm, ea)) +
                            dot3(bbar, ba);
-          rb[0] += dw[a][0] * s;
-          rb[1] += dw[a][1] * s;
-          rb[2] += dw[a][2] * s;
-          acc[a * 3 + 0] += w[a] * bbar[0];
-          acc[a * 3 + 1] += w[a] * bbar[1];
-          acc[a * 3 + 2] += w[a] * bbar[2];
+          w.add_gradient(a, s, rb);
+          const double wa = w.w(a);
+          acc[a * 3 + 0] += wa * bbar[0];
+          acc[a * 3 + 1] += wa * bbar[1];
+          acc[a * 3 + 2] += wa * bbar[2];
+          if (a & 1) __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int c3 = 0; c3 < 3; ++c3) {
@@ -349,10 +383,9 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_deposit(Grid g, SpeciesPas
         }
         sp.qbar[at] = qb;
       }
-      __builtin_amdgcn_wave_barrier();
-      asm volatile("" ::: "memory");
     }
-    flush_corners(acc, lane, cell, cells, record);
+    wave_sync();
+    flush_corners<Group>(acc, lane, active, cell, cells, record);
   }
 }
 
@@ -424,9 +457,8 @@ __global__ __launch_bounds__(kThreads) void k_id_inverse(const uint64_t* __restr
 __global__ __launch_bounds__(kThreads) void k_permute(const uint64_t* __restrict__ from_ids,
                                                       const uint64_t* __restrict__ to_ids, uint32_t count,
                                                       uint64_t first, const uint32_t* __restrict__ inverse,
-                                                      const double* __restrict__ rbar,
-                                                      const double* __restrict__ vbar,
-                                                      const double* __restrict__ qbar, double* __restrict__ stage,
+                                                      const double* __restrict__ from, double* __restrict__ to,
+                                                      uint64_t* __restrict__ held_ids,
                                                       unsigned* __restrict__ flag) {
   for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < count; j += gridDim.x * blockDim.x) {
     const uint64_t d = from_ids[j] - first;
@@ -440,11 +472,8 @@ __global__ __launch_bounds__(kThreads) void k_permute(const uint64_t* __restrict
       continue;
     }
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      stage[size_t(c) * count + i] = rbar[size_t(c) * count + j];
-      stage[size_t(3 + c) * count + i] = vbar[size_t(c) * count + j];
-    }
-    stage[size_t(6) * count + i] = qbar[j];
+    for (int c = 0; c < 7; ++c) to[size_t(c) * count + i] = from[size_t(c) * count + j];
+    held_ids[i] = from_ids[j];
   }
 }
 
@@ -454,8 +483,14 @@ unsigned grid_for(const Context& ctx, uint64_t work) {
   return unsigned(want < cap ? (want ? want : 1) : cap);
 }
 
-unsigned cell_blocks(const Context& ctx) {
-  const unsigned want = (ctx.grid.cells() + kWaves - 1) / kWaves;
+// Lanes per cell of the particle passes.
+unsigned cell_group(const Context& ctx, uint32_t count) {
+  const uint64_t cells = ctx.grid.cells();
+  return count > 36 * cells ? 64u : (count > 18 * cells ? 32u : 16u);
+}
+
+unsigned cell_blocks(const Context& ctx, unsigned group) {
+  const unsigned groups = kThreads / group, want = (ctx.grid.cells() + groups - 1) / groups;
   const unsigned cap = unsigned(ctx.cus > 0 ? ctx.cus : 256) * 16;
   return want < cap ? want : cap;
 }
@@ -497,8 +532,8 @@ namespace {
 
 void free_adjoint(tpic_mi_adjoint* a) {
   for (auto& s : a->species) {
-    device_free(s.rbar); device_free(s.vbar); device_free(s.qbar); device_free(s.wbar);
-    device_free(s.ids); device_free(s.stage); device_free(s.inverse);
+    device_free(s.slot[0]); device_free(s.slot[1]); device_free(s.id_slot[0]); device_free(s.id_slot[1]);
+    device_free(s.wbar); device_free(s.inverse);
   }
   device_free(a->ebar); device_free(a->bbar); device_free(a->ethetabar); device_free(a->mu);
   device_free(a->bnbar); device_free(a->curl); device_free(a->curl_cells); device_free(a->record);
@@ -516,15 +551,10 @@ int adjoint_supported(Context& c) {
   return 0;
 }
 
-int read_flag(Context& c, tpic_mi_adjoint* a, unsigned* out) {
-  int rc = check_hip(c, hipMemcpyAsync(a->host_flag, a->flag, sizeof(unsigned), hipMemcpyDeviceToHost, c.stream),
-                     "adjoint flag");
-  if (!rc) rc = check_hip(c, hipStreamSynchronize(c.stream), "adjoint flag");
-  if (!rc) *out = *a->host_flag;
-  return rc;
-}
-
-// Moves the particle adjoints into the context's current particle order.
+// The particle adjoints permuted into the context's current particle order in
+// each species' other slot, and the id check word on its way to the host
+// (valid after the stream's next synchronisation; the slots change when it is
+// clear).
 int permute_to_context(Context& c, tpic_mi_adjoint* a) {
   int rc = check_hip(c, hipMemsetAsync(a->flag, 0, sizeof(unsigned), c.stream), "adjoint flag");
   if (rc) return rc;
@@ -533,28 +563,14 @@ int permute_to_context(Context& c, tpic_mi_adjoint* a) {
     if (ad.count == 0) continue;
     const ParticleView v = c.species[s].view();
     const unsigned blocks = grid_for(c, ad.count);
+    const int other = ad.current ^ 1;
     k_id_inverse<<<blocks, kThreads, 0, c.stream>>>(v.id, ad.count, ad.first_id, ad.inverse, a->flag);
-    k_permute<<<blocks, kThreads, 0, c.stream>>>(ad.ids, v.id, ad.count, ad.first_id, ad.inverse, ad.rbar, ad.vbar,
-                                                 ad.qbar, ad.stage, a->flag);
+    k_permute<<<blocks, kThreads, 0, c.stream>>>(ad.ids(), v.id, ad.count, ad.first_id, ad.inverse,
+                                                 ad.slot[ad.current], ad.slot[other], ad.id_slot[other], a->flag);
     if ((rc = check_hip(c, hipGetLastError(), "adjoint permutation"))) return rc;
-    // The staged values become the arrays; ids follow the context.
-    const size_t n = ad.count;
-    if ((rc = check_hip(c, hipMemcpyAsync(ad.rbar, ad.stage, 3 * n * sizeof(double), hipMemcpyDeviceToDevice, c.stream),
-                        "adjoint permutation")) ||
-        (rc = check_hip(c, hipMemcpyAsync(ad.vbar, ad.stage + 3 * n, 3 * n * sizeof(double), hipMemcpyDeviceToDevice,
-                                          c.stream),
-                        "adjoint permutation")) ||
-        (rc = check_hip(c, hipMemcpyAsync(ad.qbar, ad.stage + 6 * n, n * sizeof(double), hipMemcpyDeviceToDevice,
-                                          c.stream),
-                        "adjoint permutation")) ||
-        (rc = check_hip(c, hipMemcpyAsync(ad.ids, v.id, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, c.stream),
-                        "adjoint permutation")))
-      return rc;
   }
-  unsigned bad = 0;
-  if ((rc = read_flag(c, a, &bad))) return rc;
-  if (bad) return fail(c, TPIC_MI_INVALID_STATE, "particle ids are not a permutation of each species' first ids");
-  return 0;
+  return check_hip(c, hipMemcpyAsync(a->host_flag, a->flag, sizeof(unsigned), hipMemcpyDeviceToHost, c.stream),
+                   "adjoint flag");
 }
 
 SpeciesPass species_pass(Context& c, AdjointArrays& ad, size_t s) {
@@ -563,9 +579,9 @@ SpeciesPass species_pass(Context& c, AdjointArrays& ad, size_t s) {
   p.count = c.species[s].count;
   p.counts = c.species[s].counts;
   p.offsets = c.species[s].offsets;
-  p.rbar = ad.rbar;
-  p.vbar = ad.vbar;
-  p.qbar = ad.qbar;
+  p.rbar = ad.rbar();
+  p.vbar = ad.vbar();
+  p.qbar = ad.qbar();
   p.wbar = ad.wbar;
   // prepare_particle_mover_parameters: beta = (q/m) dt / 2; the response
   // and the mass scale use beta / c.
@@ -619,9 +635,9 @@ int tpic_mi_adjoint_create(tpic_mi_context* h, tpic_mi_adjoint** out) {
     AdjointArrays& ad = a->species[s];
     ad.count = c.species[s].count;
     const size_t n = ad.count;
-    if ((rc = device_alloc(c, &ad.rbar, 3 * n, "adjoint")) || (rc = device_alloc(c, &ad.vbar, 3 * n, "adjoint")) ||
-        (rc = device_alloc(c, &ad.qbar, n, "adjoint")) || (rc = device_alloc(c, &ad.wbar, 3 * n, "adjoint")) ||
-        (rc = device_alloc(c, &ad.ids, n, "adjoint")) || (rc = device_alloc(c, &ad.stage, 7 * n, "adjoint")))
+    if ((rc = device_alloc(c, &ad.slot[0], 7 * n, "adjoint")) || (rc = device_alloc(c, &ad.slot[1], 7 * n, "adjoint")) ||
+        (rc = device_alloc(c, &ad.id_slot[0], n, "adjoint")) || (rc = device_alloc(c, &ad.id_slot[1], n, "adjoint")) ||
+        (rc = device_alloc(c, &ad.wbar, 3 * n, "adjoint")))
       break;
     rc = device_alloc(c, &ad.inverse, n, "adjoint");
   }
@@ -671,11 +687,9 @@ int tpic_mi_adjoint_seed(tpic_mi_context* h, tpic_mi_adjoint* a, double weight_e
     ad.first_id = first_ids[s];
     const size_t n = ad.count;
     if (!n) continue;
-    if ((rc = check_hip(c, hipMemsetAsync(ad.rbar, 0, 3 * n * sizeof(double), c.stream), "adjoint seed")) ||
-        (rc = check_hip(c, hipMemsetAsync(ad.vbar, 0, 3 * n * sizeof(double), c.stream), "adjoint seed")) ||
-        (rc = check_hip(c, hipMemsetAsync(ad.qbar, 0, n * sizeof(double), c.stream), "adjoint seed")))
+    if ((rc = check_hip(c, hipMemsetAsync(ad.slot[ad.current], 0, 7 * n * sizeof(double), c.stream), "adjoint seed")))
       break;
-    rc = check_hip(c, hipMemcpyAsync(ad.ids, c.species[s].view().id, n * sizeof(uint64_t), hipMemcpyDeviceToDevice,
+    rc = check_hip(c, hipMemcpyAsync(ad.ids(), c.species[s].view().id, n * sizeof(uint64_t), hipMemcpyDeviceToDevice,
                                      c.stream),
                    "adjoint seed");
   }
@@ -692,11 +706,16 @@ int tpic_mi_adjoint_cycle(tpic_mi_context* h, tpic_mi_adjoint* a, tpic_mi_solve_
     if (!sp.sorted) return fail(c, TPIC_MI_INVALID_STATE, "the adjoint cycle starts from a sorted state");
   const Grid& g = c.grid;
   const size_t nodes = g.nodes(), cells = g.cells();
-  // 1. The particle adjoints into this state's order.
+  // 1. The particle adjoints into this state's order; 2. E_theta of this
+  // cycle, recomputed as the forward cycle computed it (its solve waits for
+  // the stream, the id check word with it).
   int rc = permute_to_context(c, a);
   if (rc) return rc;
-  // 2. E_theta of this cycle, recomputed as the forward cycle computed it.
-  if ((rc = tpic_mi_solve(h, forward))) return rc;
+  const int solved = tpic_mi_solve(h, forward);
+  if (solved && (rc = check_hip(c, hipStreamSynchronize(c.stream), "adjoint flag"))) return rc;
+  if (*a->host_flag) return fail(c, TPIC_MI_INVALID_STATE, "particle ids are not a permutation of each species' first ids");
+  for (AdjointArrays& ad : a->species) ad.current ^= 1;
+  if (solved) return solved;
   // 3. Field update: Ebar_theta = Ebar'/theta - c dt curl_C2N(Bbar');
   //    Ebar^n = -(1 - theta)/theta Ebar'; Bbar^n = Bbar' (in place).
   const double theta = c.num.theta;
@@ -715,11 +734,13 @@ int tpic_mi_adjoint_cycle(tpic_mi_context* h, tpic_mi_adjoint* a, tpic_mi_solve_
   pc.dtx[2] = c.num.dt / g.dz;
   pc.inverse_volume = c.inverse_volume;
   pc.k = c.current_factor;
-  const unsigned cblocks = cell_blocks(c), nblocks = grid_for(c, nodes);
+  const unsigned nblocks = grid_for(c, nodes);
   for (size_t s = 0; s < c.species.size(); ++s) {
     if (c.species[s].count == 0) continue;
     SpeciesPass sp = species_pass(c, a->species[s], s);
-    k_adjoint_push<<<cblocks, kThreads, 0, c.stream>>>(g, sp, pc, c.bn, c.particle_field(), a->record);
+    const unsigned group = cell_group(c, sp.count), cblocks = cell_blocks(c, group);
+    const auto push = group == 64 ? k_adjoint_push<64> : (group == 32 ? k_adjoint_push<32> : k_adjoint_push<16>);
+    push<<<cblocks, kThreads, 0, c.stream>>>(g, sp, pc, c.bn, c.particle_field(), a->record);
     k_corner_sum<<<nblocks, kThreads, 0, c.stream>>>(g, a->record, a->ethetabar, 1);
     if ((rc = check_hip(c, hipGetLastError(), "adjoint push"))) return rc;
   }
@@ -745,7 +766,10 @@ int tpic_mi_adjoint_cycle(tpic_mi_context* h, tpic_mi_adjoint* a, tpic_mi_solve_
   for (size_t s = 0; s < c.species.size(); ++s) {
     if (c.species[s].count == 0) continue;
     SpeciesPass sp = species_pass(c, a->species[s], s);
-    k_adjoint_deposit<<<cblocks, kThreads, 0, c.stream>>>(g, sp, pc, c.bn, c.particle_field(), a->mu, a->record);
+    const unsigned group = cell_group(c, sp.count), cblocks = cell_blocks(c, group);
+    const auto deposit =
+        group == 64 ? k_adjoint_deposit<64> : (group == 32 ? k_adjoint_deposit<32> : k_adjoint_deposit<16>);
+    deposit<<<cblocks, kThreads, 0, c.stream>>>(g, sp, pc, c.bn, c.particle_field(), a->mu, a->record);
     k_corner_sum<<<nblocks, kThreads, 0, c.stream>>>(g, a->record, a->bnbar, first ? 0 : 1);
     if ((rc = check_hip(c, hipGetLastError(), "adjoint deposit"))) return rc;
     first = false;
@@ -754,7 +778,7 @@ int tpic_mi_adjoint_cycle(tpic_mi_context* h, tpic_mi_adjoint* a, tpic_mi_solve_
     k_c2n_transposed<<<grid_for(c, cells), kThreads, 0, c.stream>>>(g, a->bnbar, a->bbar);
     if ((rc = check_hip(c, hipGetLastError(), "adjoint cell to node"))) return rc;
   }
-  return check_hip(c, hipStreamSynchronize(c.stream), "adjoint cycle");
+  return 0;
 }
 
 int tpic_mi_adjoint_get_field(tpic_mi_adjoint* a, int which, double* host) {
@@ -784,11 +808,11 @@ int tpic_mi_adjoint_get_particles(tpic_mi_adjoint* a, int species, double* rbar,
   AdjointArrays& ad = a->species[size_t(species)];
   const size_t n = ad.count;
   int rc = 0;
-  if (n && rbar) rc = check_hip(c, hipMemcpyAsync(rbar, ad.rbar, 3 * n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
+  if (n && rbar) rc = check_hip(c, hipMemcpyAsync(rbar, ad.rbar(), 3 * n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
   if (!rc && n && vbar)
-    rc = check_hip(c, hipMemcpyAsync(vbar, ad.vbar, 3 * n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
-  if (!rc && n && qbar) rc = check_hip(c, hipMemcpyAsync(qbar, ad.qbar, n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
-  if (!rc && n && ids) rc = check_hip(c, hipMemcpyAsync(ids, ad.ids, n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
+    rc = check_hip(c, hipMemcpyAsync(vbar, ad.vbar(), 3 * n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
+  if (!rc && n && qbar) rc = check_hip(c, hipMemcpyAsync(qbar, ad.qbar(), n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
+  if (!rc && n && ids) rc = check_hip(c, hipMemcpyAsync(ids, ad.ids(), n * 8, hipMemcpyDeviceToHost, c.stream), "adjoint");
   if (!rc) rc = check_hip(c, hipStreamSynchronize(c.stream), "adjoint");
   return rc;
 }

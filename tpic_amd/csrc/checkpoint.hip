@@ -65,6 +65,68 @@ bool read_header(std::FILE* f, tpic_mi_checkpoint_header& hd) {
          std::fread(&version, 1, 4, f) == 4 && version == kVersion && std::fread(&hd, 1, sizeof hd, f) == sizeof hd;
 }
 
+// Every array of a list copied by one launch (blockIdx.y the array), 16 bytes
+// a thread and turn: as copies of their own, a save or restore of two species
+// was 22 launches.
+struct CopyList {
+  static constexpr unsigned kMost = 9 * kMaxSpecies + 4;
+  struct Item {
+    void* dst;
+    const void* src;
+    uint64_t bytes;  // a multiple of 4; both ends start 16-byte aligned (hipMalloc)
+  } item[kMost];
+  unsigned count = 0;
+  void add(void* dst, const void* src, size_t bytes) {
+    if (bytes) item[count++] = Item{dst, src, bytes};
+  }
+};
+
+constexpr unsigned kCopyThreads = 256;
+constexpr unsigned kCopyTurns = 4;  // 16-byte loads in flight per thread
+
+__global__ __launch_bounds__(kCopyThreads) void k_copy_list(CopyList list) {
+  const CopyList::Item& it = list.item[blockIdx.y];
+  const uint4* src = static_cast<const uint4*>(it.src);
+  uint4* dst = static_cast<uint4*>(it.dst);
+  const uint64_t words = it.bytes / 16;
+  const uint64_t step = uint64_t(gridDim.x) * kCopyThreads * kCopyTurns;
+  for (uint64_t base = uint64_t(blockIdx.x) * kCopyThreads * kCopyTurns + threadIdx.x; base < words; base += step) {
+    uint4 v[kCopyTurns];
+#pragma unroll
+    for (unsigned t = 0; t < kCopyTurns; ++t)
+      if (base + t * kCopyThreads < words) v[t] = src[base + t * kCopyThreads];
+#pragma unroll
+    for (unsigned t = 0; t < kCopyTurns; ++t)
+      if (base + t * kCopyThreads < words) dst[base + t * kCopyThreads] = v[t];
+  }
+  const unsigned rest = unsigned(it.bytes % 16) / 4;
+  if (blockIdx.x == 0 && threadIdx.x < rest)
+    reinterpret_cast<uint32_t*>(dst + words)[threadIdx.x] = reinterpret_cast<const uint32_t*>(src + words)[threadIdx.x];
+}
+
+int launch_copies(Context& c, const CopyList& list, const char* what) {
+  if (list.count == 0) return 0;
+  uint64_t most = 0;
+  for (unsigned i = 0; i < list.count; ++i) most = std::max(most, list.item[i].bytes);
+  const uint64_t per_block = 16ull * kCopyThreads * kCopyTurns;
+  const unsigned blocks = unsigned(std::max<uint64_t>(1, std::min<uint64_t>((most + per_block - 1) / per_block, 2048)));
+  k_copy_list<<<dim3(blocks, list.count), kCopyThreads, 0, c.stream>>>(list);
+  return check_hip(c, hipGetLastError(), what);
+}
+
+// A species' particle arrays.
+void add_particles(CopyList& list, const ParticleView& to, const ParticleView& from, size_t n) {
+  list.add(to.rx, from.rx, 8 * n);
+  list.add(to.ry, from.ry, 8 * n);
+  list.add(to.rz, from.rz, 8 * n);
+  list.add(to.u, from.u, 8 * n);
+  list.add(to.v, from.v, 8 * n);
+  list.add(to.w, from.w, 8 * n);
+  list.add(to.q, from.q, 8 * n);
+  list.add(to.cell, from.cell, 4 * n);
+  list.add(to.id, from.id, 8 * n);
+}
+
 }  // namespace
 
 void release_checkpoints(Context& c) {
@@ -128,24 +190,16 @@ int tpic_mi_checkpoint_save(tpic_mi_context* h, int slot) {
     return fail(c, TPIC_MI_INVALID_ARGUMENT, "checkpoint slot out of range (reserve slots first)");
   auto& cp = c.checkpoints[size_t(slot)];
   const size_t nodes = c.grid.nodes(), cells = c.grid.cells(), bins = c.grid.bins(), ns = c.species.size();
-  auto copy = [&](void* dst, const void* src, size_t bytes) {
-    return check_hip(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, c.stream), "checkpoint save");
-  };
-  int rc = 0;
-  for (size_t s = 0; s < ns && !rc; ++s) {
-    const ParticleView from = c.species[s].view();
-    const ParticleView& to = cp.particles[s];
-    const size_t n = c.species[s].count;
-    if ((rc = copy(to.rx, from.rx, 8 * n)) || (rc = copy(to.ry, from.ry, 8 * n)) || (rc = copy(to.rz, from.rz, 8 * n)) ||
-        (rc = copy(to.u, from.u, 8 * n)) || (rc = copy(to.v, from.v, 8 * n)) || (rc = copy(to.w, from.w, 8 * n)) ||
-        (rc = copy(to.q, from.q, 8 * n)) || (rc = copy(to.cell, from.cell, 4 * n)) || (rc = copy(to.id, from.id, 8 * n)))
-      break;
+  CopyList list;
+  for (size_t s = 0; s < ns; ++s) {
+    add_particles(list, cp.particles[s], c.species[s].view(), c.species[s].count);
     cp.sorted[s] = c.species[s].sorted;
   }
-  if (!rc) rc = copy(cp.counts, c.bin_counts, 4 * ns * bins);
-  if (!rc) rc = copy(cp.offsets, c.bin_offsets, 4 * ns * (bins + 1));
-  if (!rc) rc = copy(cp.e, c.e, 24 * nodes);
-  if (!rc) rc = copy(cp.b, c.b, 24 * cells);
+  list.add(cp.counts, c.bin_counts, 4 * ns * bins);
+  list.add(cp.offsets, c.bin_offsets, 4 * ns * (bins + 1));
+  list.add(cp.e, c.e, 24 * nodes);
+  list.add(cp.b, c.b, 24 * cells);
+  const int rc = launch_copies(c, list, "checkpoint save");
   if (!rc) cp.saved = true;
   return rc;
 }
@@ -157,24 +211,16 @@ int tpic_mi_checkpoint_restore(tpic_mi_context* h, int slot) {
     return fail(c, TPIC_MI_INVALID_ARGUMENT, "checkpoint slot out of range or never saved");
   auto& cp = c.checkpoints[size_t(slot)];
   const size_t nodes = c.grid.nodes(), cells = c.grid.cells(), bins = c.grid.bins(), ns = c.species.size();
-  auto copy = [&](void* dst, const void* src, size_t bytes) {
-    return check_hip(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, c.stream), "checkpoint restore");
-  };
-  int rc = 0;
-  for (size_t s = 0; s < ns && !rc; ++s) {
-    const ParticleView to = c.species[s].view();
-    const ParticleView& from = cp.particles[s];
-    const size_t n = c.species[s].count;
-    if ((rc = copy(to.rx, from.rx, 8 * n)) || (rc = copy(to.ry, from.ry, 8 * n)) || (rc = copy(to.rz, from.rz, 8 * n)) ||
-        (rc = copy(to.u, from.u, 8 * n)) || (rc = copy(to.v, from.v, 8 * n)) || (rc = copy(to.w, from.w, 8 * n)) ||
-        (rc = copy(to.q, from.q, 8 * n)) || (rc = copy(to.cell, from.cell, 4 * n)) || (rc = copy(to.id, from.id, 8 * n)))
-      break;
+  CopyList list;
+  for (size_t s = 0; s < ns; ++s) {
+    add_particles(list, c.species[s].view(), cp.particles[s], c.species[s].count);
     c.species[s].sorted = cp.sorted[s];
   }
-  if (!rc) rc = copy(c.bin_counts, cp.counts, 4 * ns * bins);
-  if (!rc) rc = copy(c.bin_offsets, cp.offsets, 4 * ns * (bins + 1));
-  if (!rc) rc = copy(c.e, cp.e, 24 * nodes);
-  if (!rc) rc = copy(c.b, cp.b, 24 * cells);
+  list.add(c.bin_counts, cp.counts, 4 * ns * bins);
+  list.add(c.bin_offsets, cp.offsets, 4 * ns * (bins + 1));
+  list.add(c.e, cp.e, 24 * nodes);
+  list.add(c.b, cp.b, 24 * cells);
+  int rc = launch_copies(c, list, "checkpoint restore");
   if (rc) return rc;
   return refresh(c);
 }
