@@ -1181,8 +1181,8 @@ def test_walled_solve_projects_a_field_set_after_startup(kind):
         ref.close()
 
 
-# Grids on both sides of the line between the operator's two forms (16384
-# nodes), with a part-filled last block, one-cell axes, walls and smoothing, and
+# Grids on both sides of the lines between the operator's forms (16384 and
+# 262144 nodes), with a part-filled last block, one-cell axes, walls and smoothing, and
 # restarts shorter than the solve.
 SOLVER_GRIDS = {
     "small": ((24, 24, 24), None, None, 30),
@@ -1194,6 +1194,7 @@ SOLVER_GRIDS = {
     "large_plane": ((40, 210, 1), None, None, 30),
     "large_walls": ((25, 26, 23), (1, R.FACE_PEC), None, 30),
     "large_smoothed": ((25, 26, 23), None, (R.SMOOTH_FACE7, 2, 0.5), 30),
+    "largest": ((66, 64, 61), None, None, 30),
 }
 
 
@@ -1212,7 +1213,8 @@ def test_operator_and_solve_on_both_forms(name):
     if wall:
         faces[wall[0]] = (wall[1],) * 2
         periodic[wall[0]] = 0
-    arrays = [random_state(cells, lengths, 2, rng, vscale=0.05)[1] for _ in qom]
+    per_cell = 1 if name == "largest" else 2
+    arrays = [random_state(cells, lengths, per_cell, rng, vscale=0.05)[1] for _ in qom]
     for a, q in zip(arrays, qom):
         a["q"] = np.full(len(a["q"]), (1.0 if q > 0 else -1.0) * 0.25 ** 3 / 2 / (4 * np.pi))
     counts = [len(a["q"]) for a in arrays]

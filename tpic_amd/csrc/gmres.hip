@@ -19,10 +19,11 @@
 // the orthogonalised image w_j with its factor s_j = 1 / |w_j| beside it (the
 // operator's image, the dots and the update take the factor), so no pass
 // normalises. The dots are formed by the operator's kernel where it can
-// (operator_tail_blocks), else by k_dot_batch, and the last block of
-// k_orthogonalize to finish adds the squared norm and runs the Givens update. A step is two launches on small
-// grids and four on large ones (seven before; 16^3: the solve's 10 operator
-// calls and 8 steps took 340 us of kernels).
+// (operator_tail_form: up to 262144 nodes), else by k_dot_batch, and the last
+// block of k_orthogonalize to finish adds the squared norm and runs the Givens
+// update. A step is two launches up to 16384 nodes, three (four with walls) up
+// to 262144 and four above, where it was seven (16^3: the solve's 10 operator
+// calls and 8 steps took 340 us of kernels, now 140).
 //
 // The reference's host reads two control scalars per step. Here the Givens
 // update tests them (the estimate against the tolerance, the breakdown) and
@@ -33,6 +34,7 @@
 //
 // Reductions are deterministic: fixed partials added in a fixed order.
 #include "internal.hpp"
+#include "arrival.hpp"
 
 #include <cmath>
 
@@ -43,11 +45,6 @@ constexpr unsigned kThreads = 256;
 constexpr unsigned kWaves = kThreads / 64;
 constexpr unsigned kTile = 4;
 constexpr int kMaxColumns = 64;  // tpic_mi_config.gmres_restart's limit
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;  // valid in lane 0
-}
 
 __device__ inline double block_reduce(double v, double* lds) {
   v = wave_sum(v);
@@ -101,44 +98,6 @@ SolverState solver_state(const GmresWorkspace& w, int m, double tolerance) {
   s.word = s.scale + (m + 1);
   s.tolerance = tolerance;
   return s;
-}
-
-// The last block of a launch to finish adds what the others left. Only
-// `partials` values and the arrival counters (zero between launches) pass
-// between blocks within a launch: both are agent-scope accesses, which go past
-// the XCDs' caches, and a block waits for its stores of partials before it
-// arrives. (An agent-scope release instead writes back the XCD's whole L2 for
-// every block: 33 us instead of 20 for an orthogonalisation at 100,000 nodes.)
-__device__ __forceinline__ void put_partial(double* at, double v) {
-  __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double get_partial(const double* at) {
-  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Counters of one launch's arrivals, in words: a root, then one per kGroup
-// blocks, each on a cache line of its own. Arrivals at one address follow one
-// another at about 20 ns (1024 blocks at one counter: 20 us), so a block
-// arrives at its group's and the last of a group at the root.
-constexpr unsigned kGroup = 32, kCounterStride = 32, kMaxBlocks = 1024;
-constexpr unsigned kCounters = (1 + kMaxBlocks / kGroup) * kCounterStride;
-
-__device__ __forceinline__ bool arrive(unsigned* counter, unsigned expected) {
-  if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != expected - 1) return false;
-  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return true;
-}
-
-// True in every thread of the last of `blocks` blocks to get here. Thread 0's
-// wave must have stored the block's partials itself.
-__device__ __forceinline__ bool last_to_arrive(unsigned* counters, unsigned block, unsigned blocks, bool* lds) {
-  if (threadIdx.x == 0) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const unsigned group = block / kGroup, begin = group * kGroup;
-    const unsigned size = blocks - begin < kGroup ? blocks - begin : kGroup;
-    *lds = arrive(counters + (1 + group) * kCounterStride, size) && arrive(counters, (blocks + kGroup - 1) / kGroup);
-  }
-  __syncthreads();
-  return *lds;
 }
 
 // Products of the image with the first `columns` basis vectors, kTile columns
@@ -427,7 +386,8 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
   const unsigned n = w.count;
   const int m = ctx.num.restart;
   const SolverState s = solver_state(w, m, ctx.num.gmres_tol);
-  const unsigned tail_blocks = operator_tail_blocks(ctx.grid);
+  const OperatorTailForm form = operator_tail_form(ctx.grid);
+  const unsigned tail_blocks = form.blocks;
   const unsigned rows = tail_blocks ? tail_blocks : w.blocks;  // partials per dot or norm
   double* const basis = w.basis;
   double* const norms = w.partials + size_t(std::max(m, 2)) * rows;
@@ -465,6 +425,8 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
       call.tail.basis = basis;
       call.tail.columns = unsigned(col + 1);
       call.tail.partials = w.partials;
+      call.tail.dots = dots;
+      call.tail.arrivals = w.arrivals + kCounters;
     }
     if (int e = launch_operator(ctx, basis + size_t(col) * n, w.image, call)) return e;
     if (!tail_blocks) {
@@ -474,7 +436,8 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
       if (int e = check_hip(ctx, hipGetLastError(), "gmres dots")) return e;
     }
     k_orthogonalize<<<w.blocks, kThreads, 0, st>>>(basis, w.image, basis + size_t(col + 1) * n,
-                                                   tail_blocks ? w.partials : dots, tail_blocks ? rows : 1u, norms,
+                                                   form.finishes_dots ? dots : w.partials,
+                                                   form.finishes_dots ? 1u : rows, norms,
                                                    w.arrivals, n, col, last ? 1 : 0, s, running);
     return check_hip(ctx, hipGetLastError(), "gmres orthogonalize");
   };

@@ -212,14 +212,17 @@ struct Guard {
   __device__ bool skips() const { return word && *word == skip; }
 };
 // What the solver wants of an operator image: products with `columns` basis
-// vectors of 3 nodes() values (kDots: row c of partials holds one value per
-// block), or rhs - image in its place with the blocks' parts of its squared
-// norm and of rhs's in rows 0 and 1 (kResidual).
+// vectors of 3 nodes() values (kDots), or rhs - image in its place with the
+// blocks' parts of its squared norm and of rhs's in rows 0 and 1 of partials
+// (kResidual). Row c of partials holds one value per block; forms that finish
+// the dots themselves write them to `dots`, with the counters of `arrivals`.
 struct OperatorTail {
   const double* basis = nullptr;
   unsigned columns = 0;
   const double* rhs = nullptr;
   double* partials = nullptr;
+  double* dots = nullptr;
+  unsigned* arrivals = nullptr;
 };
 enum class OperatorEpilogue : int { plain = 0, dots = 1, residual = 2 };
 struct OperatorCall {
@@ -229,9 +232,13 @@ struct OperatorCall {
   OperatorTail tail{};
 };
 // Blocks (values per row of partials) of an operator whose kernel takes the
-// epilogue, or 0 on grids whose kernel does not: the caller then works on
-// the plain image.
-unsigned operator_tail_blocks(const Grid& g);
+// epilogue, or 0 on grids too large for it: the caller then works on the plain
+// image. finishes_dots: whether it adds the dots' partials itself.
+struct OperatorTailForm {
+  unsigned blocks;
+  bool finishes_dots;
+};
+OperatorTailForm operator_tail_form(const Grid& g);
 int launch_operator(Context& ctx, const double* in, double* out, const OperatorCall& call = {});
 // The configured smoothing S(src) of a node vector (ctx.num.smoothing must be
 // set; constrained rows of src read as zero, those of every pass zeroed): the

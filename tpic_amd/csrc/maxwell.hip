@@ -17,6 +17,7 @@
 // the entry-major matrix (coalesced: neighbouring nodes read neighbouring
 // words) and the three-term combination. Bound: HBM, 1008 B of matrix per node.
 #include "internal.hpp"
+#include "arrival.hpp"
 #include "../../include/tpic_mi.h"
 
 namespace tpic_mi {
@@ -468,20 +469,33 @@ __device__ __forceinline__ void mass_rows(const Grid& g, const double* __restric
 // smoothed response (combine_image, maxwell_device.hpp:419-433).
 constexpr int kFused = 0, kMassResponse = 1, kCombine = 2;
 
-template <class MassT, bool Walls, int Stage = kFused, bool Transposed = false>
+// What a kernel does with the image in its registers (OperatorTail).
+constexpr int kPlain = 0, kDots = 1, kResidual = 2;
+
+// A node per thread. With an epilogue (grids of at most kMaxBlocks blocks) a
+// block goes on to what the solver reads the image for: kDots forms its
+// products with `columns` basis vectors, the last block to arrive adding the
+// blocks' parts, and kResidual writes rhs - image instead of the image and the
+// block's parts of its squared norm and of rhs's. As a launch of their own
+// the dots took 12 us at 100,000 nodes, the residual 5.
+template <class MassT, bool Walls, int Stage, bool Transposed, int Epilogue>
 __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __restrict__ v,
                                                     const double* __restrict__ curl_cells,
                                                     const MassT* __restrict__ mass,
                                                     const double* __restrict__ response, double d2, double k,
                                                     double inverse_volume, double* __restrict__ out,
                                                     unsigned tile_rows, const double* __restrict__ scale,
-                                                    Guard guard) {
+                                                    OperatorTail tail, Guard guard) {
   // A launch of a GMRES step after the solver stopped does nothing.
   if (guard.skips()) return;
   const unsigned nodes = g.nodes();
   const unsigned sx = unsigned(g.nx + 1), sy = unsigned(g.ny + 1), sz = unsigned(g.nz + 1);
-  const unsigned L = xcd_logical_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (L >= nodes) return;
+  unsigned L = xcd_logical_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const bool present = L < nodes;
+  if (!present) {
+    if (Epilogue == kPlain) return;
+    L = nodes - 1;  // the lane goes along to the block's sums
+  }
   // Traversal: full x rows, grouped into tiles of tile_rows rows; a tile's
   // planes are visited in z order, so the blocks of the planes k - 1 and k of
   // a tile are close in time (within one XCD) and the backward reads of the
@@ -534,9 +548,54 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
     oy *= by;
     oz *= by;
   }
-  out[n] = ox;
-  out[nodes + n] = oy;
-  out[2 * size_t(nodes) + n] = oz;
+  if constexpr (Epilogue == kResidual) {
+    __shared__ double s_norm[kThreads / 64][2];
+    const double bx = tail.rhs[n], by = tail.rhs[nodes + n], bz = tail.rhs[2 * size_t(nodes) + n];
+    ox = bx - ox;
+    oy = by - oy;
+    oz = bz - oz;
+    const double r2 = wave_sum(present ? ox * ox + oy * oy + oz * oz : 0.0);
+    const double b2 = wave_sum(present ? bx * bx + by * by + bz * bz : 0.0);
+    if ((threadIdx.x & 63u) == 0) {
+      s_norm[threadIdx.x >> 6][0] = r2;
+      s_norm[threadIdx.x >> 6][1] = b2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      double total = 0.0;
+      for (unsigned w = 0; w < kThreads / 64; ++w) total += s_norm[w][threadIdx.x];
+      tail.partials[size_t(threadIdx.x) * gridDim.x + blockIdx.x] = total;
+    }
+  }
+  if (present) {
+    out[n] = ox;
+    out[nodes + n] = oy;
+    out[2 * size_t(nodes) + n] = oz;
+  }
+  if constexpr (Epilogue == kDots) {
+    __shared__ double s_dot[kThreads / 64][64];
+    __shared__ bool s_last;
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    for (unsigned col = 0; col < tail.columns; ++col) {
+      const double* w = tail.basis + 3 * size_t(col) * nodes + n;
+      const double total = wave_sum(present ? w[0] * ox + w[nodes] * oy + w[2 * size_t(nodes)] * oz : 0.0);
+      if (lane == 0) s_dot[wave][col] = total;
+    }
+    __syncthreads();
+    // Wave 0 stores the block's partials (at most 64 columns).
+    if (threadIdx.x < tail.columns) {
+      double total = 0.0;
+      for (unsigned w = 0; w < kThreads / 64; ++w) total += s_dot[w][threadIdx.x];
+      put_partial(tail.partials + size_t(threadIdx.x) * gridDim.x + blockIdx.x, total);
+    }
+    if (!last_to_arrive(tail.arrivals, blockIdx.x, gridDim.x, &s_last)) return;
+    for (unsigned col = wave; col < tail.columns; col += kThreads / 64) {
+      double total = 0.0;
+      for (unsigned b = lane; b < gridDim.x; b += 64) total += get_partial(tail.partials + size_t(col) * gridDim.x + b);
+      total = wave_sum(total);
+      if (lane == 0) tail.dots[col] = total;
+    }
+  }
 }
 
 // The operator on a grid too small to fill the chip with a thread per node:
@@ -547,11 +606,6 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
 // and the eight parts meet in LDS. At 16^3 a thread per node leaves 20 blocks,
 // whose lanes wait for their 27 x 12 loads in many turns: 14.6 us, and 3.6 us
 // for the curl pass before it.
-// With the image in registers the block goes on to what the solver reads it
-// for: Epilogue kDots forms the block's part of the image's products with
-// `columns` basis vectors, kResidual writes rhs - image instead of the image
-// and the block's parts of its squared norm and of rhs's.
-constexpr int kPlain = 0, kDots = 1, kResidual = 2;
 constexpr unsigned kParts = 8;
 
 // One cell's part of curl_C2N(curl_N2C v) at node (i, j, k): the cell at
@@ -607,12 +661,6 @@ __device__ __forceinline__ void operator_share(const Grid& g, const double* __re
     for (int c = 0; c < 3; ++c) sum[c] = f * m[c];
   }
   if constexpr (Stage != kMassResponse) cell.add(g, d2, sum);
-}
-
-// Sum over the wave, in lane 0.
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
 }
 
 template <class MassT, bool Walls, int Stage, bool Transposed, int Epilogue>
@@ -855,12 +903,25 @@ unsigned apply_tile_rows(const Grid& g) {
   return std::min({kApplyTileRows, fit, unsigned(g.ny + 1)});
 }
 
-template <class MassT, bool Walls, int Stage, bool Transposed = false>
-void node_stage(const OperatorArgs& a, const double* in, const double* curl, const MassT* mass,
-                const double* response, double* out) {
+template <class MassT, bool Walls, int Stage, bool Transposed, int Epilogue>
+void node_kernel(const OperatorArgs& a, const double* in, const double* curl, const MassT* mass,
+                 const double* response, double* out) {
   const unsigned rows = apply_tile_rows<MassT>(a.g);
-  k_apply<MassT, Walls, Stage, Transposed><<<(a.g.nodes() + kThreads - 1) / kThreads, kThreads, 0, a.stream>>>(
-      a.g, in, curl, mass, response, a.d2, a.k, a.inverse_volume, out, rows, a.scale, a.guard);
+  k_apply<MassT, Walls, Stage, Transposed, Epilogue>
+      <<<(a.g.nodes() + kThreads - 1) / kThreads, kThreads, 0, a.stream>>>(
+          a.g, in, curl, mass, response, a.d2, a.k, a.inverse_volume, out, rows, a.scale, a.tail, a.guard);
+}
+
+template <class MassT, bool Walls, int Stage, bool Transposed = false>
+void node_stage(const OperatorArgs& a, int epilogue, const double* in, const double* curl, const MassT* mass,
+                const double* response, double* out) {
+  if constexpr (Stage != kMassResponse) {
+    if (epilogue == kDots)
+      return node_kernel<MassT, Walls, Stage, Transposed, kDots>(a, in, curl, mass, response, out);
+    if (epilogue == kResidual)
+      return node_kernel<MassT, Walls, Stage, Transposed, kResidual>(a, in, curl, mass, response, out);
+  }
+  node_kernel<MassT, Walls, Stage, Transposed, kPlain>(a, in, curl, mass, response, out);
 }
 
 // image = A in by either form. Walls and smoothing take the mass response by
@@ -883,7 +944,7 @@ int operator_image(Context& ctx, const OperatorArgs& a, bool split, int epilogue
     if (split)
       split_stage<MassT, Walls, kMassResponse, false>(plain, kPlain, x, mass, nullptr, r);
     else
-      node_stage<MassT, Walls, kMassResponse>(plain, x, nullptr, mass, nullptr, r);
+      node_stage<MassT, Walls, kMassResponse>(plain, kPlain, x, nullptr, mass, nullptr, r);
     if (int rc = check_hip(ctx, hipGetLastError(), "mass response")) return rc;
     if (int rc = launch_smooth(ctx, r, nullptr, &response, a.guard)) return rc;
   } else if (Walls && !split) {
@@ -891,19 +952,19 @@ int operator_image(Context& ctx, const OperatorArgs& a, bool split, int epilogue
       return fail(ctx, TPIC_MI_INVALID_STATE, "walled operator without its mass response buffer");
     OperatorArgs plain = a;
     plain.scale = nullptr;
-    node_stage<MassT, Walls, kMassResponse>(plain, in, nullptr, mass, nullptr, ctx.mass_response);
+    node_stage<MassT, Walls, kMassResponse>(plain, kPlain, in, nullptr, mass, nullptr, ctx.mass_response);
     if (int rc = check_hip(ctx, hipGetLastError(), "walled mass response")) return rc;
   } else {
     if (split)
       split_stage<MassT, Walls, kFused, false>(a, epilogue, in, mass, nullptr, out);
     else if constexpr (!Walls)
-      node_stage<MassT, Walls, kFused>(a, in, curl, mass, nullptr, out);
+      node_stage<MassT, Walls, kFused>(a, epilogue, in, curl, mass, nullptr, out);
     return check_hip(ctx, hipGetLastError(), "operator apply");
   }
   if (split)
     split_stage<double, Walls, kCombine, false>(a, epilogue, in, nullptr, response, out);
   else
-    node_stage<double, Walls, kCombine>(a, in, curl, nullptr, response, out);
+    node_stage<double, Walls, kCombine>(a, epilogue, in, curl, nullptr, response, out);
   return check_hip(ctx, hipGetLastError(), "operator combination");
 }
 
@@ -915,20 +976,24 @@ int transposed_image(Context& ctx, const OperatorArgs& a, bool split, int epilog
   if (split)
     split_stage<MassT, false, kFused, true>(a, epilogue, in, mass, nullptr, out);
   else
-    node_stage<MassT, false, kFused, true>(a, in, ctx.gmres.curl_cells, mass, nullptr, out);
+    node_stage<MassT, false, kFused, true>(a, epilogue, in, ctx.gmres.curl_cells, mass, nullptr, out);
   return check_hip(ctx, hipGetLastError(), "transposed operator apply");
 }
 
 }  // namespace
 
-unsigned operator_tail_blocks(const Grid& g) { return g.nodes() <= kSplitNodes ? (g.nodes() + 63u) / 64u : 0u; }
+OperatorTailForm operator_tail_form(const Grid& g) {
+  if (g.nodes() <= kSplitNodes) return {(g.nodes() + 63u) / 64u, false};
+  const unsigned blocks = (g.nodes() + kThreads - 1) / kThreads;
+  return blocks <= kMaxBlocks ? OperatorTailForm{blocks, true} : OperatorTailForm{0, true};
+}
 
 int launch_operator(Context& ctx, const double* in, double* out, const OperatorCall& call) {
   const Grid& g = ctx.grid;
-  const bool split = operator_tail_blocks(g) != 0;
+  const bool split = g.nodes() <= kSplitNodes;
   const OperatorArgs a{g, ctx.stream, ctx.delta * ctx.delta, ctx.current_factor, ctx.inverse_volume, call.scale,
                        call.guard, call.tail};
-  const int epilogue = split ? int(call.epilogue) : kPlain;
+  const int epilogue = int(call.epilogue);
   phase_begin(ctx, Phase::spmv);
   int rc = 0;
   if (!split) {
