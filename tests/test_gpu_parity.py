@@ -1194,7 +1194,10 @@ SOLVER_GRIDS = {
     "large_plane": ((40, 210, 1), None, None, 30),
     "large_walls": ((25, 26, 23), (1, R.FACE_PEC), None, 30),
     "large_smoothed": ((25, 26, 23), None, (R.SMOOTH_FACE7, 2, 0.5), 30),
-    "largest": ((66, 64, 61), None, None, 30),
+    "large_one_cell_walled_plane": ((30, 320, 1), (1, R.FACE_PEC), None, 30),
+    "large_plane_restarted": ((150, 60, 1), None, None, 4),
+    "largest_fused": ((66, 64, 61), None, None, 30),
+    "largest": ((84, 80, 79), None, None, 30),
 }
 
 
@@ -1213,7 +1216,7 @@ def test_operator_and_solve_on_both_forms(name):
     if wall:
         faces[wall[0]] = (wall[1],) * 2
         periodic[wall[0]] = 0
-    per_cell = 1 if name == "largest" else 2
+    per_cell = 1 if name.startswith("largest") else 2
     arrays = [random_state(cells, lengths, per_cell, rng, vscale=0.05)[1] for _ in qom]
     for a, q in zip(arrays, qom):
         a["q"] = np.full(len(a["q"]), (1.0 if q > 0 else -1.0) * 0.25 ** 3 / 2 / (4 * np.pi))

@@ -28,7 +28,7 @@ __device__ __forceinline__ double get_partial(const double* at) {
 // blocks, each on a cache line of its own. Arrivals at one address follow one
 // another at about 20 ns (1024 blocks at one counter: 20 us), so a block
 // arrives at its group's and the last of a group at the root.
-constexpr unsigned kGroup = 32, kCounterStride = 32, kMaxBlocks = 1024;
+constexpr unsigned kGroup = 32, kCounterStride = 32, kMaxBlocks = 2048;
 constexpr unsigned kCounters = (1 + kMaxBlocks / kGroup) * kCounterStride;
 
 __device__ __forceinline__ bool arrive(unsigned* counter, unsigned expected) {

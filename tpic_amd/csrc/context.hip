@@ -266,7 +266,7 @@ int allocate(tpic_mi_context* h) {
   TPIC_ALLOC(gm.basis, (m + 1) * gm.count);
   TPIC_ALLOC(gm.x, gm.count);
   TPIC_ALLOC(gm.image, gm.count);
-  TPIC_ALLOC(gm.partials, gmres_partial_words(c.num.restart, gm.blocks, operator_tail_form(g).blocks));
+  TPIC_ALLOC(gm.partials, gmres_partial_words(c.num.restart, gm.blocks, operator_tail_form(c).blocks));
   TPIC_ALLOC(gm.state, gmres_state_words(c.num.restart));
   TPIC_ALLOC(gm.arrivals, gmres_arrival_words(c.num.restart));
   TPIC_ALLOC(gm.curl_cells, 3 * cells);

@@ -19,10 +19,11 @@
 // the orthogonalised image w_j with its factor s_j = 1 / |w_j| beside it (the
 // operator's image, the dots and the update take the factor), so no pass
 // normalises. The dots are formed by the operator's kernel where it can
-// (operator_tail_form: up to 262144 nodes), else by k_dot_batch, and the last
+// (operator_tail_form: up to 2048 blocks of 256 nodes, or of 256 columns of a
+// plane), else by k_dot_batch, and the last
 // block of k_orthogonalize to finish adds the squared norm and runs the Givens
 // update. A step is two launches up to 16384 nodes, three (four with walls) up
-// to 262144 and four above, where it was seven (16^3: the solve's 10 operator
+// to 524288 nodes and four above, where it was seven (16^3: the solve's 10 operator
 // calls and 8 steps took 340 us of kernels, now 140).
 //
 // The reference's host reads two control scalars per step. Here the Givens
@@ -44,6 +45,8 @@ namespace {
 constexpr unsigned kThreads = 256;
 constexpr unsigned kWaves = kThreads / 64;
 constexpr unsigned kTile = 4;
+constexpr unsigned kReduceBlocks = 1024;
+static_assert(kReduceBlocks <= kMaxBlocks);
 constexpr int kMaxColumns = 64;  // tpic_mi_config.gmres_restart's limit
 
 __device__ inline double block_reduce(double v, double* lds) {
@@ -361,10 +364,11 @@ __global__ __launch_bounds__(kThreads) void k_commit(const double* __restrict__ 
 }  // namespace
 
 // Words of GmresWorkspace::arrivals: the orthogonalisation's counters, then
-// those of each row of k_dot_batch's blocks; and the blocks of both.
+// those of each row of k_dot_batch's blocks.
 size_t gmres_arrival_words(int m) { return (1 + size_t(m + kTile - 1) / kTile) * kCounters; }
+// Blocks of both: more than four per CU only lengthen the last block's sum.
 unsigned gmres_blocks(unsigned count, int cus) {
-  return std::max(1u, std::min({(count + kThreads - 1) / kThreads, unsigned(cus > 0 ? cus : 256) * 4, kMaxBlocks}));
+  return std::max(1u, std::min({(count + kThreads - 1) / kThreads, unsigned(cus > 0 ? cus : 256) * 4, kReduceBlocks}));
 }
 // Doubles of GmresWorkspace::partials: dots per block, norms per block, dots.
 size_t gmres_partial_words(int m, unsigned blocks, unsigned tail_blocks) {
@@ -386,7 +390,7 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
   const unsigned n = w.count;
   const int m = ctx.num.restart;
   const SolverState s = solver_state(w, m, ctx.num.gmres_tol);
-  const OperatorTailForm form = operator_tail_form(ctx.grid);
+  const OperatorTailForm form = operator_tail_form(ctx);
   const unsigned tail_blocks = form.blocks;
   const unsigned rows = tail_blocks ? tail_blocks : w.blocks;  // partials per dot or norm
   double* const basis = w.basis;

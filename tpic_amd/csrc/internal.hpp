@@ -238,7 +238,7 @@ struct OperatorTailForm {
   unsigned blocks;
   bool finishes_dots;
 };
-OperatorTailForm operator_tail_form(const Grid& g);
+OperatorTailForm operator_tail_form(const Context& ctx);
 int launch_operator(Context& ctx, const double* in, double* out, const OperatorCall& call = {});
 // The configured smoothing S(src) of a node vector (ctx.num.smoothing must be
 // set; constrained rows of src read as zero, those of every pass zeroed): the

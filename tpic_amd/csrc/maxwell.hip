@@ -472,6 +472,75 @@ constexpr int kFused = 0, kMassResponse = 1, kCombine = 2;
 // What a kernel does with the image in its registers (OperatorTail).
 constexpr int kPlain = 0, kDots = 1, kResidual = 2;
 
+// The end of an operator kernel whose threads hold the images of N nodes each:
+// stores them, or what `Epilogue` makes of them. Every thread of the block
+// comes along; one that is not `present` holds a copy of another's nodes.
+template <int Epilogue, int N>
+__device__ __forceinline__ void finish_image(const double (&image)[N][3], const unsigned (&at)[N], bool present,
+                                             unsigned nodes, double* __restrict__ out, const OperatorTail& tail) {
+  if constexpr (Epilogue == kResidual) {
+    __shared__ double s_norm[kThreads / 64][2];
+    double r2 = 0.0, b2 = 0.0;
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const size_t n = size_t(c) * nodes + at[t];
+        const double b = tail.rhs[n], r = b - image[t][c];
+        if (present) out[n] = r;
+        r2 += r * r;
+        b2 += b * b;
+      }
+    r2 = wave_sum(present ? r2 : 0.0);
+    b2 = wave_sum(present ? b2 : 0.0);
+    if ((threadIdx.x & 63u) == 0) {
+      s_norm[threadIdx.x >> 6][0] = r2;
+      s_norm[threadIdx.x >> 6][1] = b2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      double total = 0.0;
+      for (unsigned w = 0; w < kThreads / 64; ++w) total += s_norm[w][threadIdx.x];
+      tail.partials[size_t(threadIdx.x) * gridDim.x + blockIdx.x] = total;
+    }
+  } else {
+    if (present)
+#pragma unroll
+      for (int t = 0; t < N; ++t)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) out[size_t(c) * nodes + at[t]] = image[t][c];
+  }
+  if constexpr (Epilogue == kDots) {
+    __shared__ double s_dot[kThreads / 64][64];
+    __shared__ bool s_last;
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    for (unsigned col = 0; col < tail.columns; ++col) {
+      const double* w = tail.basis + 3 * size_t(col) * nodes;
+      double v = 0.0;
+#pragma unroll
+      for (int t = 0; t < N; ++t)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) v += w[size_t(c) * nodes + at[t]] * image[t][c];
+      v = wave_sum(present ? v : 0.0);
+      if (lane == 0) s_dot[wave][col] = v;
+    }
+    __syncthreads();
+    // Wave 0 stores the block's partials (at most 64 columns).
+    if (threadIdx.x < tail.columns) {
+      double total = 0.0;
+      for (unsigned w = 0; w < kThreads / 64; ++w) total += s_dot[w][threadIdx.x];
+      put_partial(tail.partials + size_t(threadIdx.x) * gridDim.x + blockIdx.x, total);
+    }
+    if (!last_to_arrive(tail.arrivals, blockIdx.x, gridDim.x, &s_last)) return;
+    for (unsigned col = wave; col < tail.columns; col += kThreads / 64) {
+      double total = 0.0;
+      for (unsigned b = lane; b < gridDim.x; b += 64) total += get_partial(tail.partials + size_t(col) * gridDim.x + b);
+      total = wave_sum(total);
+      if (lane == 0) tail.dots[col] = total;
+    }
+  }
+}
+
 // A node per thread. With an epilogue (grids of at most kMaxBlocks blocks) a
 // block goes on to what the solver reads the image for: kDots forms its
 // products with `columns` basis vectors, the last block to arrive adding the
@@ -548,54 +617,110 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
     oy *= by;
     oz *= by;
   }
-  if constexpr (Epilogue == kResidual) {
-    __shared__ double s_norm[kThreads / 64][2];
-    const double bx = tail.rhs[n], by = tail.rhs[nodes + n], bz = tail.rhs[2 * size_t(nodes) + n];
-    ox = bx - ox;
-    oy = by - oy;
-    oz = bz - oz;
-    const double r2 = wave_sum(present ? ox * ox + oy * oy + oz * oz : 0.0);
-    const double b2 = wave_sum(present ? bx * bx + by * by + bz * bz : 0.0);
-    if ((threadIdx.x & 63u) == 0) {
-      s_norm[threadIdx.x >> 6][0] = r2;
-      s_norm[threadIdx.x >> 6][1] = b2;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-      double total = 0.0;
-      for (unsigned w = 0; w < kThreads / 64; ++w) total += s_norm[w][threadIdx.x];
-      tail.partials[size_t(threadIdx.x) * gridDim.x + blockIdx.x] = total;
-    }
+  const double image[1][3] = {{ox, oy, oz}};
+  const unsigned at[1] = {n};
+  finish_image<Epilogue>(image, at, present, nodes, out, tail);
+}
+
+// The operator of a plane, one periodic cell deep (nz = 1, periodic fields): a
+// thread takes both of a column's nodes. They read the same matrix blocks and
+// the same four cells, and the same neighbours in the blocks with a z offset
+// (-1 is node 0, +1 node 1 for both), so a pair costs little more than a
+// node: 18 of the 27 products and the curl term are shared. 512 x 512 x 1 in
+// FP64 reads 267 MB of blocks in 90 us where a thread per node took 126 (55 us
+// at the rate of a copy); 52000 columns' waves fill the chip, and below 16384
+// nodes k_apply_split keeps its eight waves per 64 nodes.
+template <class MassT, bool Transposed>
+__device__ __forceinline__ void add_block(const MassT (&b)[9], const double (&a)[3], double (&m)[3]) {
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+    m[r] += a[0] * double(b[Transposed ? r : 3 * r]) + a[1] * double(b[Transposed ? 3 + r : 3 * r + 1]) +
+            a[2] * double(b[Transposed ? 6 + r : 3 * r + 2]);
+}
+
+// The stencil whose forward (ahead) or backward block couples a node to its
+// neighbour at (x, y, z).
+struct BlockOf {
+  int stencil;
+  bool ahead;
+};
+constexpr BlockOf block_of(int x, int y, int z) {
+  for (int s = 0; s < kStencils; ++s) {
+    if (c_offsets[s][0] == x && c_offsets[s][1] == y && c_offsets[s][2] == z) return {s, true};
+    if (c_offsets[s][0] == -x && c_offsets[s][1] == -y && c_offsets[s][2] == -z) return {s, false};
   }
-  if (present) {
-    out[n] = ox;
-    out[nodes + n] = oy;
-    out[2 * size_t(nodes) + n] = oz;
+  return {0, true};
+}
+
+template <class MassT, int X, int Y, int Z>
+__device__ __forceinline__ void load_plane_block(const Grid& g, const MassT* __restrict__ mass, const VertexWalk& w,
+                                                 MassT (&b)[9]) {
+  constexpr BlockOf of = block_of(X, Y, Z);
+  const MassT* rows = mass + size_t(of.stencil) * 9 * g.vstride + (of.ahead ? w.v0 : w.v0 + X * w.sx + Y * w.sy);
+#pragma unroll
+  for (int e = 0; e < 9; ++e) b[e] = rows[size_t(e) * g.vstride];
+}
+
+// The three blocks of the neighbouring column at (X, Y), then the others of a
+// 3 x 3 patch: the column's two values are loaded once for all three.
+template <class MassT, bool Transposed, int Position>
+__device__ __forceinline__ void plane_columns(const Grid& g, const double* __restrict__ v,
+                                              const MassT* __restrict__ mass, const NodeImages& im,
+                                              const VertexWalk& w, double (&shared)[3], double (&own)[2][3]) {
+  constexpr int X = Position % 3 - 1, Y = Position / 3 - 1;
+  const unsigned nodes = g.nodes(), upper = unsigned(g.nx + 1) * unsigned(g.ny + 1);
+  const unsigned node = unsigned(im.x[1 + X]) + unsigned(g.nx + 1) * unsigned(im.y[1 + Y]);
+  MassT below[9], level[9], above[9];
+  load_plane_block<MassT, X, Y, -1>(g, mass, w, below);
+  load_plane_block<MassT, X, Y, 0>(g, mass, w, level);
+  load_plane_block<MassT, X, Y, 1>(g, mass, w, above);
+  double a[2][3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    a[0][c] = v[size_t(c) * nodes + node];
+    a[1][c] = v[size_t(c) * nodes + node + upper];
   }
-  if constexpr (Epilogue == kDots) {
-    __shared__ double s_dot[kThreads / 64][64];
-    __shared__ bool s_last;
-    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    for (unsigned col = 0; col < tail.columns; ++col) {
-      const double* w = tail.basis + 3 * size_t(col) * nodes + n;
-      const double total = wave_sum(present ? w[0] * ox + w[nodes] * oy + w[2 * size_t(nodes)] * oz : 0.0);
-      if (lane == 0) s_dot[wave][col] = total;
-    }
-    __syncthreads();
-    // Wave 0 stores the block's partials (at most 64 columns).
-    if (threadIdx.x < tail.columns) {
-      double total = 0.0;
-      for (unsigned w = 0; w < kThreads / 64; ++w) total += s_dot[w][threadIdx.x];
-      put_partial(tail.partials + size_t(threadIdx.x) * gridDim.x + blockIdx.x, total);
-    }
-    if (!last_to_arrive(tail.arrivals, blockIdx.x, gridDim.x, &s_last)) return;
-    for (unsigned col = wave; col < tail.columns; col += kThreads / 64) {
-      double total = 0.0;
-      for (unsigned b = lane; b < gridDim.x; b += 64) total += get_partial(tail.partials + size_t(col) * gridDim.x + b);
-      total = wave_sum(total);
-      if (lane == 0) tail.dots[col] = total;
-    }
+  add_block<MassT, Transposed>(below, a[0], shared);
+  add_block<MassT, Transposed>(above, a[1], shared);
+  add_block<MassT, Transposed>(level, a[0], own[0]);
+  add_block<MassT, Transposed>(level, a[1], own[1]);
+  // The sums are formed here: left to the compiler they sink past the next
+  // columns' loads (256 registers and a wave per SIMD, here about 90 and five).
+#pragma unroll
+  for (int c = 0; c < 3; ++c) asm volatile("" : "+v"(shared[c]), "+v"(own[0][c]), "+v"(own[1][c]) : : "memory");
+  if constexpr (Position < 8) plane_columns<MassT, Transposed, Position + 1>(g, v, mass, im, w, shared, own);
+}
+
+template <class MassT, bool Transposed, int Epilogue>
+__global__ __launch_bounds__(kThreads) void k_apply_plane(Grid g, const double* __restrict__ v,
+                                                          const double* __restrict__ curl_cells,
+                                                          const MassT* __restrict__ mass, double d2, double k,
+                                                          double inverse_volume, double* __restrict__ out,
+                                                          const double* __restrict__ scale, OperatorTail tail,
+                                                          Guard guard) {
+  if (guard.skips()) return;
+  const unsigned sx = unsigned(g.nx + 1), columns = sx * unsigned(g.ny + 1), nodes = g.nodes();
+  unsigned n = xcd_logical_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const bool present = n < columns;
+  if (!present) {
+    if (Epilogue == kPlain) return;
+    n = columns - 1;
   }
+  const int i = int(n % sx), j = int(n / sx);
+  const NodeImages im = node_images<false>(g, i, j, 0);
+  double shared[3] = {0.0, 0.0, 0.0}, own[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+  plane_columns<MassT, Transposed, 0>(g, v, mass, im, vertex_walk(g, i, j, 0), shared, own);
+  double cc[3];
+  c2n_at<false>(g, curl_cells, i, j, 0, cc[0], cc[1], cc[2]);
+  const double by = scale ? *scale : 1.0;
+  const unsigned at[2] = {n, n + columns};
+  double image[2][3];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      image[t][c] = (v[size_t(c) * nodes + at[t]] + d2 * cc[c] + k * (inverse_volume * (shared[c] + own[t][c]))) * by;
+  finish_image<Epilogue>(image, at, present, nodes, out, tail);
 }
 
 // The operator on a grid too small to fill the chip with a thread per node:
@@ -912,9 +1037,31 @@ void node_kernel(const OperatorArgs& a, const double* in, const double* curl, co
           a.g, in, curl, mass, response, a.d2, a.k, a.inverse_volume, out, rows, a.scale, a.tail, a.guard);
 }
 
+// Grids whose thread takes a column's two nodes.
+bool plane_form(const Grid& g) { return g.nz == 1 && !g.walls; }
+
+// Threads of the forms that take whole nodes or columns.
+unsigned node_threads(const Grid& g, bool plane) {
+  return plane ? unsigned(g.nx + 1) * unsigned(g.ny + 1) : g.nodes();
+}
+
+template <class MassT, bool Transposed, int Epilogue>
+void plane_kernel(const OperatorArgs& a, const double* in, const double* curl, const MassT* mass, double* out) {
+  k_apply_plane<MassT, Transposed, Epilogue>
+      <<<(node_threads(a.g, true) + kThreads - 1) / kThreads, kThreads, 0, a.stream>>>(
+          a.g, in, curl, mass, a.d2, a.k, a.inverse_volume, out, a.scale, a.tail, a.guard);
+}
+
 template <class MassT, bool Walls, int Stage, bool Transposed = false>
 void node_stage(const OperatorArgs& a, int epilogue, const double* in, const double* curl, const MassT* mass,
                 const double* response, double* out) {
+  if constexpr (Stage == kFused && !Walls) {
+    if (plane_form(a.g)) {
+      if (epilogue == kDots) return plane_kernel<MassT, Transposed, kDots>(a, in, curl, mass, out);
+      if (epilogue == kResidual) return plane_kernel<MassT, Transposed, kResidual>(a, in, curl, mass, out);
+      return plane_kernel<MassT, Transposed, kPlain>(a, in, curl, mass, out);
+    }
+  }
   if constexpr (Stage != kMassResponse) {
     if (epilogue == kDots)
       return node_kernel<MassT, Walls, Stage, Transposed, kDots>(a, in, curl, mass, response, out);
@@ -982,9 +1129,11 @@ int transposed_image(Context& ctx, const OperatorArgs& a, bool split, int epilog
 
 }  // namespace
 
-OperatorTailForm operator_tail_form(const Grid& g) {
+OperatorTailForm operator_tail_form(const Context& ctx) {
+  const Grid& g = ctx.grid;
   if (g.nodes() <= kSplitNodes) return {(g.nodes() + 63u) / 64u, false};
-  const unsigned blocks = (g.nodes() + kThreads - 1) / kThreads;
+  const bool plane = plane_form(g) && !ctx.num.smoothing;
+  const unsigned blocks = (node_threads(g, plane) + kThreads - 1) / kThreads;
   return blocks <= kMaxBlocks ? OperatorTailForm{blocks, true} : OperatorTailForm{0, true};
 }
 
