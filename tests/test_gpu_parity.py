@@ -528,6 +528,39 @@ def test_deposition_thin_axes_and_empty_cells():
     assert np.abs(j - cur).max() <= 3e-12 * np.abs(cur).max() + 1e-15
 
 
+@pytest.mark.parametrize("cells,wall", [((70, 9, 1), None), ((64, 5, 1), 0), ((13, 17, 1), 1), ((12, 5, 2), 2)])
+def test_assembly_of_planes(cells, wall):
+    """The mass matrix of shallow grids, every stored vertex plane,
+    against the oracle's (3e-12 of its largest entry, as
+    tests/ecsim/sorted_mass_device.cpp:359-367), with the last strip of a
+    tile partly filled; the planes of a one-cell z axis are equal bit for bit."""
+    lengths = tuple(0.25 * n for n in cells)
+    rng = np.random.default_rng(41)
+    faces, periodic = [(R.FACE_PERIODIC,) * 2] * 3, [1, 1, 1]
+    if wall is not None:
+        faces[wall], periodic[wall] = (R.FACE_PEC,) * 2, 0
+    a = random_state(cells, lengths, 3, rng, vscale=0.05)[1]
+    n = len(a["q"])
+    b = cases.uniform_b(cells, (0.0, 0.2, 0.4), amplitude=0.3)
+    kw = dict(particle_periodic=periodic, field_faces=faces)
+    say("planes", cells, wall)
+    with gpu(cells, lengths, [(-4.0, n)], **kw) as sim:
+        sim.set_particles(0, a)
+        sim.set_field(R.FIELD_B, b)
+        sim.initialize()
+        got = sim.get_field(R.FIELD_MASS)
+    ref = O.Sim(cells, lengths, [-4.0], [n], 0.1, **kw)
+    ref.set_particles(0, a)
+    ref.field("B")[:] = b
+    ref.initialize()
+    want = ref.field("mass")
+    assert np.abs(got - want).max() <= 3e-12 * np.abs(want).max()
+    if wall != 2:
+        planes = got.reshape(4, -1)
+        assert np.array_equal(planes, np.broadcast_to(planes[:1], planes.shape))
+    ref.close()
+
+
 # ---- operator, solve and cycle ---------------------------------------------
 
 def test_operator_parity():

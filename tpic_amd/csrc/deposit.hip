@@ -822,9 +822,11 @@ __device__ __forceinline__ int wrap_vertex(int i, int n) { return i < 0 ? n - 1 
 // (vertex, part) sums entries 3 part .. 3 part + 2 of its vertex's record over
 // the stencil's pairs t, reading each pair's moment (m_t, cell) straight from
 // the cell mass records (the three parts of a vertex read one moment's nine
-// entries together), in a fixed order in FP64, and writes them as rows of the
-// entry-major matrix in its storage type (double, or float for the mixed
-// forms). The cell records are double, or float in the mixed forms (their
+// entries together), in a fixed order in FP64. The sums cross LDS, so that
+// the rows of the entry-major matrix are stored by whole waves, in its storage
+// type (double, or float for the mixed forms): stored by the threads that
+// formed them, thirds of a wave to each of three rows, 512 x 512 x 1 took 491 us
+// (now 416; 1.6 GB, 323 at the rate of a copy) and 64^3 in floats 175 (now 160). The cell records are double, or float in the mixed forms (their
 // per-cell sums are FP32, so widening them here gives the same FP64 sums).
 constexpr int kStrip = 64;
 constexpr unsigned kStripThreads = 3 * kStrip;  // (vertex, part)
@@ -837,9 +839,14 @@ constexpr unsigned kAssembleTileRows = 8;
 // vertices each) in tiles of kAssembleTileRows rows (the last tile holds the
 // remaining `last` rows); a tile's planes are visited in z order, and each
 // tile plane, a contiguous range of vertices, is cut into 64-vertex strips.
+// The four vertex planes of a periodic z axis of one cell are images of one
+// sum over the same cells in the same order: it is formed once and stored to
+// all of them (512 x 512 x 1 in FP64: 747 us with every plane summed,
+// 491 with one).
 struct StripWalk {
   unsigned full, last;          // full tiles, rows of the last tile (0: none)
   unsigned per_full, per_last;  // strips of a full tile plane, of a last-tile plane
+  unsigned planes, images;      // planes summed, copies of each that are stored
 };
 
 StripWalk strip_walk(const Grid& g) {
@@ -849,6 +856,9 @@ StripWalk strip_walk(const Grid& g) {
   w.last = ey - w.full * kAssembleTileRows;
   w.per_full = (kAssembleTileRows * ex + kStrip - 1) / kStrip;
   w.per_last = (w.last * ex + kStrip - 1) / kStrip;
+  const bool one = g.nz == 1 && !g.field_wall[2];
+  w.planes = one ? 1u : unsigned(g.nz + 3);
+  w.images = one ? unsigned(g.nz + 3) : 1u;
   return w;
 }
 
@@ -857,12 +867,13 @@ __global__ __launch_bounds__(kStripThreads) void k_assemble_mass(Grid g, StripWa
                                                                  const RecT* __restrict__ cellbuf,
                                                                  MassT* __restrict__ mass,
                                                                  unsigned* __restrict__ validation) {
-  const unsigned ex = unsigned(g.nx + 3), ey = unsigned(g.ny + 3), ez = unsigned(g.nz + 3);
+  const unsigned ex = unsigned(g.nx + 3), ey = unsigned(g.ny + 3), ez = walk.planes;
   // Strip-major block order (the 14 stencil blocks of a strip are adjacent
   // logical blocks, on one XCD), so a strip's cell moments are fetched once
   // into that XCD's L2 and reused by all stencils; the tiles' z order keeps
   // the moments of the cells between two vertex planes in L2 until the
   // second plane reads them.
+  __shared__ MassT s_sum[9][kStrip];
   const unsigned lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const int s = int(lb % kStencils);
   unsigned q = lb / kStencils, first, length, u;
@@ -879,8 +890,8 @@ __global__ __launch_bounds__(kStripThreads) void k_assemble_mass(Grid g, StripWa
     length = walk.last * ex;
   }
   const unsigned lv = threadIdx.x / 3u, part = threadIdx.x % 3u;
-  if (u * kStrip + lv >= length) return;
-  const unsigned v = first + u * kStrip + lv;
+  // A vertex past the tile's end repeats its last one and is not stored.
+  const unsigned v = first + min(u * kStrip + lv, length - 1);
   const int np = c_pairs.count[s];
   const int vi = int(v % ex) - 1, vj = int((v / ex) % ey) - 1, vk = int(v / (ex * ey)) - 1;
   double sum[3] = {0.0, 0.0, 0.0};
@@ -927,9 +938,19 @@ __global__ __launch_bounds__(kStripThreads) void k_assemble_mass(Grid g, StripWa
 #pragma unroll
   for (int e = 0; e < 3; ++e) {
     if (!finite_value(sum[e])) flags |= kInvalidNonfinite;
-    mass[size_t(s * 9 + int(3 * part) + e) * g.vstride + v] = MassT(sum[e]);
+    s_sum[3 * part + e][lv] = MassT(sum[e]);
   }
   if (flags) atomicOr(validation, flags);
+  // The strip's rows are stored by whole waves.
+  __syncthreads();
+  const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  if (u * kStrip + lane >= length) return;
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    const MassT value = s_sum[3 * wave + e][lane];
+    MassT* row = mass + size_t(s * 9 + int(3 * wave) + e) * g.vstride + first + u * kStrip + lane;
+    for (unsigned image = 0; image < walk.images; ++image) row[size_t(image) * ex * ey] = value;
+  }
 }
 
 // Current assembly: per node, 3 components, the corner current of the
@@ -1116,8 +1137,7 @@ int launch_assemble(Context& ctx) {
   phase_begin(ctx, Phase::assemble);
   const Grid& g = ctx.grid;
   const StripWalk walk = strip_walk(g);
-  const unsigned ez = unsigned(g.nz + 3);
-  const unsigned mass_blocks = (walk.full * walk.per_full + walk.per_last) * ez * kStencils;
+  const unsigned mass_blocks = (walk.full * walk.per_full + walk.per_last) * walk.planes * kStencils;
   if (ctx.mass_single)
     k_assemble_mass<<<mass_blocks, kStripThreads, 0, ctx.stream>>>(
         g, walk, static_cast<const float*>(ctx.cellbuf), static_cast<float*>(ctx.mass), ctx.validation);
