@@ -774,7 +774,7 @@ __device__ __forceinline__ void deposit_cells(Grid g, const DepositArgs& args, c
   if (flags) atomicOr(validation, flags);
 }
 
-// FP64 form: its LDS rows (13 KB per wave) hold it to 3 waves per SIMD.
+// FP64 form: its LDS rows (13 KB per wave) hold it to 2 waves per SIMD.
 __global__ __launch_bounds__(kThreads) void k_deposit_fp64(Grid g, DepositArgs args, const double* __restrict__ bnode,
                                                            double inverse_volume, double* __restrict__ cellbuf,
                                                            double* __restrict__ corner, int accumulate,

@@ -988,7 +988,7 @@ int launch_rhs(Context& ctx) {
 namespace {
 
 // Grids up to this many nodes take k_apply_split, larger ones the curl pass
-// and a thread per node.
+// and a thread per node, or per column of a plane.
 constexpr unsigned kSplitNodes = 16384;
 
 struct OperatorArgs {
