@@ -103,6 +103,49 @@ def test_transposed_solve_residual():
     assert np.linalg.norm(atx - b) <= 1e-11 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("cells", [(24, 24, 24), (25, 26, 23), (40, 210, 1)])
+def test_transposed_operator_on_every_form(cells):
+    """At the sizes where the operator's form changes (waves sharing a node's
+    blocks, a thread per node, a thread per column of a plane): <u, A v> =
+    <A^T u, v> to 1e-12 of the products' scale, periodic duplicates equal to
+    1e-12, and |A^T x - b| <= 1e-11 |b| after a solve to 1e-12."""
+    rng = np.random.default_rng(45)
+    lengths, qoms = tuple(0.5 * n for n in cells), (-8.0, 1.0)
+    g, arrays = case(rng, cells, lengths, ppc=2, qoms=qoms)
+    nx, ny, nz = cells
+
+    def expand(x):
+        return np.pad(x.reshape(3, nz, ny, nx), ((0, 0), (0, 1), (0, 1), (0, 1)), mode="wrap").ravel()
+
+    def reduce(x):
+        return x.reshape(3, nz + 1, ny + 1, nx + 1)[:, :nz, :ny, :nx].ravel()
+
+    say("transposed operator", cells)
+    with started(cells, lengths, arrays, qoms, np.zeros(3 * O.node_count(g)), rng.normal(size=3 * O.cell_count(g)) * 0.3,
+                 tol=1e-12) as sim:
+        u = expand(rng.normal(size=3 * nx * ny * nz))
+        v = expand(rng.normal(size=3 * nx * ny * nz))
+        ein, rhs = sim.device_field(R.FIELD_E), sim.device_field(R.FIELD_RHS)
+        sim.set_field(R.FIELD_E, v)
+        sim.apply_operator(ein, rhs)
+        av = sim.get_field(R.FIELD_RHS)
+        sim.set_field(R.FIELD_E, u)
+        sim.apply_operator_transposed(ein, rhs)
+        atu = sim.get_field(R.FIELD_RHS)
+        sim.set_field(R.FIELD_RHS, u)
+        sim.set_field(R.FIELD_ETHETA, np.zeros_like(u))
+        r = sim.solve_transposed(rhs, sim.device_field(R.FIELD_ETHETA))
+        sim.set_field(R.FIELD_E, sim.get_field(R.FIELD_ETHETA))
+        sim.apply_operator_transposed(ein, rhs)
+        atx = sim.get_field(R.FIELD_RHS)
+    left = np.dot(reduce(u), reduce(av))
+    right = np.dot(reduce(atu), reduce(v))
+    assert abs(left - right) <= 1e-12 * np.linalg.norm(reduce(u)) * np.linalg.norm(reduce(av))
+    assert np.abs(atu - expand(reduce(atu))).max() <= 1e-12 * np.abs(atu).max()
+    assert r["converged"] == 1
+    assert np.linalg.norm(atx - u) <= 1e-11 * np.linalg.norm(u)
+
+
 def test_checkpoint_restart_repeats_the_run_bit_for_bit():
     """Six cycles straight; three cycles, a checkpoint, three more; and a
     restore of the checkpoint followed by three cycles: E, B and every
