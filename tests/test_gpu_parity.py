@@ -816,7 +816,7 @@ def test_cycle_incremental_plan_equals_the_run_based_plan(case):
             sim.close()
 
 
-@pytest.mark.parametrize("arrivals", [2, 12, 13, 64, 65, 130, 1100])
+@pytest.mark.parametrize("arrivals", [2, 12, 13, 64, 65, 130, 900, 1100])
 def test_cycle_plan_at_every_arrival_count(arrivals):
     """Bins that receive few to many particles in one step (a thread's list, a
     wave's, several rounds of one, and more than the crosser plan orders) in

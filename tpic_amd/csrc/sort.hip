@@ -624,12 +624,37 @@ __global__ __launch_bounds__(kThreads) void k_cross_bases(CrossPlans plans) {
   }
 }
 
+// The present lanes of a wave that hold the lane's key: the first, how many,
+// and how many before it. A turn per distinct key.
+struct KeyGroup {
+  uint32_t first, size, rank;
+};
+__device__ __forceinline__ KeyGroup key_group(bool present, int32_t key, unsigned lane) {
+  KeyGroup g{lane, 1u, 0u};
+  uint64_t left = __ballot(present);
+  while (left) {
+    const unsigned first = unsigned(__builtin_ctzll(left));
+    const bool same = present && key == __builtin_amdgcn_readlane(key, first);
+    const uint64_t lanes = __ballot(same);
+    if (same) g = KeyGroup{first, uint32_t(__popcll(lanes)), bits_below(uint32_t(lanes), uint32_t(lanes >> 32))};
+    left &= ~lanes;
+  }
+  return g;
+}
+
 // Per crosser one arrival in its new bin (integer atomics: crosser t of the
 // position-ordered crosser list keeps the arrival's index j within the bin in
 // slot[t]; the bins order their arrivals by position afterwards), counted as
 // from a lower bin when its position precedes the bin's old range. Tiles of
 // kTile particles: the crosser words of a wave span and every crosser's key
 // are loaded first, then the atomics and range starts, then the stores.
+// Grouped: the crossers of a wave's item that enter the same bin arrive with
+// one atomic of their number. Atomics at one address follow one another, and in
+// full cells the neighbours cross into the same few bins: a line of 1000 a cell
+// 423 us a cycle one by one, 389 grouped; 512 x 512 of 100 a cell 5992 and 5894.
+// In cells of few particles nearly every key is its own turn of the grouping,
+// so below 80 a cell each arrives alone.
+template <bool Grouped>
 __global__ __launch_bounds__(kThreads) void k_cross_arrivals(CrossPlans plans, uint32_t bins) {
   const CrossPlan& s = plans.species[blockIdx.y];
   const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -654,14 +679,30 @@ __global__ __launch_bounds__(kThreads) void k_cross_arrivals(CrossPlans plans, u
   if (crossers == 0) return;
   wait_loads();
   uint32_t j[kWaveItems], start[kWaveItems];
+  KeyGroup group[kWaveItems];
 #pragma unroll
   for (unsigned r = 0; r < kWaveItems; ++r) {
     const int32_t k = key[r];
     const bool ok = ((crossers >> r) & 1u) && k >= 0 && uint32_t(k) < bins;
-    j[r] = ok ? atomicAdd(s.arrivals + k, 1u) : 0u;
+    if constexpr (Grouped) {
+      group[r] = key_group(ok, k, lane);
+      j[r] = ok && group[r].first == lane ? atomicAdd(s.arrivals + k, group[r].size) : 0u;
+    } else {
+      j[r] = ok ? atomicAdd(s.arrivals + k, 1u) : 0u;
+    }
     start[r] = ok ? s.offsets[k] : 0u;
   }
   wait_loads();
+  if constexpr (Grouped) {
+#pragma unroll
+    for (unsigned r = 0; r < kWaveItems; ++r) {
+      const bool ok = ((crossers >> r) & 1u) && key[r] >= 0 && uint32_t(key[r]) < bins;
+      j[r] = uint32_t(__shfl(int(j[r]), int(group[r].first))) + group[r].rank;
+      const bool below = ok && sub + r * 64 + lane < start[r];
+      const KeyGroup lower = key_group(below, key[r], lane);
+      if (below && lower.first == lane) atomicAdd(s.lower + key[r], lower.size);
+    }
+  }
 #pragma unroll
   for (unsigned r = 0; r < kWaveItems; ++r) {
     if (!((crossers >> r) & 1u)) continue;
@@ -671,7 +712,8 @@ __global__ __launch_bounds__(kThreads) void k_cross_arrivals(CrossPlans plans, u
       continue;
     }
     s.slot[list[r]] = j[r];
-    if (sub + r * 64 + lane < start[r]) atomicAdd(s.lower + k, 1u);
+    if constexpr (!Grouped)
+      if (sub + r * 64 + lane < start[r]) atomicAdd(s.lower + k, 1u);
   }
 }
 
@@ -1104,17 +1146,21 @@ int launch_sort_plan_incremental(Context& ctx, int first, int species, SortWorks
   }
   const unsigned y = unsigned(species);
   const unsigned block_tiles = (blocks + kPlanTile - 1) / kPlanTile, bin_tiles = (bins + kPlanTile - 1) / kPlanTile;
+  uint64_t particles = 0;
+  for (int t = 0; t < species; ++t) particles = std::max<uint64_t>(particles, plans.species[t].n);
+  const bool grouped = particles >= 80ull * g.cells();
   k_cross_begin<<<dim3(std::max(block_tiles, bin_tiles), y), kThreads, 0, st>>>(plans, bins);
   k_cross_bases<<<dim3(block_tiles, y), kThreads, 0, st>>>(plans);
-  k_cross_arrivals<<<dim3(tiles, y), kThreads, 0, st>>>(plans, bins);
+  if (grouped)
+    k_cross_arrivals<true><<<dim3(tiles, y), kThreads, 0, st>>>(plans, bins);
+  else
+    k_cross_arrivals<false><<<dim3(tiles, y), kThreads, 0, st>>>(plans, bins);
   k_cross_counts_new<<<dim3(bin_tiles, y), kThreads, 0, st>>>(plans, bins);
   k_cross_offsets<<<dim3(bin_tiles, y), kThreads, 0, st>>>(plans, g, ctx.validation);
   k_cross_sources<<<dim3(tiles, y), kThreads, 0, st>>>(plans, bins);
   // A species' arrivals a bin grow with its particles a cell (a few percent to
   // a sixth of them): at 1000 a cell nearly every bin is listed, and 256 bins
   // a block leave four waves 64 lists each (479 us for a 1024-cell line).
-  uint64_t particles = 0;
-  for (int t = 0; t < species; ++t) particles = std::max<uint64_t>(particles, plans.species[t].n);
   const uint32_t per_block = particles >= 256ull * g.cells() ? 4u : (particles >= 80ull * g.cells() ? 64u : kThreads);
   k_cross_bins<<<dim3((bins + per_block - 1) / per_block, y), kThreads, 0, st>>>(plans, g, per_block);
   const int rc = check_hip(ctx, hipGetLastError(), "sort plan from crossers");
