@@ -103,6 +103,56 @@ def test_transposed_solve_residual():
     assert np.linalg.norm(atx - b) <= 1e-11 * np.linalg.norm(b)
 
 
+def test_transposed_solve_from_its_solution():
+    """A solve warm-started from its own solution, after a solve of another
+    right-hand side, takes no step and keeps the solution bit for bit."""
+    rng = np.random.default_rng(44)
+    cells, lengths, qoms = (6, 4, 2), (3.0, 2.0, 1.0), (-8.0, 1.0)
+    g, arrays = case(rng, cells, lengths, ppc=4, qoms=qoms)
+    box = AD.Box(g)
+    say("transposed solve from its solution")
+    with started(cells, lengths, arrays, qoms, np.zeros(3 * box.nodes), rng.normal(size=3 * O.cell_count(g)) * 0.3,
+                 tol=1e-12) as sim:
+        def solved(b, x):
+            sim.set_field(R.FIELD_RHS, b)
+            sim.set_field(R.FIELD_ETHETA, x)
+            r = sim.solve_transposed(sim.device_field(R.FIELD_RHS), sim.device_field(R.FIELD_ETHETA))
+            return r["iterations"], sim.get_field(R.FIELD_ETHETA)
+
+        b, other = (box.expand(rng.normal(size=3 * box.unique)) for _ in range(2))
+        steps, x = solved(b, np.zeros_like(b))
+        assert steps > 0
+        assert solved(other, np.zeros_like(b))[0] > 0
+        again, same = solved(b, x)
+    assert again == 0 and np.array_equal(same, x)
+
+
+def test_adjoint_of_nothing_is_zero():
+    """Adjoint cycles seeded with zero weights, whose transposed solves have
+    no right-hand side: every gradient is exactly zero."""
+    rng = np.random.default_rng(52)
+    cells, lengths, qoms = (5, 4, 3), (2.5, 2.0, 1.5), (-8.0, 1.0)
+    g, arrays = case(rng, cells, lengths, ppc=4, qoms=qoms)
+    box = AD.Box(g)
+    e0 = box.expand(rng.normal(size=3 * box.unique) * 0.01)
+    say("adjoint of nothing")
+    with started(cells, lengths, arrays, qoms, e0, rng.normal(size=3 * O.cell_count(g)) * 0.05) as sim:
+        sim.checkpoint_reserve(2)
+        for n in range(2):
+            sim.checkpoint_save(n)
+            sim.cycle(1)
+        with sim.adjoint() as adj:
+            adj.seed_field_energy(0.0, 0.0, [0, 100000])
+            for n in (1, 0):
+                sim.checkpoint_restore(n)
+                _, transposed = adj.cycle()
+                assert transposed["converged"] and transposed["iterations"] == 0
+            assert not adj.field(R.FIELD_E).any() and not adj.field(R.FIELD_B).any()
+            for s in range(2):
+                parts = adj.particles(s)
+                assert not any(parts[key].any() for key in ("rbar", "vbar", "qbar"))
+
+
 @pytest.mark.parametrize("cells", [(24, 24, 24), (25, 26, 23), (40, 210, 1)])
 def test_transposed_operator_on_every_form(cells):
     """At the sizes where the operator's form changes (waves sharing a node's

@@ -1306,6 +1306,100 @@ def test_operator_and_solve_on_both_forms(name):
     ref.close()
 
 
+# A grid of every form of the operator, with what its walls leave uniform.
+REST_GRIDS = {
+    "small": ((24, 24, 24), None, None),
+    "small_walls": ((12, 11, 10), (1, R.FACE_PMC), None),
+    "small_smoothed": ((9, 8, 7), None, (R.SMOOTH_BINOMIAL27, 3, 0.25)),
+    "nodes": ((25, 26, 23), None, None),
+    "walls": ((25, 26, 23), (1, R.FACE_PEC), None),
+    "smoothed": ((25, 26, 23), None, (R.SMOOTH_FACE7, 2, 0.5)),
+    "plane": ((150, 120, 1), None, None),
+    "largest": ((84, 80, 79), None, None),
+}
+
+
+@pytest.mark.parametrize("name", list(REST_GRIDS))
+def test_solve_whose_guess_meets_the_tolerance(name):
+    """A solve that needs no step leaves E_theta at its guess, E^n with its
+    constrained rows zeroed, bit for bit: a context's first solve and one
+    after another solve, from a uniform E and from none."""
+    cells, wall, smoothing = REST_GRIDS[name]
+    lengths = tuple(0.25 * n for n in cells)
+    nx, ny, nz = cells
+    rng = np.random.default_rng(53)
+    faces, periodic = [(R.FACE_PERIODIC,) * 2] * 3, [1, 1, 1]
+    uniform = np.zeros((3, nz + 1, ny + 1, nx + 1))
+    uniform += np.array([0.3, -0.2, 0.7]).reshape(3, 1, 1, 1)
+    given = uniform.copy()
+    if wall:
+        axis, kind = wall
+        faces[axis], periodic[axis] = (kind,) * 2, 0
+        for c in range(3):
+            if (c == axis) == (kind == R.FACE_PMC):  # held at zero on the walls
+                uniform[c] = given[c] = 0.0
+                planes = [slice(None)] * 3
+                planes[2 - axis] = [0, -1]
+                given[(c, *planes)] = 0.4
+    moving = periodic_duplicates(cells, rng.normal(size=uniform.size), wall[0] if wall else None)
+    b = np.zeros(3 * nx * ny * nz) if wall else cases.uniform_b(cells, (0.1, 0.2, 0.4), amplitude=0.0)
+    rest = ((given, uniform), (np.zeros_like(given), np.zeros_like(given)))
+    say("solve at rest", name)
+
+    def solved(sim, e):
+        sim.set_field(R.FIELD_E, e.ravel())
+        _, r = sim.solve()
+        assert r["converged"]
+        return r["iterations"], sim.get_field(R.FIELD_ETHETA)
+
+    for first in (0, 1):
+        with gpu(cells, lengths, [(-1.0, 0)], gmres_tolerance=1e-3, particle_periodic=periodic, field_faces=faces,
+                 smoothing=smoothing) as sim:
+            sim.set_field(R.FIELD_B, b)
+            sim.initialize()
+            for e, want in rest[first:]:
+                steps, theta = solved(sim, e)
+                assert steps == 0 and np.array_equal(theta, want.ravel())
+            steps, theta = solved(sim, moving)
+            assert steps > 0 and not np.array_equal(theta, moving)
+            for e, want in rest:
+                steps, theta = solved(sim, e)
+                assert steps == 0 and np.array_equal(theta, want.ravel())
+
+
+def test_cycles_at_a_loose_tolerance_against_the_oracle():
+    """A thin plasma in a nearly uniform E at GMRES 1e-3: cycles that need a
+    step and cycles that need none, with the oracle's iteration counts and its
+    fields to 1e-10."""
+    cells, lengths, qom = (10, 9, 8), (2.5, 2.25, 2.0), [-16.0, 1.0]
+    arrays, b = setup_plasma(cells, lengths, (2, 2, 2), qom, [0.05, 0.01], (0.01, 0.02, 0.05), 0.02)
+    for a in arrays:
+        a["q"] = a["q"] * 1e-3
+    counts = [len(a["q"]) for a in arrays]
+    ref = O.Sim(cells, lengths, qom, counts, dt=0.1, tol=1e-3)
+    e = np.repeat([0.12, 0.18, -0.06], ref.field("E").size // 3)
+    with gpu(cells, lengths, list(zip(qom, counts)), gmres_tolerance=1e-3) as sim:
+        for s, a in enumerate(arrays):
+            sim.set_particles(s, a)
+            ref.set_particles(s, a)
+        sim.set_field(R.FIELD_E, e)
+        sim.set_field(R.FIELD_B, b)
+        ref.field("E")[:], ref.field("B")[:] = e, b
+        sim.initialize()
+        ref.initialize()
+        steps = []
+        for _ in range(12):
+            got = sim.cycle(1)
+            rc, want = ref.cycle(1)
+            assert rc == 0 and got["iterations"] == want.iterations
+            steps.append(want.iterations)
+            for which, field in ((R.FIELD_ETHETA, "theta"), (R.FIELD_E, "E"), (R.FIELD_B, "B"), (R.FIELD_J, "J")):
+                assert rel(sim.get_field(which), ref.field(field)) <= 1e-10, field
+    say("iterations", steps)
+    assert min(steps) == 0 and max(steps) > 0
+    ref.close()
+
+
 @pytest.mark.parametrize("case", ["GEMHarris", "DoubleGEM"])
 def test_harris_load_matches_the_oracle(case):
     """tpic_mi_load_harris against the oracle's Harris profile: positions,

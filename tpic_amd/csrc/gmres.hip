@@ -72,6 +72,7 @@ enum Word : int {
   kNonfinite,   // 1: a non-finite recurrence
   kGo,          // 1: the restart's tail (update, true residual) is to run
   kConverged,   // 1: the true residual met the tolerance
+  kCommit,      // 1: it did so after a restart, whose x is the solution (a guess that met it stays)
   kTails,       // tails run
   kDone,        // steps of the last tail
   kDoneBreakdown,
@@ -201,6 +202,7 @@ __global__ __launch_bounds__(kThreads) void k_residual_test(const double* __rest
   const bool converged = good && r <= absolute;
   w[kResidual2] = r2;
   w[kConverged] = converged ? 1.0 : 0.0;
+  w[kCommit] = converged && !first ? 1.0 : 0.0;
   w[kStop] = converged || !good || (!first && w[kBreakdown] != 0.0) ? 1.0 : 0.0;
   w[kGo] = 0.0;
   w[kSteps] = 0.0;
@@ -452,7 +454,7 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
     k_update<<<w.blocks, kThreads, 0, st>>>(basis, x, w.x, n, s, going);
     if (int e = check_hip(ctx, hipGetLastError(), "gmres update")) return e;
     if (int e = residual(w.x, 0, going)) return e;
-    k_commit<<<w.blocks, kThreads, 0, st>>>(w.x, solution, n, Guard{s.word + kConverged, 0.0});
+    k_commit<<<w.blocks, kThreads, 0, st>>>(w.x, solution, n, Guard{s.word + kCommit, 0.0});
     return check_hip(ctx, hipGetLastError(), "gmres commit");
   };
   phase_begin(ctx, Phase::solve);
