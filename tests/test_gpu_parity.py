@@ -1367,6 +1367,40 @@ def test_solve_whose_guess_meets_the_tolerance(name):
                 assert steps == 0 and np.array_equal(theta, want.ravel())
 
 
+@pytest.mark.parametrize("smoothing", [None, (R.SMOOTH_FACE7, 5, 0.5)], ids=["plain", "smoothed"])
+def test_repeated_solves_enqueue_the_steps_they_take(smoothing):
+    """Operator calls of solves repeated with the same number of steps: one
+    per step and one per residual (of the guess, and after the steps)."""
+    cells, lengths = (12, 11, 10), (3.0, 2.75, 2.5)
+    arrays, b = setup_plasma(cells, lengths, (2, 2, 2), [-16.0], [0.05], (0.0, 0.2, 0.4), 0.3)
+    rng = np.random.default_rng(54)
+    moving = periodic_nodes(cells, rng, 0.05)
+    with gpu(cells, lengths, [(-16.0, len(arrays[0]["q"]))], gmres_tolerance=1e-3, smoothing=smoothing) as sim:
+        sim.set_particles(0, arrays[0])
+        sim.initialize()
+        sim.enable_timing()
+
+        def solved(e):
+            sim.set_field(R.FIELD_E, e)
+            sim.reset_timing()
+            steps = sim.solve()[1]["iterations"]
+            return steps, sim.phase_time("spmv")[1]
+
+        say("repeated solves", smoothing)
+        sim.set_field(R.FIELD_B, b)
+        first, _ = solved(moving)
+        assert 1 < first < 8
+        for _ in range(2):
+            assert solved(moving) == (first, 2 + first)
+        sim.set_field(R.FIELD_B, 0.0 * b)
+        sim.set_field(R.FIELD_J, 0.0 * moving)
+        assert solved(0.0 * moving)[0] == 0
+        for _ in range(2):
+            assert solved(0.0 * moving) == (0, 1)
+        again, _ = solved(moving)
+        assert again > 1 and solved(moving) == (again, 2 + again)
+
+
 def test_cycles_at_a_loose_tolerance_against_the_oracle():
     """A thin plasma in a nearly uniform E at GMRES 1e-3: cycles that need a
     step and cycles that need none, with the oracle's iteration counts and its

@@ -29,8 +29,8 @@
 // The reference's host reads two control scalars per step. Here the Givens
 // update tests them (the estimate against the tolerance, the breakdown) and
 // raises a stop word, and the tests of the first and of the true residual are
-// kernels too: the host enqueues the first residual, a batch of steps, the
-// update, the true residual and the commit, each guarded by those words, and
+// kernels too: the host enqueues the first residual, the steps it expects,
+// the update, the true residual and the commit, each guarded by those words, and
 // reads the words once. The same steps run and stop where they would.
 //
 // Reductions are deterministic: fixed partials added in a fixed order.
@@ -459,18 +459,29 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
   };
   phase_begin(ctx, Phase::solve);
   if ((rc = residual(solution, 1, Guard{}))) return rc;
-  // Steps enqueued between two reads of the words.
-  constexpr int kStepsPerRead = 8;
+  // Steps enqueued before the next read of the words, after `done` of this
+  // solve: up to those that the operator's last solve took, then half as many
+  // again. A step past the stop costs its launches (3.6 us each at 16^3; with
+  // ten smoothing passes 23 of them), a read the time to refill the queue, and
+  // the solves of a run change their steps slowly. With eight steps to every
+  // read, a solve of two steps with ten passes at 16^3 took 1014 us, now 500
+  // (one step to a read: 600), and a guess that met the tolerance 128, now 27
+  // (a read of its own: 70); without smoothing two steps took 118, now 78.
+  int& expected = w.expected[ctx.transposed_operator ? 1 : 0];
+  const auto batch = [&](int done, bool first) {
+    if (done < expected) return std::min(kStepsPerRead, expected - done);
+    return first ? 0 : std::min(kStepsPerRead, std::max(2, done / 2));
+  };
   bool converged = false, first_read = true;
   int iterations = 0, enqueued = 0, tails = 0;
   double word[kWords];
   while (!converged && iterations < ctx.num.max_iterations) {
     const int columns = std::min(m, ctx.num.max_iterations - iterations);
-    const int upto = std::min(columns, enqueued + kStepsPerRead);
+    const int upto = std::min(columns, enqueued + batch(iterations + enqueued, first_read));
     for (int col = enqueued; col < upto; ++col)
       if ((rc = arnoldi(col, col + 1 == columns))) return rc;
     enqueued = upto;
-    if ((rc = finish(tails ? w.x : solution))) return rc;
+    if (enqueued && (rc = finish(tails ? w.x : solution))) return rc;
     TPIC_TRY(hipMemcpyAsync(w.controls, s.word, kWords * sizeof(double), hipMemcpyDeviceToHost, st),
              "gmres readback");
     TPIC_TRY(hipStreamSynchronize(st), "gmres readback");
@@ -488,6 +499,7 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
     if (word[kDoneBreakdown] != 0.0) break;
   }
   phase_end(ctx, Phase::solve);
+  expected = iterations;
   const double res = std::sqrt(word[kResidual2]), rhs_norm = std::sqrt(word[kRhs2]);
   *converged_out = converged ? 1 : 0;
   *iterations_out = iterations;

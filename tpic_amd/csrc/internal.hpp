@@ -70,6 +70,9 @@ struct SortWorkspace {
   uint32_t* bin_lower = nullptr;   // [bins] arrivals from lower bins
 };
 
+// Most solver steps enqueued between two reads of the solver's words.
+constexpr int kStepsPerRead = 8;
+
 struct GmresWorkspace {
   unsigned count = 0;       // 3 * nodes
   unsigned blocks = 0;      // reduction blocks
@@ -81,6 +84,9 @@ struct GmresWorkspace {
   unsigned* arrivals = nullptr;  // blocks of a running launch that are done (0 between launches)
   double* controls = nullptr;  // pinned host copy of the words
   double* curl_cells = nullptr;   // [3 * cells] scratch of the operator
+  // Steps of the last solve with the operator and with its transpose: how many
+  // the next one enqueues before it looks whether they were needed.
+  int expected[2] = {kStepsPerRead, kStepsPerRead};
 };
 
 struct Context {
