@@ -281,6 +281,48 @@ def test_adjoint_cycles_match_the_oracle_adjoint():
             assert np.abs(g_ - exp[key]).max() <= 1e-8 * np.abs(exp[key]).max(), (s, key)
 
 
+def test_refused_adjoint_cycle_changes_nothing():
+    """An adjoint cycle on particles with other ids is refused before it
+    replaces anything: the context's E_theta and right-hand side and the
+    adjoint stay, bit for bit, and the cycle on the right state then gives the
+    gradients of a run without the refused call."""
+    rng = np.random.default_rng(56)
+    cells, lengths, qoms = (5, 4, 3), (2.5, 2.0, 1.5), (-8.0, 1.0)
+    g, arrays = case(rng, cells, lengths, ppc=4, qoms=qoms)
+    box = AD.Box(g)
+    e0 = box.expand(rng.normal(size=3 * box.unique) * 0.01)
+    b0 = rng.normal(size=3 * O.cell_count(g)) * 0.05
+    foreign = dict(arrays[1], id=arrays[1]["id"] + np.uint64(7))
+    say("refused adjoint cycle")
+
+    def state(sim, adj):
+        out = [sim.get_field(f) for f in (R.FIELD_ETHETA, R.FIELD_RHS, R.FIELD_E, R.FIELD_B)]
+        out += [adj.field(R.FIELD_E), adj.field(R.FIELD_B)]
+        return out + [v for s in range(2) for v in adj.particles(s).values()]
+
+    results = []
+    for refuse in (False, True):
+        with started(cells, lengths, arrays, qoms, e0, b0) as sim:
+            sim.checkpoint_reserve(1)
+            sim.checkpoint_save(0)
+            sim.cycle(1)
+            with sim.adjoint() as adj:
+                adj.seed_field_energy(1.0, 0.5, [0, 100000])
+                if refuse:
+                    sim.set_particles(1, foreign)
+                    sim.set_field(R.FIELD_E, 3.0 * e0)
+                    sim.initialize()
+                    before = state(sim, adj)
+                    with pytest.raises(R.TpicError) as failed:
+                        adj.cycle()
+                    assert failed.value.status == R.INVALID_STATE
+                    assert all(np.array_equal(x, y) for x, y in zip(before, state(sim, adj)))
+                sim.checkpoint_restore(0)
+                adj.cycle()
+                results.append(state(sim, adj))
+    assert all(np.array_equal(x, y) for x, y in zip(*results))
+
+
 @pytest.mark.parametrize("ppc", [1, 7, 18, 19, 36, 37, 71])
 def test_adjoint_cycle_at_every_lane_group(ppc):
     """Two adjoint cycles at the particles per cell on both sides of the lines

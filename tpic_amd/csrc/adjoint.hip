@@ -526,6 +526,7 @@ struct tpic_mi_adjoint {
   double* record = nullptr;      // [24][cells] per-cell corner sums
   unsigned* flag = nullptr;      // id check word
   unsigned* host_flag = nullptr; // pinned
+  hipEvent_t checked = nullptr;  // the id check word is on the host
 };
 
 namespace {
@@ -540,6 +541,8 @@ void free_adjoint(tpic_mi_adjoint* a) {
   device_free(a->flag);
   if (a->host_flag) (void)hipHostFree(a->host_flag);
   a->host_flag = nullptr;
+  if (a->checked) (void)hipEventDestroy(a->checked);
+  a->checked = nullptr;
 }
 
 // The adjoint is built for periodic fields and particles, no smoothing.
@@ -553,8 +556,7 @@ int adjoint_supported(Context& c) {
 
 // The particle adjoints permuted into the context's current particle order in
 // each species' other slot, and the id check word on its way to the host
-// (valid after the stream's next synchronisation; the slots change when it is
-// clear).
+// (valid after `checked`; the slots change when it is clear).
 int permute_to_context(Context& c, tpic_mi_adjoint* a) {
   int rc = check_hip(c, hipMemsetAsync(a->flag, 0, sizeof(unsigned), c.stream), "adjoint flag");
   if (rc) return rc;
@@ -569,8 +571,9 @@ int permute_to_context(Context& c, tpic_mi_adjoint* a) {
                                                  ad.slot[ad.current], ad.slot[other], ad.id_slot[other], a->flag);
     if ((rc = check_hip(c, hipGetLastError(), "adjoint permutation"))) return rc;
   }
-  return check_hip(c, hipMemcpyAsync(a->host_flag, a->flag, sizeof(unsigned), hipMemcpyDeviceToHost, c.stream),
-                   "adjoint flag");
+  rc = check_hip(c, hipMemcpyAsync(a->host_flag, a->flag, sizeof(unsigned), hipMemcpyDeviceToHost, c.stream),
+                 "adjoint flag");
+  return rc ? rc : check_hip(c, hipEventRecord(a->checked, c.stream), "adjoint flag");
 }
 
 SpeciesPass species_pass(Context& c, AdjointArrays& ad, size_t s) {
@@ -649,6 +652,7 @@ int tpic_mi_adjoint_create(tpic_mi_context* h, tpic_mi_adjoint** out) {
       !(rc = device_alloc(c, &a->curl_cells, 3 * cells, "adjoint")) &&
       !(rc = device_alloc(c, &a->record, 24 * cells, "adjoint")) && !(rc = device_alloc(c, &a->flag, 1, "adjoint")))
     rc = check_hip(c, hipHostMalloc(reinterpret_cast<void**>(&a->host_flag), sizeof(unsigned)), "adjoint pinned");
+  if (!rc) rc = check_hip(c, hipEventCreateWithFlags(&a->checked, hipEventDisableTiming), "adjoint event");
   if (rc) {
     free_adjoint(a);
     delete a;
@@ -706,24 +710,25 @@ int tpic_mi_adjoint_cycle(tpic_mi_context* h, tpic_mi_adjoint* a, tpic_mi_solve_
     if (!sp.sorted) return fail(c, TPIC_MI_INVALID_STATE, "the adjoint cycle starts from a sorted state");
   const Grid& g = c.grid;
   const size_t nodes = g.nodes(), cells = g.cells();
-  // 1. The particle adjoints into this state's order; 2. E_theta of this
-  // cycle, recomputed as the forward cycle computed it (its solve waits for
-  // the stream, the id check word with it).
+  // 1. The particle adjoints into this state's order, and while their id check
+  // word travels Ebar_theta = Ebar'/theta - c dt curl_C2N(Bbar') into scratch: a
+  // refused call has changed nothing that can be read.
   int rc = permute_to_context(c, a);
   if (rc) return rc;
-  const int solved = tpic_mi_solve(h, forward);
-  if (solved && (rc = check_hip(c, hipStreamSynchronize(c.stream), "adjoint flag"))) return rc;
-  if (*a->host_flag) return fail(c, TPIC_MI_INVALID_STATE, "particle ids are not a permutation of each species' first ids");
-  for (AdjointArrays& ad : a->species) ad.current ^= 1;
-  if (solved) return solved;
-  // 3. Field update: Ebar_theta = Ebar'/theta - c dt curl_C2N(Bbar');
-  //    Ebar^n = -(1 - theta)/theta Ebar'; Bbar^n = Bbar' (in place).
   const double theta = c.num.theta;
   const bool copy = std::abs(theta - 1.0) < 1e-10;
   const double c0 = copy ? 1.0 : 1.0 / theta, c1 = copy ? 0.0 : -(1.0 - theta) / theta;
   if ((rc = launch_curl_c2n(c, a->bbar, a->curl))) return rc;
   k_combine<<<grid_for(c, 3 * nodes), kThreads, 0, c.stream>>>(unsigned(3 * nodes), c0, a->ebar, -c.num.c * c.num.dt,
                                                                  a->curl, a->ethetabar);
+  if ((rc = check_hip(c, hipGetLastError(), "adjoint field update"))) return rc;
+  if ((rc = check_hip(c, hipEventSynchronize(a->checked), "adjoint flag"))) return rc;
+  if (*a->host_flag) return fail(c, TPIC_MI_INVALID_STATE, "particle ids are not a permutation of each species' first ids");
+  for (AdjointArrays& ad : a->species) ad.current ^= 1;
+  // 2. E_theta of this cycle, recomputed as the forward cycle computed it.
+  if ((rc = tpic_mi_solve(h, forward))) return rc;
+  // 3. The rest of the field update: Ebar^n = -(1 - theta)/theta Ebar';
+  //    Bbar^n = Bbar' (in place).
   k_combine<<<grid_for(c, 3 * nodes), kThreads, 0, c.stream>>>(unsigned(3 * nodes), c1, a->ebar, 0.0, nullptr,
                                                                  a->ebar);
   if ((rc = check_hip(c, hipGetLastError(), "adjoint field update"))) return rc;
