@@ -856,6 +856,67 @@ def test_cycle_plan_at_every_arrival_count(arrivals):
             sim.close()
 
 
+class DeviceArray:
+    """A context's device array for torch."""
+
+    def __init__(self, address, count, kind):
+        self.__cuda_array_interface__ = {"data": (address, False), "shape": (count,), "typestr": kind, "version": 2}
+
+
+@pytest.mark.parametrize("case", ["two", "three", "handed-over"])
+def test_cycle_plan_on_the_side_stream(case):
+    """From 40 million particles on, species 0's crosser plan runs beside the
+    moves of the others. Two and three species, the last of them small, and a
+    species 0 with more arrivals a bin than the crosser plan orders (planned
+    again, by runs, after the join): as the run-based plans, bit for bit."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(59)
+    cells = lengths = (32, 32, 16)
+    ppc = (14, 14, 13)
+    many = int(np.prod(cells)) * int(np.prod(ppc))
+    assert many >= 40_000_000
+    small = cases.uniform_maxwellian(cells, lengths, (3, 3, 3), 1.0, thermal=(0.4,) * 3, seed=5)
+    arrays = {0: converging_slab(cells, 1100, 10.0, rng) if case == "handed-over" else small}
+    if case == "three":
+        arrays[2] = converging_slab(cells, 30, 10.0, rng)
+    for a in arrays.values():
+        a["q"] = a["q"] * 1e-3
+    spec = [(-1.0, len(arrays[0]["q"])), (1.0, many)]
+    if case == "three":
+        spec.append((-2.0, len(arrays[2]["q"])))
+    b = cases.uniform_b(cells, (0.01, 0.02, 0.05), amplitude=0.2)
+    say("side stream", case, "particles", [n for _, n in spec])
+    sims = [gpu(cells, lengths, spec, dt=0.1, gmres_tolerance=1e-12) for _ in range(2)]
+    try:
+        sims[1].record_permutation(True)
+        for sim in sims:
+            for s, a in arrays.items():
+                sim.set_particles(s, a)
+            sim.load_maxwellian(1, ppc, rho=1e-3, thermal=(0.3,) * 3, seed=7, first_id=10 ** 9)
+            sim.set_field(R.FIELD_B, b)
+            sim.initialize()
+        for _ in range(3):
+            steps = [sim.cycle(1)["iterations"] for sim in sims]
+            assert steps[0] == steps[1]
+            for sim in sims:
+                sim.synchronize()
+            for s, (_, n) in enumerate(spec):
+                for at, name in enumerate(R.ATTRIBUTES):
+                    kind = {"cell": "<i4", "id": "<i8"}.get(name, "<f8")
+                    x, y = (torch.as_tensor(DeviceArray(sim.device_particles(s, at), n, kind), device="cuda")
+                            for sim in sims)
+                    assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), (s, name)
+                for x, y in zip(sims[0].get_bins(s), sims[1].get_bins(s)):
+                    assert np.array_equal(x, y), s
+            torch.cuda.synchronize()
+        for which in (R.FIELD_E, R.FIELD_B, R.FIELD_J, R.FIELD_MASS):
+            assert np.array_equal(sims[0].get_field(which), sims[1].get_field(which)), which
+        assert sims[0].validation() == sims[1].validation() == 0
+    finally:
+        for sim in sims:
+            sim.close()
+
+
 def test_energy_conservation_on_gpu():
     cells, lengths = (12, 10, 8), (3.0, 2.5, 2.0)
     arrays, b = setup_plasma(cells, lengths, (2, 2, 2), [-25.0, 1.0], [0.08, 0.016], (0.0, 0.0, 0.02), 0.3)
@@ -1214,9 +1275,10 @@ def test_walled_solve_projects_a_field_set_after_startup(kind):
         ref.close()
 
 
-# Grids on both sides of the lines between the operator's forms (16384 and
-# 262144 nodes), with a part-filled last block, one-cell axes, walls and smoothing, and
-# restarts shorter than the solve.
+# Grids on both sides of the lines between the operator's forms (16384 nodes,
+# and 2048 blocks of 256 nodes or columns: 524288), with a part-filled last
+# block and last arrival group, one-cell axes, walls and smoothing, and restarts
+# shorter than the solve.
 SOLVER_GRIDS = {
     "small": ((24, 24, 24), None, None, 30),
     "small_restarted": ((13, 9, 11), None, None, 3),
@@ -1229,7 +1291,8 @@ SOLVER_GRIDS = {
     "large_smoothed": ((25, 26, 23), None, (R.SMOOTH_FACE7, 2, 0.5), 30),
     "large_one_cell_walled_plane": ((30, 320, 1), (1, R.FACE_PEC), None, 30),
     "large_plane_restarted": ((150, 60, 1), None, None, 4),
-    "largest_fused": ((66, 64, 61), None, None, 30),
+    "middle_fused": ((66, 64, 61), None, None, 30),
+    "largest_fused": ((79, 79, 80), None, None, 30),
     "largest": ((84, 80, 79), None, None, 30),
 }
 
