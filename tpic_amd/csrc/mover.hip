@@ -643,11 +643,12 @@ int launch_moves(Context& ctx, int first, int last, const bool* record_crossers)
     MoveBatch batch{};
     unsigned species = 0, blocks = 0;
     for (int s = first; s < last; ++s) {
-      const SpeciesState& sp = ctx.species[size_t(s)];
+      SpeciesState& sp = ctx.species[size_t(s)];
       if (sp.count == 0 || !sp.sorted || slots_for(ctx, sp) != slots) continue;
       batch.species[species++] = MoveSpecies{mover_params(ctx, sp), sp.view(), sp.count, sp.counts, sp.offsets,
                                              record_crossers[s - first] ? sp.cross : nullptr};
       blocks = std::max(blocks, block_walk_blocks(ctx, sp.count));
+      sp.sorted = false;  // also where this launch or a later one fails
     }
     if (species == 0) continue;
     const dim3 grid(blocks, species);
@@ -660,8 +661,6 @@ int launch_moves(Context& ctx, int first, int last, const bool* record_crossers)
     if (int rc = check_hip(ctx, hipGetLastError(), "mover")) return rc;
   }
   phase_end(ctx, Phase::move);
-  for (int s = first; s < last; ++s)
-    if (ctx.species[size_t(s)].count != 0) ctx.species[size_t(s)].sorted = false;
   return 0;
 }
 
