@@ -842,7 +842,9 @@ constexpr unsigned kAssembleTileRows = 8;
 // The four vertex planes of a periodic z axis of one cell are images of one
 // sum over the same cells in the same order: it is formed once and stored to
 // all of them (512 x 512 x 1 in FP64: 747 us with every plane summed,
-// 491 with one).
+// 491 with one). The images of an x or y axis of one cell lie within the rows
+// and planes that the strips walk and are summed each; planes of the decks and
+// tests are one cell deep in z.
 struct StripWalk {
   unsigned full, last;          // full tiles, rows of the last tile (0: none)
   unsigned per_full, per_last;  // strips of a full tile plane, of a last-tile plane

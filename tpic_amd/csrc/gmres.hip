@@ -467,10 +467,12 @@ int run_gmres_system(Context& ctx, const double* rhs_in, double* solution, int* 
   // read, a solve of two steps with ten passes at 16^3 took 1014 us, now 500
   // (one step to a read: 600), and a guess that met the tolerance 128, now 27
   // (a read of its own: 70); without smoothing two steps took 118, now 78.
+  // Solves of one and two steps in turn, each expecting the other's: 97 us (110
+  // with eight to a read), with ten passes 475 (one to a read: 425 to 545).
   int& expected = w.expected[ctx.transposed_operator ? 1 : 0];
   const auto batch = [&](int done, bool first) {
     if (done < expected) return std::min(kStepsPerRead, expected - done);
-    return first ? 0 : std::min(kStepsPerRead, std::max(2, done / 2));
+    return first ? 0 : std::min(kStepsPerRead, std::max(ctx.num.smoothing ? 1 : 2, done / 2));
   };
   bool converged = false, first_read = true;
   int iterations = 0, enqueued = 0, tails = 0;

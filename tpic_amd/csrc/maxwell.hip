@@ -628,8 +628,7 @@ __global__ __launch_bounds__(kThreads) void k_apply(Grid g, const double* __rest
 // (-1 is node 0, +1 node 1 for both), so a pair costs little more than a
 // node: 18 of the 27 products and the curl term are shared. 512 x 512 x 1 in
 // FP64 reads 267 MB of blocks in 90 us where a thread per node took 126 (55 us
-// at the rate of a copy); 52000 columns' waves fill the chip, and below 16384
-// nodes k_apply_split keeps its eight waves per 64 nodes.
+// at the rate of a copy).
 template <class MassT, bool Transposed>
 __device__ __forceinline__ void add_block(const MassT (&b)[9], const double (&a)[3], double (&m)[3]) {
 #pragma unroll
@@ -1037,7 +1036,14 @@ void node_kernel(const OperatorArgs& a, const double* in, const double* curl, co
           a.g, in, curl, mass, response, a.d2, a.k, a.inverse_volume, out, rows, a.scale, a.tail, a.guard);
 }
 
-// Grids whose thread takes a column's two nodes.
+// Grids whose thread takes a column's two nodes, where they are past
+// k_apply_split: an operator call (curl included) at 92 x 92 x 1 takes 14 us and
+// 16 with a thread per node, at 181 x 181 17 and 26, at 512 x 512 98 and 121 (in
+// floats 12 and 12, 12 and 17, 57 and 74). Decks and tests lay a plane in x and
+// y; one that is a cell deep in x or y has its columns' nodes apart and takes
+// the general form, as do planes with walls, whose two nodes differ in images
+// and signs (cycles of 256 x 256 cells with 64 a cell: 1.27 ms one cell deep in
+// z, 1.39 in y, 1.95 in x).
 bool plane_form(const Grid& g) { return g.nz == 1 && !g.walls; }
 
 // Threads of the forms that take whole nodes or columns.
